@@ -130,9 +130,9 @@ typedef struct atm_tuning {
     int32_t list_capacity;    /* neighbour-list entries per group to start from; 0 = sized
                                  from the density.  A list that overflows grows it (the
                                  evaluation reports ATM_ERR_CAPACITY and is re-run) */
-    int32_t pair_split;       /* waves sharing one group's list in the tile kernel (variant 0
-                                 and FP32 pairs): 1, 2, 4 or 8; more, shorter waves shorten
-                                 the end of the launch where few waves are left */
+    int32_t pair_split;       /* least waves sharing one group's list in the tile kernel (variant 0
+                                 and FP32 pairs): 1, 2, 4 or 8; a launch takes more (2 to 16)
+                                 when its groups are few, so that they fill the chip */
     int32_t full_state2;      /* 0: when every system displaces at most a quarter of its atoms,
                                  x + d is evaluated as the difference from x (the pairs and
                                  exception terms with a displaced atom at both states; the

@@ -236,6 +236,23 @@ SetDesc make_set(const atm_system_desc& d, const Tuning& tu, int s, int state, c
     return D;
 }
 
+// The launch is fastest with some 5,000 to 10,000 waves (the chip holds 4,096 to 5,120 of
+// the tile kernel's): fewer leave SIMDs idle behind one long serial walk, more spend their
+// time on each wave's start.  k_pairs in us with 2 / 4 / 8 / 16 waves per group: 200 groups
+// (4 x 2,501 atoms) 86 / 50 / 36 / 30; 400 (23,000) 83 / 48 / 37 / 41; 1,000 (6 x 9,001,
+// triclinic) 122 / 73 / 69 / 81; 2,400 (6 x 23,000) 106 / 95 / 114 / 155; 8,800
+// (22 x 23,000) 301 / 300 / 374 / 540; 24,000 (64 of 5,000 to 60,000) 610 / 643 / 798 / 1490.
+int pair_split_for(const SetDesc* D, int n, int stride, int asked) {
+    double groups = 0.0;
+    for (int k = 0; k < n; ++k) {
+        const SetDesc& S = D[(long long)k * stride];
+        // clusters per column: its atoms in eights, about half of the last one padding
+        const double ncols = (double)S.nx * S.ny, perCol = S.natoms / (ncols * kClusterSize) + 0.45;
+        groups += ncols * std::ceil(perCol / kGroupClusters);
+    }
+    return std::max(asked, groups <= 256 ? 16 : (groups <= 1280 ? 8 : (groups <= 5120 ? 4 : 2)));
+}
+
 // Largest partial force (kJ/mol/nm) that enters a set's 64-bit fixed-point sums.
 // One slot receives at most: one flush per group that lists its cluster (tile
 // kernel), up to 64 pair terms per group's j-batch sum (compacted kernel), one
@@ -406,7 +423,7 @@ void alloc_layout(Context& C) {
         C.dAcount.release();
     }
     C.dSetEnergy.alloc(sizeof(double) * S2);
-    C.dLptItems.alloc(sizeof(int) * std::max<long long>(C.totalGroups, 1));
+    C.dLptItems.alloc(sizeof(int4) * std::max<long long>(C.totalGroups, 1));
     C.dGq.release(); C.dGsig.release(); C.dGeps.release();
     C.gradsReady = false;
     zero_on_stream(C, C.dRt.p, sizeof(SetRuntime) * S2);
@@ -452,7 +469,7 @@ void alloc_layout(Context& C) {
     P.acount = C.dAcount.as<int>();
     P.setEnergy = C.dSetEnergy.as<double>();
     P.eoff = C.dEoff.as<double>();
-    P.lptItems = C.dLptItems.as<int>();
+    P.lptItems = C.dLptItems.as<int4>();
     P.lptMode = C.tuning.pairOrder;
     P.anyTri = 0;
     for (const SetDesc& D : C.sets) P.anyTri |= D.tri;
@@ -547,9 +564,13 @@ bool uses_atom_lists(const Context& C, int flags) {
     return effective_pair_variant(C.P, C.tuning.pairKernel) == kPairKernelAtomLists && (flags & ATM_EVAL_FP32_PAIRS) == 0;
 }
 
+// Waves per group of a tile-kernel launch over `nsets` sets from `first`, `stride` apart.
+int launch_split(const Context& C, int first, int nsets, int stride) {
+    return pair_split_for(C.sets.data() + first, nsets, stride, C.tuning.pairSplit);
+}
+
 int energy_stride(const Context& C, int flags) {
-    return pair_energy_stride(effective_pair_variant(C.P, C.tuning.pairKernel), (flags & ATM_EVAL_FP32_PAIRS) == 0,
-                              C.tuning.pairSplit);
+    return pair_energy_stride(effective_pair_variant(C.P, C.tuning.pairKernel), (flags & ATM_EVAL_FP32_PAIRS) == 0);
 }
 
 void require_ready(const Context& C) {
@@ -599,6 +620,7 @@ void enqueue_batched(Context& C, int flags, hipEvent_t* ev = nullptr) {
     P.setStride = delta ? 2 : 1;
     P.lptMode = C.tuning.pairOrder;
     const int nsets = delta ? C.nsys : 2 * C.nsys;
+    const int split = launch_split(C, 0, nsets, P.setStride);
     const bool forces = (flags & ATM_EVAL_FORCES) != 0;
     const bool grads = (flags & ATM_EVAL_PARAM_GRADS) != 0;
     if (ev) HIPCHK(hipEventRecord(ev[0], st));
@@ -629,10 +651,10 @@ void enqueue_batched(Context& C, int flags, hipEvent_t* ev = nullptr) {
     if (grads) {
         // the backward mode of the tile kernel with unit weights: energies, pair counts
         // and dU/d(q', h, e') of every set in one pass over the pairs
-        HIPCHK(launch_backward(P, C.totalSlots, 0, nsets, C.maxGroups, nullptr, C.tuning.pairSplit, st));
+        HIPCHK(launch_backward(P, C.totalSlots, 0, nsets, C.maxGroups, nullptr, split, st));
     } else {
         HIPCHK(launch_pairs(P, 0, nsets, C.maxGroups, C.tuning.pairWaves, forces, (flags & ATM_EVAL_FP32_PAIRS) == 0,
-                            C.tuning.pairKernel, C.tuning.pairSplit, st));
+                            C.tuning.pairKernel, split, st));
     }
     if (ev) HIPCHK(hipEventRecord(ev[3], st));
     if (has_exception_terms(C)) HIPCHK(launch_exceptions(P, 0, nsets, forces, st));
@@ -642,7 +664,7 @@ void enqueue_batched(Context& C, int flags, hipEvent_t* ev = nullptr) {
     }
     if (fork) HIPCHK(hipStreamWaitEvent(st, C.evJoin, 0));
     if (ev) HIPCHK(hipEventRecord(ev[4], st));
-    HIPCHK(launch_energy(P, 0, C.nsys, grads ? C.tuning.pairSplit : energy_stride(C, flags), st, delta));
+    HIPCHK(launch_energy(P, 0, C.nsys, grads ? 1 : energy_stride(C, flags), st, delta));
     if (ev) HIPCHK(hipEventRecord(ev[5], st));
     if (forces)
         HIPCHK(launch_blend(P, 0, C.nsys, C.maxAtoms, 0, 0.0, 0.0, (flags & ATM_EVAL_CLEAR_FORCES) != 0, st, delta));
@@ -701,12 +723,13 @@ void eval_plain(Context& C, int flags) {
         for (int stt = 0; stt < 2; ++stt) {
             const int c = 2 * s + stt;
             const SetDesc& D = C.sets[c];
+            const int split = launch_split(C, c, 1, 1);
             HIPCHK(launch_zero_counts(P, c, 1, D.nx * D.ny * D.nz, nullptr, 0, st));
             HIPCHK(launch_build(P, c, 1, D.natoms, D.nx * D.ny * D.nz, D.slotCap, st));
             HIPCHK(launch_pairlist(P, c, 1, D.groupCap, 4, st));
             if (uses_atom_lists(C, flags)) HIPCHK(launch_alist(P, c, 1, D.groupCap, st));
             HIPCHK(launch_pairs(P, c, 1, D.groupCap, C.tuning.pairWaves, true, (flags & ATM_EVAL_FP32_PAIRS) == 0,
-                                C.tuning.pairKernel, C.tuning.pairSplit, st));
+                                C.tuning.pairKernel, split, st));
             if (D.excCount > 0) HIPCHK(launch_exceptions(P, c, 1, true, st));
             HIPCHK(launch_set_energy(P, c, energy_stride(C, flags), true, st));
             HIPCHK(hipMemcpyAsync(&U[stt], P.setEnergy + c, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -732,14 +755,14 @@ void eval_state1(Context& C, int flags) {
     const DevPtrs& P = C.P;
     for (int s = 0; s < C.nsys; ++s) {
         const SetDesc& D = C.sets[2 * s];
-        const int c = 2 * s;
+        const int c = 2 * s, split = launch_split(C, c, 1, 1);
         if (flags & ATM_EVAL_CLEAR_FORCES) HIPCHK(launch_fill_zero(P.outF + 3ll * D.atomOff, 3ll * D.natoms, st));
         HIPCHK(launch_zero_counts(P, c, 1, D.nx * D.ny * D.nz, nullptr, 0, st));
         HIPCHK(launch_build(P, c, 1, D.natoms, D.nx * D.ny * D.nz, D.slotCap, st));
         HIPCHK(launch_pairlist(P, c, 1, D.groupCap, 4, st));
         if (uses_atom_lists(C, flags)) HIPCHK(launch_alist(P, c, 1, D.groupCap, st));
         HIPCHK(launch_pairs(P, c, 1, D.groupCap, C.tuning.pairWaves, (flags & ATM_EVAL_FORCES) != 0,
-                            (flags & ATM_EVAL_FP32_PAIRS) == 0, C.tuning.pairKernel, C.tuning.pairSplit, st));
+                            (flags & ATM_EVAL_FP32_PAIRS) == 0, C.tuning.pairKernel, split, st));
         if (D.excCount > 0) HIPCHK(launch_exceptions(P, c, 1, (flags & ATM_EVAL_FORCES) != 0, st));
         HIPCHK(launch_set_energy(P, c, energy_stride(C, flags), false, st));
         double U = 0.0;
@@ -1429,9 +1452,9 @@ int atm_autotune(void* context, int32_t repeats, atm_tuning* out) {
         const int waves[] = {1, 2, 4};
         // (the atom-list kernel, 5, is left out: it measured slower than the tile kernel on every
         // column scale tried, and its lists need their own buffers)
-        // (kernel, group split): the tile kernel with its lists split 1, 2 or 4 ways,
-        // the compacted kernel 1 and the filtered kernel
-        const int kernels[][2] = {{0, 1}, {0, 2}, {0, 4}, {1, 1}, {kPairKernelFiltered, 1}};
+        // (kernel, group split): the tile kernel at its own choice of waves per group and at
+        // 4 and 8 where that is more, the compacted kernel 1 and the filtered kernel
+        const int kernels[][2] = {{0, 1}, {0, 4}, {0, 8}, {1, 1}, {kPairKernelFiltered, 1}};
         const int nk = (int)(sizeof(kernels) / sizeof(kernels[0]));
         const int zpcs[] = {2, 4};
         const Tuning orig = C.tuning;
@@ -1488,6 +1511,17 @@ int atm_autotune(void* context, int32_t repeats, atm_tuning* out) {
                     C.tuning.pairKernel = kernels[kv / 3][0];
                     C.tuning.pairSplit = kernels[kv / 3][1];
                     C.tuning.pairWaves = waves[kv % 3];
+                    if (C.tuning.pairKernel == 0) {
+                        // blocks are one group: the waves per block do not enter, and a split below
+                        // the launch's own choice is that choice again
+                        if (kv % 3 != 0) continue;
+                        const int asked = C.tuning.pairSplit, delta = use_delta(C, flags);
+                        C.tuning.pairSplit = 1;
+                        const int own = launch_split(C, 0, delta ? C.nsys : 2 * C.nsys, delta ? 2 : 1);
+                        C.tuning.pairSplit = asked;
+                        if (asked > 1 && asked <= own) continue;
+                        C.tuning.pairWaves = orig.pairWaves;
+                    }
                     const double per = time_config(reps);
                     if (per < 1e300) timed.emplace_back(per, C.tuning);
                 }
@@ -1612,8 +1646,8 @@ void backward_impl(Context& C, const double* grad_energy, double* d_charges, dou
         if (C.dWset.bytes < sizeof(double) * 2 * S) C.dWset.alloc(sizeof(double) * 2 * S);
         HIPCHK(hipMemcpyAsync(C.dWset.p, wset.data(), sizeof(double) * 2 * S, hipMemcpyHostToDevice, C.stream));
         if (!fused)
-            HIPCHK(launch_backward(C.P, C.totalSlots, 0, 2 * S, C.maxGroups, C.dWset.as<double>(), C.tuning.pairSplit,
-                                   C.stream));
+            HIPCHK(launch_backward(C.P, C.totalSlots, 0, 2 * S, C.maxGroups, C.dWset.as<double>(),
+                                   launch_split(C, 0, 2 * S, 1), C.stream));
         const size_t nb = sizeof(double) * C.totalAtoms;
         double *oq = d_charges, *os = d_sigmas, *oe = d_epsilons;
         if (!deviceOut) {

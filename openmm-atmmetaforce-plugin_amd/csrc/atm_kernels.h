@@ -46,9 +46,9 @@ struct DevPtrs {
     float4* bbc;
     float4* bbh;
     // groups
-    int4* ginfo;
+    int4* ginfo;           // (first cluster, clusters, column, list entries) per group
     int* gcount;
-    double* genergy;       // pair-kernel energy slots: one per group, or one per i-cluster wave (8 per group)
+    double* genergy;       // pair-kernel energy slots, pair_energy_stride per group
     uint32_t* entries;
     uint32_t* alist;       // atom-level j lists per i-cluster (pair kernel 5)
     int* acount;           // entries (whole 8-atom blocks) per i-cluster
@@ -69,7 +69,7 @@ struct DevPtrs {
     const int* lxidx;      // exception terms (batch index) with a displaced atom, at SetDesc::lxOff
     // group order of the tile kernel, longest lists first per set (k_order, run by the pair
     // launchers; the set's range at groupOff); null: launch order
-    int* lptItems;
+    int4* lptItems;
     int lptMode;           // kOrder*: how the tile kernel's launch ranks map to the groups
     int anyTri = 0;        // some system has a triclinic box (SetDesc::tri)
     // backward
@@ -97,15 +97,14 @@ constexpr int kPairKernelCount = 7;
 // A batch with exceptions or a triclinic box runs the tile kernel whatever the
 // variant asked for: only it applies the exclusion masks and the triclinic images.
 inline int effective_pair_variant(const DevPtrs& P, int variant) { return (P.xmask || P.anyTri) ? 0 : variant; }
-// split (1-8): the tile kernel divides each group's list between that many waves.
+// split (1 to kMaxPairSplit): the tile kernel divides each group's list between that many waves (at
+// least 2; pair_split_for chooses).  waves: waves per block of the other variants.
+constexpr int kMaxPairSplit = 16;
 hipError_t launch_pairs(const DevPtrs& P, int setBegin, int nsets, int maxGroups, int waves, bool forces, bool fp64,
                         int variant, int split, hipStream_t st);
 // Energy slots the pair kernel fills per group in genergy: 8 for the filtered
-// kernel, `split` for the tile kernel, 1 for the others.
-inline int pair_energy_stride(int variant, bool fp64, int split) {
-    if (fp64 && variant == kPairKernelFiltered) return 8;
-    return (variant == 0 || !fp64) ? split : 1;
-}
+// kernel, 1 for the others.
+inline int pair_energy_stride(int variant, bool fp64) { return fp64 && variant == kPairKernelFiltered ? 8 : 1; }
 // Exception terms of sets [setBegin, setBegin + nsets): energy into xenergy[c], with
 // `forces` their forces added to the set's slot sums (call after the pair kernel
 // and before launch_energy / launch_set_energy, which add xenergy when excCount > 0).

@@ -870,6 +870,7 @@ __global__ void __launch_bounds__(64 * W) k_pairlist(DevPtrs P, int setBegin) {
     if (lane == 0) {
         const int kept = min(nEnt, D.entryCap);
         P.gcount[D.groupOff + g] = kept;
+        P.ginfo[D.groupOff + g].w = kept;
         atomicMax(&P.rt[c].maxEntries, nEnt);
         if (nEnt > D.entryCap) atomicOr(&P.rt[c].overflow, 1);
     }
@@ -879,7 +880,8 @@ __global__ void __launch_bounds__(64 * W) k_pairlist(DevPtrs P, int setBegin) {
 // The tile kernel's group order, longest lists first, per set: one block per set
 // setBegin + blockIdx.x setStride files its groups by list length (bucket
 // min(63, entries >> kLptShift)) with LDS counting and writes them from the
-// longest bucket down to lptItems[groupOff ...].  The tile kernel takes rank r as
+// longest bucket down to lptItems[groupOff ...], each as (first cluster, clusters,
+// group, entries) so the tile kernel reads one record per group.  The tile kernel takes rank r as
 // the (r / nsets)-th longest group of set r mod nsets, so the launch starts with
 // every set's longest lists.  The order within a bucket follows LDS atomics,
 // which no result depends on (each group's sums are its own).
@@ -921,7 +923,11 @@ __global__ void __launch_bounds__(512) k_order(DevPtrs P, int setBegin) {
         }
 #pragma unroll
         for (int u = 0; u < NI; ++u)
-            if (bk[u] >= 0) P.lptItems[gOff + atomicAdd(hist + bk[u], 1)] = g0 + u * NT + t;
+            if (bk[u] >= 0) {
+                const int g = g0 + u * NT + t;
+                const int4 gi = P.ginfo[gOff + g];
+                P.lptItems[gOff + atomicAdd(hist + bk[u], 1)] = make_int4(gi.x, gi.y, g, gi.w);
+            }
     }
 }
 
@@ -962,6 +968,29 @@ __device__ __forceinline__ void flush_force(const DevPtrs& P, int c, float fixMa
     }
 }
 
+// The same from FP64 sums (partial forces of several waves added before the flush).
+__device__ __forceinline__ void flush_force64(const DevPtrs& P, int c, float fixMax, int slot, double fx, double fy,
+                                              double fz) {
+    const double m = (double)fixMax;
+    if (fabs(fx) < m && fabs(fy) < m && fabs(fz) < m) {
+        long long* f = P.sf + slot;
+        atomic_add_fixed(f, __double_as_longlong(fx * kForceScale + 6755399441055744.0) - 0x4338000000000000LL);
+        atomic_add_fixed(f + P.sfn, __double_as_longlong(fy * kForceScale + 6755399441055744.0) - 0x4338000000000000LL);
+        atomic_add_fixed(f + 2 * P.sfn, __double_as_longlong(fz * kForceScale + 6755399441055744.0) - 0x4338000000000000LL);
+        return;
+    }
+    const double v[3] = {fx, fy, fz};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        if (fabs(v[k]) < m)
+            atomic_add_fixed(P.sf + (long long)k * P.sfn + slot,
+                             __double_as_longlong(v[k] * kForceScale + 6755399441055744.0) - 0x4338000000000000LL);
+        else
+            atomicAdd(P.sd + 3ll * slot + k, v[k]);
+    }
+    mark_side(P, c, slot);
+}
+
 // b is one of the far excepted partners of atom a (system-local indices).
 __device__ __forceinline__ bool far_excluded(const DevPtrs& P, const SetDesc& D, int a, int b) {
     const int* st = P.xfarStart + D.atomOff + a;
@@ -979,15 +1008,14 @@ __device__ __forceinline__ bool excluded_pair(const DevPtrs& P, const SetDesc& D
 }
 
 
-// Fixed-order sum of a set's energy slots: one per group, or estride per group
-// (8: one per i-cluster wave of the filtered kernel; 2 or 4: one per part of a
-// group whose list the tile kernel splits between waves).
-__device__ __forceinline__ double group_energy(const DevPtrs& P, const SetDesc& D, int g, int estride) {
-    if (estride == 1) return P.genergy[D.groupOff + g];
-    const double* e = P.genergy + (long long)estride * (D.groupOff + g);
-    if (estride == 8) return ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-    double s = e[0];
-    for (int k = 1; k < estride; ++k) s += e[k];
+// This thread's share (of a block of 256) of the fixed-order sum of a set's energy
+// slots: `estride` per group (pair_energy_stride), consecutive over the set's groups,
+// so neighbouring threads read neighbouring slots whatever the stride.
+__device__ __forceinline__ double energy_share(const DevPtrs& P, const SetDesc& D, int ngroups, int estride) {
+    const double* e = P.genergy + (long long)estride * D.groupOff;
+    const int n = ngroups * estride;
+    double s = 0.0;
+    for (int k = threadIdx.x; k < n; k += 256) s += e[k];
     return s;
 }
 
@@ -1016,11 +1044,6 @@ __device__ __forceinline__ void flush_component_u(const DevPtrs& P, int c, float
 // way; forces are flushed to 64-bit fixed point, energies summed in FP64.
 // List entries are fetched 64 at a time (one per lane) and broadcast with
 // readlane, so the cluster mask and the diagonal test are scalar branches.
-// At most 80 VGPRs (6 waves per SIMD): the FP64 forces variant with its two
-// j-atom buffers then spills a few per-batch values outside the entry loop;
-// on a 22 x 23k batch that measured 5 % faster than its unconstrained 88
-// VGPRs (5 waves) and 14 % faster than 72 VGPRs (7 waves, which spill inside
-// the entry loop).
 //
 // BWD (FP64 scalars, no forces): the backward pass on the same tiles -- per
 // in-cutoff pair, the derivatives of its energy with respect to the stored
@@ -1041,62 +1064,73 @@ __device__ __forceinline__ void flush_component_u(const DevPtrs& P, int c, float
 // sets with a triclinic box take OpenMM's triclinic image (the instantiations
 // without EXC carry neither).
 //
-// split: each group's list is divided into `split` consecutive parts, one per
-// wave (blockIdx.x = group block * split + part): shorter waves, so the launch
-// ends with less of a tail when the group lists are long.  Each part adds its
-// own i-force sums and writes its own energy slot (split slots per group).
+// A block is one group: its list is divided into W consecutive parts, one per
+// wave.  The group's atoms are staged once, and the parts' i-force sums, energies
+// and pair counts are added in LDS (FP64, in part order) before one flush.
+// A wave walks its part serially (1.7 us per entry of eight 8x8 steps when it has
+// a SIMD to itself), and needs some 7 us before its first step (descriptor, group
+// record, entries and i-atoms, j-atoms: four dependent reads): W trades the two.
+// Whole k_pairs launch, one wave per group -> W: 3,000 atoms (50 groups) 319 us ->
+// 27 us with 16; 6 x 9,001 triclinic (1,000 groups) 285 -> 69 us with 8; 6 x 23,000
+// (2,400 groups) 171 -> 95 us with 4; 22 x 23,000 (8,800 groups) 342 -> 302 us with 2.
+// Registers: 5 waves per SIMD (96 VGPRs) for 2 and 4 waves per group (6 waves spill
+// inside the entry loop: 353 against 312 us on 22 x 23,000), 4 for the longer blocks.
 template <int W, bool FORCES, bool F64, bool BWD, bool EXC>
-__global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, const double* wset, int split) {
+__global__ void __launch_bounds__(64 * W, W >= 8 ? 4 : 5) k_pairs(DevPtrs P, int setBegin, const double* wset) {
     static_assert(!BWD || (F64 && !FORCES), "the backward mode is FP64 and computes no forces");
     constexpr bool JSUMS = FORCES || BWD;  // per-atom j sums flushed every kJFlush entries
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int jj = lane >> 3, ii = lane & 7;
-    int c, g, part;
+    int c;
+    int4 item = make_int4(0, 0, 0, 0);  // (first cluster, clusters, group, entries)
     bool active;
     if (P.lptItems && P.lptMode == kOrderSetMajor) {
         // each set's groups longest list first, the sets one after the other (blockIdx.y)
-        const int f = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * W + wave));
-        const int pos = f / split;
-        part = f - pos * split;
+        const int pos = (int)blockIdx.x;
         c = setBegin + (int)blockIdx.y * P.setStride;
         active = pos < P.rt[c].ngroups;
-        g = active ? __builtin_amdgcn_readfirstlane(P.lptItems[P.desc[c].groupOff + pos]) : 0;
+        if (active) item = P.lptItems[P.desc[c].groupOff + pos];
     } else if (P.lptItems && P.lptMode != kOrderLaunch) {
-        // longest lists first over windows of sets: this wave's rank f in launch order falls in
-        // window f / (K gx) of K sets (K = every set, or kOrderWindowSets; gx waves per set), where
-        // it is part (rank in the window) % split of item (rank in the window) / split: the
-        // (item / K')-th longest group of the window's set item mod K' (K' its sets; k_order)
-        const int gx = (int)gridDim.x * W;
+        // longest lists first over windows of sets: this group's rank f in launch order falls in
+        // window f / (K gx) of K sets (K = every set, or kOrderWindowSets; gx ranks per set), where
+        // it is the (rank in the window / K')-th longest group of the window's set rank mod K'
+        // (K' its sets; k_order)
+        const int gx = (int)gridDim.x;
         const int K = P.lptMode == kOrderAllSets ? (int)gridDim.y : kOrderWindowSets;
-        const int f = __builtin_amdgcn_readfirstlane((int)((blockIdx.y * gridDim.x + blockIdx.x) * W + wave));
+        const int f = (int)(blockIdx.y * gridDim.x + blockIdx.x);
         const int win = f / (K * gx), within = f - win * (K * gx);
         const int kw = min(K, (int)gridDim.y - win * K);
-        const int item = within / split;
-        part = within - item * split;
-        const int pos = item / kw;
-        c = setBegin + (win * K + (item - pos * kw)) * P.setStride;
+        const int pos = within / kw;
+        c = setBegin + (win * K + (within - pos * kw)) * P.setStride;
         active = within < kw * gx && pos < P.rt[c].ngroups;
-        g = active ? __builtin_amdgcn_readfirstlane(P.lptItems[P.desc[c].groupOff + pos]) : 0;
+        if (active) item = P.lptItems[P.desc[c].groupOff + pos];
     } else {
         c = setBegin + (int)blockIdx.y * P.setStride;
-        part = blockIdx.x % split;
-        g = (blockIdx.x / split) * W + wave;
-        active = g < P.rt[c].ngroups;
+        const int pos = blockIdx.x;
+        active = pos < P.rt[c].ngroups;
+        if (active) {
+            const int4 gi = P.ginfo[P.desc[c].groupOff + pos];
+            item = make_int4(gi.x, gi.y, pos, gi.w);
+        }
     }
+    const int g0 = __builtin_amdgcn_readfirstlane(item.x), ncl = __builtin_amdgcn_readfirstlane(item.y);
+    const int g = __builtin_amdgcn_readfirstlane(item.z), nall = __builtin_amdgcn_readfirstlane(item.w);
     const SetDesc D = P.desc[c];  // wave-uniform: lives in SGPRs for the whole kernel
-    __shared__ float4 sPos[W][64];
-    __shared__ float2 sPrm[W][F64 ? 1 : 64];
-    __shared__ double4 sPrm64[W][F64 ? 64 : 1];
-    __shared__ int sAi[W][EXC ? 64 : 1];                   // i-atom indices (system-local, -1: dummy)
-    __shared__ unsigned long long sXm[W][EXC ? 64 : 1];    // their near exception masks
-    int g0 = 0, ncl = 0;
-    float zlo = 3.0e38f, zhi = -3.0e38f;  // z-range of the group's real i-atoms
-    uint32_t ivm = 0;       // bit t: i-atom (t, ii) is a real atom
-    uint64_t ivLanes = 0;   // bit 8 t + ii: the same, over the group's 64 slots
+    __shared__ float4 sPos[64];
+    __shared__ float2 sPrm[F64 ? 1 : 64];
+    __shared__ double4 sPrm64[F64 ? 64 : 1];
+    __shared__ int sAi[EXC ? 64 : 1];                   // i-atom indices (system-local, -1: dummy)
+    __shared__ unsigned long long sXm[EXC ? 64 : 1];    // their near exception masks
+    // this wave's part of the list; its first 64 entries are read beside the i-atoms
+    const int eb = wave * nall / W, ne = (wave + 1) * nall / W - eb;
+    const uint32_t* E = P.entries + D.entryOff + (long long)g * D.entryCap + eb;
+    const uint32_t ebuf0 = lane < ne ? E[lane] : 0u;
+    // the i-atoms at least the cutoff (+ the list margin) inside the box in z; the FP32 D.rc
+    // carries its rounding margin
+    const float rcz = D.rc * (1.0f + 1e-5f) + 1e-4f;
+    bool zInside = false;
+    uint64_t ivLanes = 0;   // bit 8 t + ii: i-atom (t, ii) is a real atom, over the group's 64 slots
     if (active) {
-        const int4 gi = P.ginfo[D.groupOff + g];
-        g0 = __builtin_amdgcn_readfirstlane(gi.x);
-        ncl = __builtin_amdgcn_readfirstlane(gi.y);
         float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
         float2 q = make_float2(0.f, 0.f);
         double4 qd = make_double4(0.0, 0.0, 0.0, 0.0);
@@ -1106,33 +1140,25 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
         if (lane < ncl * kClusterSize) {
             const int s = D.slotOff + g0 * kClusterSize + lane;
             p = P.spos[s];
-            if (F64) qd = P.sprm64[s]; else q = P.sprm[s];
+            if (wave == 0) { if (F64) qd = P.sprm64[s]; else q = P.sprm[s]; }
             ai = P.sidx[s];
             v = ai >= 0;
-            if (EXC && v && P.xmask) xm = P.xmask[D.atomOff + ai];  // no mask: no pair is excepted
+            if (EXC && wave == 0 && v && P.xmask) xm = P.xmask[D.atomOff + ai];  // no mask: no pair is excepted
         }
-        if (EXC) {
-            sAi[wave][lane] = ai;
-            sXm[wave][lane] = xm;
+        if (wave == 0) {
+            if (EXC) {
+                sAi[lane] = ai;
+                sXm[lane] = xm;
+            }
+            sPos[lane] = p;
+            if (F64) sPrm64[lane] = qd; else sPrm[lane] = q;
         }
-        sPos[wave][lane] = p;
-        if (F64) sPrm64[wave][lane] = qd; else sPrm[wave][lane] = q;
-        zlo = v ? p.z : zlo;
-        zhi = v ? p.z : zhi;
-        for (int o = 32; o > 0; o >>= 1) {
-            zlo = fminf(zlo, __shfl_xor(zlo, o, 64));
-            zhi = fmaxf(zhi, __shfl_xor(zhi, o, 64));
-        }
-        const uint64_t vb = __ballot(v);
-        ivLanes = vb;
-#pragma unroll
-        for (int t = 0; t < kGroupClusters; ++t) ivm |= (uint32_t)((vb >> (t * kClusterSize + ii)) & 1ull) << t;
+        zInside = __ballot(v && !(p.z - rcz >= 0.f && p.z + rcz < D.L[2])) == 0ull;
+        ivLanes = __ballot(v);
     }
     __syncthreads();
-    if (!active) return;
-    // wave-uniform from here on: keep the group's values in scalar registers
-    g0 = __builtin_amdgcn_readfirstlane(g0);
-    ncl = __builtin_amdgcn_readfirstlane(ncl);
+    if (!active) return;  // the whole block: one group
+    // wave-uniform: keep the mask in scalar registers
     ivLanes = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)ivLanes) |
               (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(ivLanes >> 32)) << 32;
     const uint64_t upperLanes = __builtin_amdgcn_ballot_w64(ii < jj);  // i < j inside a diagonal cluster
@@ -1148,9 +1174,6 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
     for (int t = 0; t < kGroupClusters; ++t) fi[t][0] = fi[t][1] = fi[t][2] = 0.f;
     double eE = 0.0;  // this lane's sum of whole pair energies
     uint32_t npair = 0;  // in-cutoff pairs evaluated by this wave (wave-uniform)
-    const int nall = __builtin_amdgcn_readfirstlane(P.gcount[D.groupOff + g]);
-    const int eb = (int)(((long long)part * nall) / split), ne = (int)(((long long)(part + 1) * nall) / split) - eb;
-    const uint32_t* E = P.entries + D.entryOff + (long long)g * D.entryCap + eb;
     // This lane's j-atom of one list entry.  Two of these are in flight: entry
     // k + 1's loads are issued before entry k is evaluated, into the other
     // buffer, so the wait for them falls after entry k's work (and not behind
@@ -1175,8 +1198,8 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
     };
     // lanes of `in` whose pair (i-atom (t, ii), j-atom aj) is an exception
     auto excepted = [&](int t, int aj, uint64_t in) __attribute__((always_inline)) {
-        const int ai = sAi[wave][t * kClusterSize + ii];
-        const unsigned long long mi = sXm[wave][t * kClusterSize + ii];
+        const int ai = sAi[t * kClusterSize + ii];
+        const unsigned long long mi = sXm[t * kClusterSize + ii];
         const uint32_t dd = (uint32_t)(aj - ai + 32);
         const bool near = dd - 1u < 63u;
         bool ex = near && ((mi >> (dd & 63u)) & 1ull);
@@ -1237,11 +1260,11 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
         float fjx = 0.f, fjy = 0.f, fjz = 0.f;
         // i-atom positions read one step ahead (whether or not that step runs),
         // so the LDS latency falls behind the current step's work
-        float4 piN = sPos[wave][ii];
+        float4 piN = sPos[ii];
 #pragma unroll
         for (int t = 0; t < kGroupClusters; ++t) {
             const float4 pi = piN;
-            if (t + 1 < kGroupClusters) piN = sPos[wave][(t + 1) * kClusterSize + ii];
+            if (t + 1 < kGroupClusters) piN = sPos[(t + 1) * kClusterSize + ii];
             if (imask & (1u << t)) {
                 float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
                 if (!shiftOK) {
@@ -1267,7 +1290,7 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
                     const double r2 = fma((double)dx, (double)dx, fma((double)dy, (double)dy, (double)dz * (double)dz));
                     uint64_t inLanes = __builtin_amdgcn_ballot_w64(r2 < rc2) & okLanes;
                     if (inLanes == 0ull) continue;  // no pair of this 8x8 step is inside
-                    const double4 id = sPrm64[wave][t * kClusterSize + ii];
+                    const double4 id = sPrm64[t * kClusterSize + ii];
                     if (EXC && P.xmask) inLanes &= ~excepted(t, b.idx, inLanes);
                     npair += (uint32_t)__popcll(inLanes);
                     // lanes outside the cutoff are masked off (exec), not zeroed with selects
@@ -1301,7 +1324,7 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
                     uint64_t iv = (ivLanes >> (t * kClusterSize)) & 0xFFull;
                     iv |= iv << 8; iv |= iv << 16; iv |= iv << 32;
                     const uint64_t okLanes = (t == tdiag ? upperLanes : ~0ull) & jvLanes & iv;
-                    const float2 qi = sPrm[wave][t * kClusterSize + ii];
+                    const float2 qi = sPrm[t * kClusterSize + ii];
                     const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
                     uint64_t inLanes = __builtin_amdgcn_ballot_w64(in_cutoff(D, dx, dy, dz, r2)) & okLanes;
                     if (EXC && P.xmask && inLanes != 0ull) inLanes &= ~excepted(t, b.idx, inLanes);
@@ -1336,8 +1359,8 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
     // runs and its j sums are zero; the load after a batch's last pair wraps to
     // lane 0 and is not used.
     auto entries = [&](auto zdir) __attribute__((always_inline)) {
+        uint32_t ebuf = ebuf0;
         for (int e0 = 0; e0 < ne; e0 += 64) {
-            const uint32_t ebuf = (e0 + lane < ne) ? E[e0 + lane] : 0u;
             const int nb = min(64, ne - e0);
             JBuf bufA = load_jbuf(__builtin_amdgcn_readlane(ebuf, 0)), bufB;
             for (int k = 0; k < nb; k += 2) {
@@ -1346,39 +1369,76 @@ __global__ void __launch_bounds__(64 * W, 6) k_pairs(DevPtrs P, int setBegin, co
                 bufA = load_jbuf(__builtin_amdgcn_readlane(ebuf, (k + 2) & 63));
                 do_entry(__builtin_amdgcn_readlane(ebuf, k + 1), bufB, zdir);
             }
+            ebuf = e0 + 64 + lane < ne ? E[e0 + 64 + lane] : 0u;
         }
     };
-    // the i-atoms' z-range at least the cutoff (+ the list margin) inside the box in z; the
-    // FP32 D.rc carries its rounding margin.  Without EXC only sets with explicit x/y shifts
-    // take the z-direct loop (that loop then carries no x/y image code: fewer registers)
-    const float rcz = D.rc * (1.0f + 1e-5f) + 1e-4f;
-    const bool zDirect = (EXC || shiftOK) &&
-                         __builtin_amdgcn_readfirstlane((int)(zlo - rcz >= 0.f && zhi + rcz < Lz)) != 0;
+    // without EXC only sets with explicit x/y shifts take the z-direct loop (that loop then
+    // carries no x/y image code: fewer registers)
+    const bool zDirect = (EXC || shiftOK) && __builtin_amdgcn_readfirstlane((int)zInside) != 0;
     if (zDirect) entries(std::true_type{}); else entries(std::false_type{});
     if (JSUMS && (ecount & (kJFlush - 1)) != 0) flush_j(ecount & (kJFlush - 1));
     if (JSUMS) {
+        // sum over the 8 j-columns and hand lane 8 t + ii the sums of i-atom (t, ii): each step
+        // of the butterfly (lane bits 5, 4, 3) halves the clusters a lane still carries
+        float fx, fy, fz;
+        {
+            float h4[4][3], h2[2][3];
+            const bool up5 = (lane & 32) != 0, up4 = (lane & 16) != 0, up3 = (lane & 8) != 0;
 #pragma unroll
-        for (int t = 0; t < kGroupClusters; ++t) {
-            if (t < ncl) {
-                const float fx = stride8_sum(fi[t][0]), fy = stride8_sum(fi[t][1]), fz = stride8_sum(fi[t][2]);
-                const int is = D.slotOff + (g0 + t) * kClusterSize + ii;
-                if (jj == 0 && ((ivm >> t) & 1u)) {
-                    if (BWD) {
-                        if (fx != 0.f) atomicAdd(P.gq + is, wgt * (double)fx);
-                        if (fy != 0.f) atomicAdd(P.gsig + is, wgt * (double)fy);
-                        if (fz != 0.f) atomicAdd(P.geps + is, wgt * (double)fz);
-                    } else {
-                        flush_force(P, c, fixMax, is, fx, fy, fz);
-                    }
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const float keep = up5 ? fi[t + 4][k] : fi[t][k], give = up5 ? fi[t][k] : fi[t + 4][k];
+                    h4[t][k] = keep + __shfl_xor(give, 32, 64);
                 }
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const float keep = up4 ? h4[t + 2][k] : h4[t][k], give = up4 ? h4[t][k] : h4[t + 2][k];
+                    h2[t][k] = keep + __shfl_xor(give, 16, 64);
+                }
+            const float kx = up3 ? h2[1][0] : h2[0][0], gx = up3 ? h2[0][0] : h2[1][0];
+            const float ky = up3 ? h2[1][1] : h2[0][1], gy = up3 ? h2[0][1] : h2[1][1];
+            const float kz = up3 ? h2[1][2] : h2[0][2], gz = up3 ? h2[0][2] : h2[1][2];
+            fx = kx + __shfl_xor(gx, 8, 64);
+            fy = ky + __shfl_xor(gy, 8, 64);
+            fz = kz + __shfl_xor(gz, 8, 64);
+        }
+        const int is = D.slotOff + g0 * kClusterSize + lane;
+        const bool real = (ivLanes >> lane) & 1ull;
+        // the parts' sums through the flush buffers (each wave's own rows)
+        wave_sync();
+        sJF[wave][0][lane] = fx; sJF[wave][1][lane] = fy; sJF[wave][2][lane] = fz;
+        __syncthreads();
+        if (wave == 0 && real) {
+            double sx = 0.0, sy = 0.0, sz = 0.0;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                sx += (double)sJF[w][0][lane]; sy += (double)sJF[w][1][lane]; sz += (double)sJF[w][2][lane];
+            }
+            if (BWD) {
+                if (sx != 0.0) atomicAdd(P.gq + is, wgt * sx);
+                if (sy != 0.0) atomicAdd(P.gsig + is, wgt * sy);
+                if (sz != 0.0) atomicAdd(P.geps + is, wgt * sz);
+            } else {
+                flush_force64(P, c, fixMax, is, sx, sy, sz);
             }
         }
     }
     if (BWD && wset) return;  // a backward pass after the evaluation: energies and counts are the evaluation's
     double eacc = eE;
     eacc = wave_sum_d(eacc);
-    if (lane == 0) {
-        P.genergy[(long long)(D.groupOff + g) * split + part] = eacc;
+    __shared__ double sE[W];
+    __shared__ uint32_t sN[W];
+    if (lane == 0) { sE[wave] = eacc; sN[wave] = npair; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        eacc = 0.0;
+        npair = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) { eacc += sE[w]; npair += sN[w]; }
+        P.genergy[D.groupOff + g] = eacc;
         atomicAdd(&P.rt[c].npairs, (unsigned long long)npair);
     }
 }
@@ -2494,8 +2554,7 @@ __global__ void __launch_bounds__(256) k_energy(DevPtrs P, int sysBegin, int est
         const int c0 = 2 * s, c1 = 2 * s + 1;
         const SetDesc& D = P.desc[c0];
         const int ng = P.rt[c0].ngroups;
-        double acc = 0.0;
-        for (int g = threadIdx.x; g < ng; g += 256) acc += group_energy(P, D, g, estride);
+        const double acc = energy_share(P, D, ng, estride);
         const double e0 = block_sum_256(acc, red) + (D.excCount > 0 ? P.xenergy[c0] : 0.0);
         double dd = 0.0;
         for (int k = threadIdx.x; k < D.ligCount; k += 256) {
@@ -2514,9 +2573,7 @@ __global__ void __launch_bounds__(256) k_energy(DevPtrs P, int sysBegin, int est
         const int c = 2 * s + st;
         const SetDesc& D = P.desc[c];
         const int ng = P.rt[c].ngroups;
-        double acc = 0.0;
-        for (int g = threadIdx.x; g < ng; g += 256) acc += group_energy(P, D, g, estride);
-        red[threadIdx.x] = acc;
+        red[threadIdx.x] = energy_share(P, D, ng, estride);
         __syncthreads();
         for (int o = 128; o > 0; o >>= 1) {
             if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
@@ -2537,9 +2594,7 @@ __global__ void __launch_bounds__(256) k_set_energy(DevPtrs P, int c, int estrid
     __shared__ double red[256];
     const SetDesc& D = P.desc[c];
     const int ng = P.rt[c].ngroups;
-    double acc = 0.0;
-    for (int g = threadIdx.x; g < ng; g += 256) acc += group_energy(P, D, g, estride);
-    red[threadIdx.x] = acc;
+    red[threadIdx.x] = energy_share(P, D, ng, estride);
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
         if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
@@ -2663,6 +2718,37 @@ hipError_t launch_alist(const DevPtrs& P, int setBegin, int nsets, int maxGroups
     return hipGetLastError();
 }
 
+// The tile kernel with `split` waves per group (at least 2: one wave walking a whole list
+// measured slower at every size).
+template <bool FORCES, bool F64, bool BWD, bool EXC>
+static void launch_tiles_x(const DevPtrs& P, int setBegin, int nsets, int maxGroups, int split, const double* wset,
+                           hipStream_t st) {
+    const dim3 grid(maxGroups, nsets);
+    if (split <= 2) k_pairs<2, FORCES, F64, BWD, EXC><<<grid, 128, 0, st>>>(P, setBegin, wset);
+    else if (split <= 4) k_pairs<4, FORCES, F64, BWD, EXC><<<grid, 256, 0, st>>>(P, setBegin, wset);
+    else if (split <= 8) k_pairs<8, FORCES, F64, BWD, EXC><<<grid, 512, 0, st>>>(P, setBegin, wset);
+    else k_pairs<16, FORCES, F64, BWD, EXC><<<grid, 1024, 0, st>>>(P, setBegin, wset);
+}
+
+template <bool FORCES, bool F64, bool BWD>
+static void launch_tiles(const DevPtrs& P, int setBegin, int nsets, int maxGroups, int split, const double* wset,
+                         hipStream_t st) {
+    if (P.xmask || P.anyTri) launch_tiles_x<FORCES, F64, BWD, true>(P, setBegin, nsets, maxGroups, split, wset, st);
+    else launch_tiles_x<FORCES, F64, BWD, false>(P, setBegin, nsets, maxGroups, split, wset, st);
+}
+
+// Files the groups longest list first (k_order), unless every wave of the launch starts at
+// once anyway (4 waves on each of the 1,024 SIMDs): then the order changes nothing and its
+// launch (4 us) is saved.
+static DevPtrs order_groups(const DevPtrs& P, int setBegin, int nsets, int maxGroups, int split, hipStream_t st) {
+    DevPtrs Pk = P;
+    if (!P.lptItems || P.lptMode == kOrderLaunch || (long long)nsets * maxGroups * std::max(split, 2) <= 4096)
+        Pk.lptItems = nullptr;
+    else
+        k_order<<<nsets, 512, 0, st>>>(P, setBegin);
+    return Pk;
+}
+
 hipError_t launch_pairs(const DevPtrs& P, int setBegin, int nsets, int maxGroups, int waves, bool forces, bool fp64,
                         int variant, int split, hipStream_t st) {
     variant = effective_pair_variant(P, variant);
@@ -2710,27 +2796,15 @@ hipError_t launch_pairs(const DevPtrs& P, int setBegin, int nsets, int maxGroups
 #undef ATM_PAIRSQ
         return hipGetLastError();
     }
-    if (split < 1 || split > 8) return hipErrorInvalidValue;
-    const DevPtrs& Pk = P;
-    if (P.lptItems && P.lptMode != kOrderLaunch) k_order<<<nsets, 512, 0, st>>>(P, setBegin);
-#define ATM_PAIRS_X(WV, F64, X)                                                                                   \
-    if (forces) k_pairs<WV, true, F64, false, X><<<dim3(cdiv(maxGroups, WV) * split, nsets), 64 * WV, 0, st>>>(   \
-        Pk, setBegin, nullptr, split);                                                                            \
-    else k_pairs<WV, false, F64, false, X><<<dim3(cdiv(maxGroups, WV) * split, nsets), 64 * WV, 0, st>>>(        \
-        Pk, setBegin, nullptr, split);
-#define ATM_PAIRS(WV, F64)                                \
-    if (P.xmask || P.anyTri) { ATM_PAIRS_X(WV, F64, true) } else { ATM_PAIRS_X(WV, F64, false) }
-#define ATM_PAIRS_W(F64)               \
-    switch (waves) {                   \
-        case 1: ATM_PAIRS(1, F64) break; \
-        case 2: ATM_PAIRS(2, F64) break; \
-        case 8: ATM_PAIRS(8, F64) break; \
-        default: ATM_PAIRS(4, F64) break; \
+    if (split < 1 || split > kMaxPairSplit) return hipErrorInvalidValue;
+    const DevPtrs Pk = order_groups(P, setBegin, nsets, maxGroups, split, st);
+    if (fp64) {
+        if (forces) launch_tiles<true, true, false>(Pk, setBegin, nsets, maxGroups, split, nullptr, st);
+        else launch_tiles<false, true, false>(Pk, setBegin, nsets, maxGroups, split, nullptr, st);
+    } else {
+        if (forces) launch_tiles<true, false, false>(Pk, setBegin, nsets, maxGroups, split, nullptr, st);
+        else launch_tiles<false, false, false>(Pk, setBegin, nsets, maxGroups, split, nullptr, st);
     }
-    if (fp64) { ATM_PAIRS_W(true) } else { ATM_PAIRS_W(false) }
-#undef ATM_PAIRS_W
-#undef ATM_PAIRS
-#undef ATM_PAIRS_X
     return hipGetLastError();
 }
 
@@ -2746,11 +2820,9 @@ hipError_t launch_set_energy(const DevPtrs& P, int c, int estride, bool withOffs
 
 hipError_t launch_backward_pairs(const DevPtrs& P, int setBegin, int nsets, int maxGroups, const double* wset,
                                  int split, hipStream_t st) {
-    if (split < 1 || split > 8) return hipErrorInvalidValue;
-    const DevPtrs& Pk = P;
-    if (P.lptItems && P.lptMode != kOrderLaunch) k_order<<<nsets, 512, 0, st>>>(P, setBegin);
-    if (P.xmask || P.anyTri) k_pairs<1, false, true, true, true><<<dim3(maxGroups * split, nsets), 64, 0, st>>>(Pk, setBegin, wset, split);
-    else k_pairs<1, false, true, true, false><<<dim3(maxGroups * split, nsets), 64, 0, st>>>(Pk, setBegin, wset, split);
+    if (split < 1 || split > kMaxPairSplit) return hipErrorInvalidValue;
+    const DevPtrs Pk = order_groups(P, setBegin, nsets, maxGroups, split, st);
+    launch_tiles<false, true, true>(Pk, setBegin, nsets, maxGroups, split, wset, st);
     return hipGetLastError();
 }
 

@@ -215,9 +215,10 @@ extern "C" int atm_eval_noalloc(const atm_system_desc* system, const atm_params*
         P.bbh = cv.take<float4>(clOff);
         P.ginfo = cv.take<int4>(gOff);
         P.gcount = cv.take<int>(gOff);
-        P.genergy = cv.take<double>(8 * gOff);
         P.entries = cv.take<uint32_t>(eOff);
         P.setEnergy = cv.take<double>(2);
+        const int split = pair_split_for(D, 2, 1, tu.pairSplit);
+        P.genergy = cv.take<double>(8 * gOff);
         P.alist = nullptr;
         P.acount = nullptr;
         P.gq = P.gsig = P.geps = nullptr;
@@ -239,9 +240,8 @@ extern "C" int atm_eval_noalloc(const atm_system_desc* system, const atm_params*
         HIPCHK(launch_build(P, 0, 2, n, maxCells, maxSlots, st));
         HIPCHK(launch_pairlist(P, 0, 2, maxGroups, 4, st));
         HIPCHK(launch_pairs(P, 0, 2, maxGroups, tu.pairWaves, withForces, (flags & ATM_EVAL_FP32_PAIRS) == 0,
-                            tu.pairKernel, tu.pairSplit, st));
-        HIPCHK(launch_energy(P, 0, 1, pair_energy_stride(tu.pairKernel, (flags & ATM_EVAL_FP32_PAIRS) == 0, tu.pairSplit),
-                             st));
+                            tu.pairKernel, split, st));
+        HIPCHK(launch_energy(P, 0, 1, pair_energy_stride(tu.pairKernel, (flags & ATM_EVAL_FP32_PAIRS) == 0), st));
         if (withForces) HIPCHK(launch_blend(P, 0, 1, n, 0, 0.0, 0.0, true, st));
         hipLaunchKernelGGL(k_noalloc_finish, dim3((std::max(n, 1) + 255) / 256), dim3(256), 0, st, P, n,
                            withForces ? 1 : 0, (flags & ATM_EVAL_CLEAR_FORCES) ? 1 : 0, forces, status);
