@@ -15,6 +15,9 @@ constexpr int kPmeHalfShell = 14;  // the cell itself and its 13 forward neighbo
 constexpr int kPmeBinLds = 4096;   // cell grids up to this size are binned through LDS histograms
 constexpr int kPmeDftLdsMax = 600; // grid lines up to this length are transformed from LDS
 constexpr int kPmeTileLdsMax = 49152;  // bytes of LDS for one cell's charge-grid tile
+constexpr int kPmeFuseNT = 512;    // threads of the fused transform kernels ...
+constexpr int kPmeFuseMax = 4096;  // ... and complex points they hold (8 per thread in registers between steps)
+constexpr int kPmeLineTile = 16;   // grid lines per block of the fused line kernel (fewer when lines are long)
 
 // Scalars of one evaluation (by value in the kernel arguments).
 struct PmeDesc {
@@ -25,6 +28,12 @@ struct PmeDesc {
     int twOff[3];                // offset of each axis' twiddle table
     int nex;                     // exception pairs
     int nslot, nslotDirect, nslotEx;  // energy slots per state (direct | exceptions | reciprocal)
+    int nslotUsed[2];            // direct slots in use per state (delta: state 1 holds the displaced atoms' differences)
+    int delta;                   // direct space and charges of x + d as the difference from x (few displaced atoms)
+    int nlig;                    // displaced atoms
+    // fused transforms (fused != 0): planes over axes pAx, qAx in LDS, then lines along lineAx with the
+    // convolution; every axis length K = fA (K / fA) in two short steps
+    int fused, lineAx, pAx, qAx, fA[3], lineTile, lineBlocks;
     int tile[3], tileBytes;      // per-cell charge-grid tile (0 bytes: spread without tiles)
     double L[3], invL[3];
     double rc2, alpha, twoAlphaSqrtPi, pi2OverAlpha2;
@@ -53,12 +62,13 @@ struct PmePtrs {
     const uint32_t* exbits; // exclusion bitmaps
     const int2* expairs;    // [nex]
     const double4* exprm;   // [nex] (k_e qq', sigma', 4 eps', k_e q_i q_j)
-    long long* qgrid;       // [ngrid] fixed-point charge grid
-    double2* g0;            // [ngrid]
-    double2* g1;            // [ngrid]
+    long long* qgrid;       // [2][ngrid] fixed-point charge grids (delta: the second is the difference)
+    double2* g0;            // [2][ngrid]
+    double2* g1;            // [2][ngrid] (fused: the potentials, [2][ngrid] doubles)
     const double2* tw;      // twiddles of the three axes
     const double* bmod;     // B-spline moduli of the three axes, concatenated
-    unsigned long long* F;  // [2][3][n] fixed-point forces per state (SoA)
+    unsigned long long* F;  // [3][3][n] fixed-point forces (SoA): of state 0, of state 1, and the part both share
+    const int* lig;         // [nlig] displaced atoms
     double* eslot;          // [2][nslot]
     double* parts;          // [2][5]
     SysResult* result;
@@ -80,7 +90,8 @@ struct BondedPtrs {
 };
 
 hipError_t launch_pme_fill(unsigned long long* p, long long n, hipStream_t st);
-hipError_t launch_pme_state(const PmeDesc& D, const PmePtrs& P, int state, hipStream_t st);
+// Every kernel of one evaluation (single: state 0 only) up to the energy sums.
+hipError_t launch_pme_states(const PmeDesc& D, const PmePtrs& P, bool single, hipStream_t st);
 hipError_t launch_pme_finish(const PmeDesc& D, const PmePtrs& P, bool single, double* forcesOut, hipStream_t st);
 hipError_t launch_bonded(const BondedPtrs& B, double* eslot, int nblocks, hipStream_t st);
 

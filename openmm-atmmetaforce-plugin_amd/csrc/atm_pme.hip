@@ -1,10 +1,9 @@
 // gfx950 kernels of the PME variable group: OpenMM's NonbondedForce with
 // particle-mesh Ewald evaluated on x and on x + d, then the ATM combine.
 //
-// Per coordinate set (state s = 0: x, 1: x + d):
-//   k_pme_fill3      clear the cell counts, charge grid and force sums
-//   k_pme_bin        (state 1: form x + d) wrap into the box, cell of edge
-//                    >= rc, rank in the cell
+// Direct space and charge spreading of x:
+//   k_pme_fill3      clear the cell counts, charge grids and force sums
+//   k_pme_bin        (form x + d) wrap into the box, cell of edge >= rc, rank in the cell
 //   k_pme_scan       cell starts (one block)
 //   k_pme_scatter    atom indices into cell order
 //   k_pme_cellsort   each cell ordered by atom index (deterministic sums), and
@@ -17,12 +16,18 @@
 //   k_pme_spread_tiles  order-5 B-spline charge spreading per cell into an LDS
 //                    tile of the grid, 64-bit fixed point (k_pme_spread: the
 //                    same straight into the grid, when a tile does not fit)
-//   k_pme_dft_lines  one axis of the 3-D complex DFT, lines staged in LDS (run
-//                    3x forward, the first reading the fixed-point charge grid,
-//                    3x back; k_pme_q2c + k_pme_dft for lines too long for LDS)
-//   k_pme_convolve   influence function, reciprocal energy, convolution
-//   k_pme_gather     reciprocal forces from the potential grid
-//   k_pme_exceptions exception pairs: own Coulomb + LJ, minus erf(alpha r)/r
+// x + d differs from x at the displaced atoms only.  When they are few (at most one in
+// 16) k_pme_displaced adds what their pairs change, and their charges move on a
+// difference grid; otherwise the same kernels run on x + d.  Then for both states at
+// once (blockIdx.y):
+//   k_pme_planes     two axes of the forward transform per plane of the grid, in LDS
+//   k_pme_lines      the third axis forward, influence function, reciprocal energy,
+//                    convolution, the third axis back
+//   k_pme_planes     the other two axes back, to the real potential
+//                    (k_pme_dft_lines / k_pme_convolve, one pass per axis, where a plane
+//                    does not fit a block; k_pme_q2c + k_pme_dft for lines too long for LDS)
+//   k_pme_gather     reciprocal forces from the potential grid; exception pairs:
+//                    own Coulomb + LJ, minus erf(alpha r)/r
 // and once per evaluation:
 //   k_pme_finish     fixed-order sums of every energy slot, U1, U2, combine
 //   k_pme_blend      F += (1 - sp) F1 + sp F2 (direction-aware), FP64 out
@@ -113,9 +118,9 @@ __device__ __forceinline__ void bspline5(double w, double th[kOrder], double dth
 // atomic per (block, occupied cell), so the few hundred atoms of a cell do not
 // serialise on one counter; grids with more than kPmeBinLds cells use global
 // atomics directly.
-// d: when not null, the positions binned are x + d (the displaced state), also
-// written to P.x2 for the kernels after this one.
-__global__ void __launch_bounds__(256) k_pme_bin(PmeDesc D, PmePtrs P, const double* x, const double* d) {
+// d: when not null, x + d (the displaced state) is written to P.x2 for the kernels
+// after this one; shifted: those positions are the ones binned.
+__global__ void __launch_bounds__(256) k_pme_bin(PmeDesc D, PmePtrs P, const double* x, const double* d, int shifted) {
     __shared__ int hist[kPmeBinLds];
     __shared__ int base[kPmeBinLds];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -129,8 +134,9 @@ __global__ void __launch_bounds__(256) k_pme_bin(PmeDesc D, PmePtrs P, const dou
         double w[3], xi[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
         if (d) {
             for (int k = 0; k < 3; ++k) {
-                xi[k] += d[3 * i + k];
-                P.x2[3 * i + k] = xi[k];
+                const double v = xi[k] + d[3 * i + k];
+                P.x2[3 * i + k] = v;
+                if (shifted) xi[k] = v;
             }
         }
         const int cx = wrap_cell(xi[0], D.L[0], D.invL[0], D.m[0], &w[0]);
@@ -199,6 +205,20 @@ __global__ void __launch_bounds__(256) k_pme_cellsort(PmeDesc D, PmePtrs P) {
     }
 }
 
+// erfc(alpha r)/r Coulomb + LJ of one pair from r^2 (qq = k_e q q', sg = mixed sigma,
+// e4 = 4 eps): the energy; fs, the force over the separation.
+__device__ __forceinline__ double direct_pair(const PmeDesc& D, double r2, double qq, double sg, double e4, double& fs) {
+    const double a = D.alpha;
+    const double rinv = 1.0 / sqrt(r2);
+    const double r = r2 * rinv, r2inv = rinv * rinv;
+    const double ec = qq * erfc(a * r) * rinv;
+    const double s2 = sg * sg * r2inv, s6 = s2 * s2 * s2;
+    const double t = e4 * s6;
+    const double elj = fma(t, s6, -t);
+    fs = (ec + qq * D.twoAlphaSqrtPi * exp(-a * a * r2) + fma(12.0, elj, 6.0 * t)) * r2inv;
+    return ec + elj;
+}
+
 // Half shell: blockIdx.x = 0 is cell c = blockIdx.y itself (pairs with the
 // j slot above the i slot), 1..13 its forward neighbour cells (all pairs);
 // blockIdx.z = chunk of 64 atoms of c (one per lane).  Every pair is visited
@@ -264,7 +284,7 @@ __global__ void __launch_bounds__(64) k_pme_direct(PmeDesc D, PmePtrs P, unsigne
     const int jall = nb == 0 ? s0 + chunk * 64 + 1 : j0;
     const int jlen = max(0, j1 - jall);
     const int jstart = jall + (jlen * part) / kPmeJSplit, jend = jall + (jlen * (part + 1)) / kPmeJSplit;
-    const double a = D.alpha, a2pi = D.twoAlphaSqrtPi, rc2 = D.rc2;
+    const double rc2 = D.rc2;
     double e = 0.0;
     int head = 0, tail = 0;  // ring [head, tail) of pending pairs (wave-uniform)
     const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -280,16 +300,8 @@ __global__ void __launch_bounds__(64) k_pme_direct(PmeDesc D, PmePtrs P, unsigne
             const double2 jp = sJp[k];
             const double dx = p.x - pj.x, dy = p.y - pj.y, dz = p.z - pj.z;
             const double r2 = dx * dx + dy * dy + dz * dz;
-            const double rinv = 1.0 / sqrt(r2);
-            const double r = r2 * rinv, r2inv = rinv * rinv;
-            const double qq = p.w * pj.w;
-            const double ec = qq * erfc(a * r) * rinv;
-            const double sg = ip.x + jp.x, e4 = ip.y * jp.y;
-            const double s2 = sg * sg * r2inv, s6 = s2 * s2 * s2;
-            const double t = e4 * s6;
-            const double elj = fma(t, s6, -t);
-            const double fs = (ec + qq * a2pi * exp(-a * a * r2) + fma(12.0, elj, 6.0 * t)) * r2inv;
-            e += ec + elj;
+            double fs;
+            e += direct_pair(D, r2, p.w * pj.w, ip.x + jp.x, ip.y * jp.y, fs);
             const long long fx = __double2ll_rn(fs * dx * kFix), fy = __double2ll_rn(fs * dy * kFix);
             const long long fz = __double2ll_rn(fs * dz * kFix);
             atomicAdd(&sF[0][il], (unsigned long long)fx);
@@ -358,7 +370,130 @@ __global__ void __launch_bounds__(64) k_pme_direct(PmeDesc D, PmePtrs P, unsigne
     if (lane == 0) eslot[blockSlot] = e;
 }
 
-__global__ void k_pme_spread(PmeDesc D, PmePtrs P, const double* x) {
+// Direct space of x + d as the difference from x (the displaced atoms are few): one
+// wave per (displaced atom k, neighbour cell, state): the pairs of atom k at that
+// state with the cell's atoms that are not displaced, at x (-) and at x + d (+); the
+// first cell's wave also takes the displaced atoms after k that are displaced
+// differently (atoms displaced alike keep their separation).  Energies into the
+// state-1 direct slots, forces into state 1's sums.  10 us for the 21-atom ligand of an
+// 8,479-atom system, where a second cell list and direct pass took 79; one wave per
+// neighbour cell because a wave walking all 27 waits on memory 50 times in a row.
+__global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P, unsigned long long* F, double* eslot) {
+    const int lane = threadIdx.x, cellOff = blockIdx.x >> 1, st = blockIdx.x & 1, k = blockIdx.y;
+    const int a = P.lig[k];
+    const double* X = st ? P.x2 : P.x;
+    double w[3];
+    const int c0 = wrap_cell(X[3 * a], D.L[0], D.invL[0], D.m[0], &w[0]);
+    const int c1 = wrap_cell(X[3 * a + 1], D.L[1], D.invL[1], D.m[1], &w[1]);
+    const int c2 = wrap_cell(X[3 * a + 2], D.L[2], D.invL[2], D.m[2], &w[2]);
+    int nx = c0 + cellOff / 9 - 1, ny = c1 + (cellOff / 3) % 3 - 1, nz = c2 + cellOff % 3 - 1;
+    double px = w[0], py = w[1], pz = w[2];  // the atom's image next to the neighbour cell
+    if (nx < 0) { nx += D.m[0]; px += D.L[0]; } else if (nx >= D.m[0]) { nx -= D.m[0]; px -= D.L[0]; }
+    if (ny < 0) { ny += D.m[1]; py += D.L[1]; } else if (ny >= D.m[1]) { ny -= D.m[1]; py -= D.L[1]; }
+    if (nz < 0) { nz += D.m[2]; pz += D.L[2]; } else if (nz >= D.m[2]) { nz -= D.m[2]; pz -= D.L[2]; }
+    const int cn = (nx * D.m[1] + ny) * D.m[2] + nz;
+    const int4 xa = P.exkey[a];
+    const double2 pa = P.prm2[a];
+    const double qa = P.prm[a].x;
+    const double dax = P.displ[3 * a], day = P.displ[3 * a + 1], daz = P.displ[3 * a + 2];
+    const double sgn = st ? 1.0 : -1.0;
+    double e = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+    auto pair = [&](int b, double dx, double dy, double dz, double r2, int grp, int rank, double qb, double2 pb) {
+        if (grp == xa.x && ((P.exbits[xa.z + (rank >> 5)] >> (rank & 31)) & 1u)) return;
+        double fs;
+        e += direct_pair(D, r2, qa * qb, pa.x + pb.x, pa.y * pb.y, fs);
+        const double gx = sgn * fs * dx, gy = sgn * fs * dy, gz = sgn * fs * dz;
+        fx += gx; fy += gy; fz += gz;
+        add_fixed(F + b, -gx);
+        add_fixed(F + D.n + b, -gy);
+        add_fixed(F + 2ll * D.n + b, -gz);
+    };
+    const int j0 = P.cellStart[cn], j1 = min(P.cellStart[cn + 1], j0 + kPmeCellMax);
+    for (int j = j0 + lane; j < j1; j += 64) {
+        const double4 pj = P.cpos[j];
+        const double dx = px - pj.x, dy = py - pj.y, dz = pz - pj.z;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        if (!(r2 < D.rc2)) continue;
+        const int4 xj = P.cex[j];
+        const double* db = P.displ + 3ll * xj.w;
+        if (db[0] != 0.0 || db[1] != 0.0 || db[2] != 0.0) continue;  // displaced itself: below
+        pair(xj.w, dx, dy, dz, r2, xj.x, xj.y, pj.w, P.cprm[j]);
+    }
+    if (cellOff == 0)
+        for (int q = k + 1 + lane; q < D.nlig; q += 64) {
+            const int b = P.lig[q];
+            const double* db = P.displ + 3ll * b;
+            if (db[0] == dax && db[1] == day && db[2] == daz) continue;
+            double v[3];
+            wrap_cell(X[3 * b], D.L[0], D.invL[0], D.m[0], &v[0]);
+            wrap_cell(X[3 * b + 1], D.L[1], D.invL[1], D.m[1], &v[1]);
+            wrap_cell(X[3 * b + 2], D.L[2], D.invL[2], D.m[2], &v[2]);
+            double dx = w[0] - v[0], dy = w[1] - v[1], dz = w[2] - v[2];
+            dx -= D.L[0] * rint(dx * D.invL[0]);
+            dy -= D.L[1] * rint(dy * D.invL[1]);
+            dz -= D.L[2] * rint(dz * D.invL[2]);
+            const double r2 = dx * dx + dy * dy + dz * dz;
+            if (!(r2 < D.rc2)) continue;
+            const int4 xb = P.exkey[b];
+            pair(b, dx, dy, dz, r2, xb.x, xb.y, P.prm[b].x, P.prm2[b]);
+        }
+    e = wave_sum(e);
+    fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
+    if (lane == 0) {
+        eslot[(27 * k + cellOff) * 2 + st] = sgn * e;
+        if (fx != 0.0) add_fixed(F + a, fx);
+        if (fy != 0.0) add_fixed(F + D.n + a, fy);
+        if (fz != 0.0) add_fixed(F + 2ll * D.n + a, fz);
+    }
+}
+
+// One axis' place on the grid of a position: scaled coordinate u (grid index floor(u)).
+// tiles: from the wrapped position, as the tile kernel spreads; otherwise as k_pme_spread.
+__device__ __forceinline__ double grid_coord(const PmeDesc& D, double x, int d, bool tiles) {
+    if (tiles) {
+        double w;
+        wrap_cell(x, D.L[d], D.invL[d], D.m[d], &w);
+        return w * D.invL[d] * D.K[d];
+    }
+    double f = x * D.invL[d];
+    f -= floor(f);
+    return f * D.K[d];
+}
+
+// The displaced atoms' charges off the grid at x and onto it at x + d, into the
+// difference grid: by the formulas of the spreading kernels, so that grid + difference is
+// the grid of x + d.  One task per (atom, state, first B-spline index).
+__device__ void spread_difference(const PmeDesc& D, const PmePtrs& P, int task) {
+    const int a = task % kOrder, st = (task / kOrder) & 1, i = P.lig[task / (2 * kOrder)];
+    const double q = P.prm[i].y;
+    if (q == 0.0) return;
+    const double* X = st ? P.x2 : P.x;
+    double th[3][kOrder], dth[kOrder];
+    int g0[3];
+    for (int d = 0; d < 3; ++d) {
+        const double u = grid_coord(D, X[3 * i + d], d, D.tileBytes > 0);
+        g0[d] = (int)floor(u);
+        bspline5(u - g0[d], th[d], dth);
+    }
+    unsigned long long* G = reinterpret_cast<unsigned long long*>(P.qgrid) + D.ngrid;
+    const int ia = wrap_index(g0[0] - a, D.K[0]);
+    for (int b = 0; b < kOrder; ++b) {
+        const int ib = wrap_index(g0[1] - b, D.K[1]);
+        const double qab = q * th[0][a] * th[1][b];
+        for (int cc = 0; cc < kOrder; ++cc) {
+            const int ic = wrap_index(g0[2] - cc, D.K[2]);
+            const long long v = __double2ll_rn(qab * th[2][cc] * kGridFix);
+            atomicAdd(G + ((long long)ia * D.K[1] + ib) * D.K[2] + ic, (unsigned long long)(st ? v : -v));
+        }
+    }
+}
+
+__global__ void k_pme_spread_difference(PmeDesc D, PmePtrs P) {
+    const int task = blockIdx.x * blockDim.x + threadIdx.x;
+    if (task < D.nlig * 2 * kOrder) spread_difference(D, P, task);
+}
+
+__global__ void k_pme_spread(PmeDesc D, PmePtrs P, const double* x, unsigned long long* grid) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= D.n) return;
     const double q = P.prm[i].y;
@@ -381,23 +516,31 @@ __global__ void k_pme_spread(PmeDesc D, PmePtrs P, const double* x) {
             const double qab = q * th[0][a] * th[1][b];
             for (int cc = 0; cc < kOrder; ++cc) {
                 const int ic = ((g0[2] - cc) % D.K[2] + D.K[2]) % D.K[2];
-                atomicAdd(reinterpret_cast<unsigned long long*>(P.qgrid) + ((long long)ia * D.K[1] + ib) * D.K[2] + ic,
+                atomicAdd(grid + ((long long)ia * D.K[1] + ib) * D.K[2] + ic,
                           (unsigned long long)__double2ll_rn(qab * th[2][cc] * kGridFix));
             }
         }
     }
 }
 
+// Charge at grid point k of a state, in fixed-point units.
+__device__ __forceinline__ long long grid_charge(const PmeDesc& D, const long long* q, int state, int k) {
+    return state == 0 ? q[k] : q[D.ngrid + k] + (D.delta ? q[k] : 0ll);
+}
+
 __global__ void k_pme_q2c(PmeDesc D, PmePtrs P) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= D.ngrid) return;
-    P.g0[k] = make_double2((double)P.qgrid[k] * (1.0 / kGridFix), 0.0);
+    const int st = blockIdx.y;
+    P.g0[(long long)st * D.ngrid + k] = make_double2((double)grid_charge(D, P.qgrid, st, k) * (1.0 / kGridFix), 0.0);
 }
 
 // One axis of an unnormalised complex DFT: out[..k..] = sum_j in[..j..] e^{sign 2 pi i j k / K}.
 __global__ void k_pme_dft(PmeDesc D, const double2* in, double2* out, const double2* tw, int axis, double sign) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= D.ngrid) return;
+    in += (long long)blockIdx.y * D.ngrid;  // blockIdx.y: state
+    out += (long long)blockIdx.y * D.ngrid;
     const int K = D.K[axis];
     const int stride = axis == 2 ? 1 : (axis == 1 ? D.K[2] : D.K[1] * D.K[2]);
     const int k = (idx / stride) % K;
@@ -424,6 +567,8 @@ __global__ void k_pme_dft(PmeDesc D, const double2* in, double2* out, const doub
 __global__ void __launch_bounds__(256) k_pme_dft_lines(PmeDesc D, const double2* in, double2* out, const double2* tw,
                                                       int axis, double sign, const long long* qfix) {
     extern __shared__ double2 sm[];
+    in += (long long)blockIdx.y * D.ngrid;  // blockIdx.y: state
+    out += (long long)blockIdx.y * D.ngrid;
     const int K = D.K[axis];
     const int stride = axis == 2 ? 1 : (axis == 1 ? D.K[2] : D.K[1] * D.K[2]);
     const int nlines = D.ngrid / K;
@@ -436,7 +581,8 @@ __global__ void __launch_bounds__(256) k_pme_dft_lines(PmeDesc D, const double2*
     if (L < nlines) {
         base = (L / stride) * K * stride + L % stride;
         if (qfix)
-            for (int j = lane; j < K; j += 64) line[j] = make_double2((double)qfix[base + j * stride] * (1.0 / kGridFix), 0.0);
+            for (int j = lane; j < K; j += 64) 
+                line[j] = make_double2((double)grid_charge(D, qfix, blockIdx.y, base + j * stride) * (1.0 / kGridFix), 0.0);
         else
             for (int j = lane; j < K; j += 64) line[j] = in[base + j * stride];
     }
@@ -463,8 +609,13 @@ __global__ void __launch_bounds__(256) k_pme_dft_lines(PmeDesc D, const double2*
 // point.  The tile covers grid indices [o, o + T) per axis with
 // o = floor(c K / m) - 5 and T = D.tile[axis]; a point outside it (rounding at
 // the cell edge) goes straight to the global grid.
-__global__ void __launch_bounds__(256) k_pme_spread_tiles(PmeDesc D, PmePtrs P) {
+__global__ void __launch_bounds__(256) k_pme_spread_tiles(PmeDesc D, PmePtrs P, unsigned long long* grid) {
     extern __shared__ unsigned long long tile[];
+    if ((int)blockIdx.x >= D.ncell * kPmeSpreadSplit) {  // the last blocks: the displaced atoms
+        const int task = ((int)blockIdx.x - D.ncell * kPmeSpreadSplit) * 256 + threadIdx.x;
+        if (task < D.nlig * 2 * kOrder) spread_difference(D, P, task);
+        return;
+    }
     // block (c, part): part `part` of kPmeSpreadSplit contiguous parts of cell c's atoms
     const int c = blockIdx.x / kPmeSpreadSplit, part = blockIdx.x % kPmeSpreadSplit;
     const int cz = c % D.m[2], cy = (c / D.m[2]) % D.m[1], cx = c / (D.m[1] * D.m[2]);
@@ -502,7 +653,7 @@ __global__ void __launch_bounds__(256) k_pme_spread_tiles(PmeDesc D, PmePtrs P) 
                     const int ia = wrap_index(g0[0] - a, D.K[0]);
                     const int ib = wrap_index(g0[1] - b, D.K[1]);
                     const int ic = wrap_index(g0[2] - cc, D.K[2]);
-                    atomicAdd(reinterpret_cast<unsigned long long*>(P.qgrid) + ((long long)ia * D.K[1] + ib) * D.K[2] + ic, v);
+                    atomicAdd(grid + ((long long)ia * D.K[1] + ib) * D.K[2] + ic, v);
                 }
             }
         }
@@ -516,25 +667,31 @@ __global__ void __launch_bounds__(256) k_pme_spread_tiles(PmeDesc D, PmePtrs P) 
         const int ia = wrap_index(o[0] + la, D.K[0]);
         const int ib = wrap_index(o[1] + lb, D.K[1]);
         const int ic = wrap_index(o[2] + lc, D.K[2]);
-        atomicAdd(reinterpret_cast<unsigned long long*>(P.qgrid) + ((long long)ia * D.K[1] + ib) * D.K[2] + ic, v);
+        atomicAdd(grid + ((long long)ia * D.K[1] + ib) * D.K[2] + ic, v);
     }
+}
+
+// The influence function at frequency indices (a, b, c): exp(-pi^2 m^2 / alpha^2) / (m^2 B),
+// 0 at m = 0.
+__device__ __forceinline__ double influence(const PmeDesc& D, const PmePtrs& P, int a, int b, int c) {
+    const double mx = (a <= D.K[0] / 2 ? a : a - D.K[0]) * D.invL[0];
+    const double my = (b <= D.K[1] / 2 ? b : b - D.K[1]) * D.invL[1];
+    const double mz = (c <= D.K[2] / 2 ? c : c - D.K[2]) * D.invL[2];
+    const double m2 = mx * mx + my * my + mz * mz;
+    if ((a | b | c) == 0) return 0.0;
+    const double B = P.bmod[a] * P.bmod[D.K[0] + b] * P.bmod[D.K[0] + D.K[1] + c];
+    return exp(-D.pi2OverAlpha2 * m2) / (m2 * B);
 }
 
 __global__ void __launch_bounds__(256) k_pme_convolve(PmeDesc D, PmePtrs P, double2* g, double* eslot) {
     __shared__ double red[4];
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    g += (long long)blockIdx.y * D.ngrid;  // blockIdx.y: state
+    eslot += (long long)blockIdx.y * D.nslot;
     double e = 0.0;
     if (idx < D.ngrid) {
         const int c = idx % D.K[2], b = (idx / D.K[2]) % D.K[1], a = idx / (D.K[1] * D.K[2]);
-        const double mx = (a <= D.K[0] / 2 ? a : a - D.K[0]) * D.invL[0];
-        const double my = (b <= D.K[1] / 2 ? b : b - D.K[1]) * D.invL[1];
-        const double mz = (c <= D.K[2] / 2 ? c : c - D.K[2]) * D.invL[2];
-        const double m2 = mx * mx + my * my + mz * mz;
-        double w = 0.0;
-        if (idx != 0) {
-            const double B = P.bmod[a] * P.bmod[D.K[0] + b] * P.bmod[D.K[0] + D.K[1] + c];
-            w = exp(-D.pi2OverAlpha2 * m2) / (m2 * B);
-        }
+        const double w = influence(D, P, a, b, c);
         const double2 f = g[idx];
         e = w * (f.x * f.x + f.y * f.y);
         g[idx] = make_double2(w * f.x, w * f.y);
@@ -543,11 +700,164 @@ __global__ void __launch_bounds__(256) k_pme_convolve(PmeDesc D, PmePtrs P, doub
     if (threadIdx.x == 0) eslot[blockIdx.x] = s * D.recipEnergyScale;
 }
 
+// ------------------------------------------------ fused transforms
+// A length-K axis, K = A B, is transformed in two short steps over an array in LDS
+// (positions `as` elements apart), in place: with n = B n1 + n2 and k = k1 + A k2,
+//   y[k1, n2] = W_K^{n2 k1} sum_{n1} x[B n1 + n2] W_K^{B n1 k1}   (at position B k1 + n2)
+//   X[k1, k2] =             sum_{n2} y[k1, n2]    W_K^{A n2 k2}   (at position B k1 + k2)
+// and backwards the same two steps in reverse order with conjugate twiddles, so
+// frequency k1 + A k2 sits at position B k1 + k2 between the two transforms and no
+// reordering pass is needed.  Each output costs A or B products instead of K.  Results
+// wait in registers while the block still reads the inputs.
+// Three launches for both states instead of seven per state (35 x 40 x 35: 34 us instead
+// of 70, 105 x 40 x 35: 44 instead of 90); what is left is LDS reads (two 16-byte reads
+// per product) and launches that fill a quarter of the chip.
+__device__ __forceinline__ int div_small(int v, float inv) { return (int)(((float)v + 0.5f) * inv); }
+
+// stepA: sums over n1 (or k1); otherwise over n2 (or k2).  twiddle: times W_K^{n2 k1}.
+__device__ __forceinline__ void dft_step(double2* buf, const double2* tw, int total, int K, int A, int as, bool stepA,
+                                         bool twiddle, double sign) {
+    const int B = K / A;
+    const float invAs = 1.0f / as, invK = 1.0f / K, invB = 1.0f / B;
+    double2 out[kPmeFuseMax / kPmeFuseNT];
+#pragma unroll
+    for (int u = 0; u < kPmeFuseMax / kPmeFuseNT; ++u) {
+        const int e = threadIdx.x + u * kPmeFuseNT;
+        if (e < total) {
+            const int row = div_small(e, invAs);
+            const int pos = row - div_small(row, invK) * K;
+            const int hi = div_small(pos, invB), lo = pos - hi * B;  // position B hi + lo
+            // summed positions: stepA B n + lo (n < A), else B hi + n (n < B)
+            const double2* v = buf + e - (stepA ? hi * B : lo) * as;
+            const int R = stepA ? A : B, es = stepA ? B * as : as, dt = stepA ? B * hi : A * lo;
+            double re = 0.0, im = 0.0;
+            int t = 0;
+            for (int n = 0; n < R; ++n) {
+                const double2 x = v[n * es], c = tw[t];
+                const double sn = sign * c.y;
+                re += x.x * c.x - x.y * sn;
+                im += x.y * c.x + x.x * sn;
+                t += dt;
+                if (t >= K) t -= K;
+            }
+            if (twiddle) {
+                const double2 c = tw[hi * lo];  // hi < A, lo < B: below K
+                const double sn = sign * c.y, r2 = re * c.x - im * sn;
+                im = im * c.x + re * sn;
+                re = r2;
+            }
+            out[u] = make_double2(re, im);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kPmeFuseMax / kPmeFuseNT; ++u) {
+        const int e = threadIdx.x + u * kPmeFuseNT;
+        if (e < total) buf[e] = out[u];
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ void dft_axis(double2* buf, const double2* tw, int total, int K, int A, int as, bool forward) {
+    if (forward) {
+        if (A > 1) dft_step(buf, tw, total, K, A, as, true, true, -1.0);
+        dft_step(buf, tw, total, K, A, as, false, false, -1.0);
+    } else {
+        dft_step(buf, tw, total, K, A, as, false, A > 1, 1.0);
+        if (A > 1) dft_step(buf, tw, total, K, A, as, true, false, 1.0);
+    }
+}
+
+// Axis strides of the grid arrays.
+__device__ __forceinline__ int axis_stride(const PmeDesc& D, int ax) {
+    return ax == 2 ? 1 : (ax == 1 ? D.K[2] : D.K[1] * D.K[2]);
+}
+
+// One plane (axes pAx, qAx) at position blockIdx.x of the line axis, state blockIdx.y, in LDS.
+// FORWARD: from the fixed-point charges to g0; otherwise from g0 to the real potential.
+template <bool FORWARD>
+__global__ void __launch_bounds__(kPmeFuseNT) k_pme_planes(PmeDesc D, PmePtrs P) {
+    extern __shared__ double2 sm[];
+    const int Kp = D.K[D.pAx], Kq = D.K[D.qAx], total = Kp * Kq, st = blockIdx.y;
+    double2 *twp = sm + total, *twq = twp + Kp;
+    for (int t = threadIdx.x; t < Kp; t += kPmeFuseNT) twp[t] = P.tw[D.twOff[D.pAx] + t];
+    for (int t = threadIdx.x; t < Kq; t += kPmeFuseNT) twq[t] = P.tw[D.twOff[D.qAx] + t];
+    const int sP = axis_stride(D, D.pAx), sQ = axis_stride(D, D.qAx);
+    const int base = blockIdx.x * axis_stride(D, D.lineAx);
+    const float invKq = 1.0f / Kq;
+    double2* g = P.g0 + (long long)st * D.ngrid;
+    for (int e = threadIdx.x; e < total; e += kPmeFuseNT) {
+        const int p = div_small(e, invKq), at = base + p * sP + (e - p * Kq) * sQ;
+        sm[e] = FORWARD ? make_double2((double)grid_charge(D, P.qgrid, st, at) * (1.0 / kGridFix), 0.0) : g[at];
+    }
+    __syncthreads();
+    dft_axis(sm, twq, total, Kq, D.fA[D.qAx], 1, FORWARD);
+    dft_axis(sm, twp, total, Kp, D.fA[D.pAx], Kq, FORWARD);
+    double* phi = reinterpret_cast<double*>(P.g1) + (long long)st * D.ngrid;
+    for (int e = threadIdx.x; e < total; e += kPmeFuseNT) {
+        const int p = div_small(e, invKq), at = base + p * sP + (e - p * Kq) * sQ;
+        if (FORWARD) g[at] = sm[e]; else phi[at] = sm[e].x;
+    }
+}
+
+// lineTile lines along the line axis (blockIdx.x), state blockIdx.y: forward transform,
+// convolution with the influence function (reciprocal energy into the block's slot),
+// backward transform.
+__global__ void __launch_bounds__(kPmeFuseNT) k_pme_lines(PmeDesc D, PmePtrs P, double* eslot) {
+    extern __shared__ double2 sm[];
+    __shared__ double red[kPmeFuseNT / 64];
+    const int K = D.K[D.lineAx], T = D.lineTile, Kq = D.K[D.qAx], nl = D.K[D.pAx] * Kq, st = blockIdx.y;
+    double2* tw = sm + K * T;
+    for (int t = threadIdx.x; t < K; t += kPmeFuseNT) tw[t] = P.tw[D.twOff[D.lineAx] + t];
+    const int sL = axis_stride(D, D.lineAx), sP = axis_stride(D, D.pAx), sQ = axis_stride(D, D.qAx);
+    const float invT = 1.0f / T, invKq = 1.0f / Kq;
+    double2* g = P.g0 + (long long)st * D.ngrid;
+    const int l0 = blockIdx.x * T, total = K * T;
+    for (int e = threadIdx.x; e < total; e += kPmeFuseNT) {
+        const int pos = div_small(e, invT), l = l0 + e - pos * T;
+        const int p = l / Kq;
+        sm[e] = l < nl ? g[p * sP + (l - p * Kq) * sQ + pos * sL] : make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    const int A = D.fA[D.lineAx];
+    dft_axis(sm, tw, total, K, A, T, true);
+    // the frequency at position B hi + lo is hi + A lo
+    auto freq = [&](int ax, int pos) {
+        const int a = D.fA[ax], b = D.K[ax] / a;
+        return pos / b + a * (pos % b);
+    };
+    double e0 = 0.0;
+    for (int e = threadIdx.x; e < total; e += kPmeFuseNT) {
+        const int pos = div_small(e, invT), l = l0 + e - pos * T;
+        if (l < nl) {
+            const int p = div_small(l, invKq);
+            int f[3];
+            const int fl = freq(D.lineAx, pos), fp = freq(D.pAx, p), fq = freq(D.qAx, l - p * Kq);
+            f[0] = D.lineAx == 0 ? fl : (D.pAx == 0 ? fp : fq);
+            f[1] = D.lineAx == 1 ? fl : (D.pAx == 1 ? fp : fq);
+            f[2] = D.lineAx == 2 ? fl : (D.pAx == 2 ? fp : fq);
+            const double w = influence(D, P, f[0], f[1], f[2]);
+            const double2 v = sm[e];
+            e0 += w * (v.x * v.x + v.y * v.y);
+            sm[e] = make_double2(w * v.x, w * v.y);
+        }
+    }
+    const double s = block_sum<kPmeFuseNT>(e0, red);  // (its barriers also order the products above)
+    if (threadIdx.x == 0) eslot[(long long)st * D.nslot + blockIdx.x] = s * D.recipEnergyScale;
+    dft_axis(sm, tw, total, K, A, T, false);
+    for (int e = threadIdx.x; e < total; e += kPmeFuseNT) {
+        const int pos = div_small(e, invT), l = l0 + e - pos * T;
+        const int p = l / Kq;
+        if (l < nl) g[p * sP + (l - p * Kq) * sQ + pos * sL] = sm[e];
+    }
+}
+
 // Reciprocal forces, 8 lanes per atom: lane a < 5 of the octet sums the 25 grid
 // points of B-spline index a, then the octet adds its partial gradients
 // (xor shuffles 1, 2, 4; lanes 5-7 add zeros).  Eight atoms per wave.
-__global__ void __launch_bounds__(256) k_pme_gather(PmeDesc D, PmePtrs P, const double* x, const double2* phi,
-                                                   unsigned long long* F) {
+// phi: the potentials of the states, ps doubles apart per point (1: real, 2: complex).
+__device__ __forceinline__ void gather_forces(const PmeDesc& D, const PmePtrs& P, const double* x, const double* phi,
+                                              int ps, unsigned long long* F) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int i = t >> 3, a = t & 7;
     const bool on = i < D.n;
@@ -579,7 +889,7 @@ __global__ void __launch_bounds__(256) k_pme_gather(PmeDesc D, PmePtrs P, const 
             const long long row = ((long long)ia * D.K[1] + ib) * D.K[2];
 #pragma unroll
             for (int cc = 0; cc < kOrder; ++cc) {
-                const double p = phi[row + ic[cc]].x;
+                const double p = phi[(row + ic[cc]) * ps];
                 gx += dt0 * th[1][b] * th[2][cc] * p;
                 gy += t0 * dth[1][b] * th[2][cc] * p;
                 gz += t0 * th[1][b] * dth[2][cc] * p;
@@ -599,10 +909,11 @@ __global__ void __launch_bounds__(256) k_pme_gather(PmeDesc D, PmePtrs P, const 
     }
 }
 
-__global__ void __launch_bounds__(256) k_pme_exceptions(PmeDesc D, PmePtrs P, const double* x, unsigned long long* F,
-                                                        double* eslot) {
+// Exception pairs, one per thread of block `blk`.
+__device__ __forceinline__ void exception_pairs(const PmeDesc& D, const PmePtrs& P, const double* x, int blk,
+                                                unsigned long long* F, double* eslot) {
     __shared__ double red[4];
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = blk * 256 + threadIdx.x;
     double e = 0.0;
     if (k < D.nex) {
         const int2 pr = P.expairs[k];
@@ -631,7 +942,18 @@ __global__ void __launch_bounds__(256) k_pme_exceptions(PmeDesc D, PmePtrs P, co
         }
     }
     const double s = block_sum<256>(e, red);
-    if (threadIdx.x == 0) eslot[blockIdx.x] = s;
+    if (threadIdx.x == 0) eslot[blk] = s;
+}
+
+// Reciprocal forces (the first gatherBlocks blocks) and exception pairs of state blockIdx.y.
+__global__ void __launch_bounds__(256) k_pme_gather(PmeDesc D, PmePtrs P, const double* phi, int ps, int gatherBlocks) {
+    const int st = blockIdx.y;
+    const double* x = st ? P.x2 : P.x;
+    unsigned long long* F = P.F + 3ll * D.n * st;
+    if ((int)blockIdx.x < gatherBlocks)
+        gather_forces(D, P, x, phi + (long long)st * D.ngrid * ps, ps, F);
+    else
+        exception_pairs(D, P, x, (int)blockIdx.x - gatherBlocks, F, P.eslot + (long long)st * D.nslot + D.nslotDirect);
 }
 
 // Fixed-order sums of the energy slots of both states; U = sum + constants;
@@ -640,23 +962,27 @@ __global__ void __launch_bounds__(256) k_pme_exceptions(PmeDesc D, PmePtrs P, co
 __global__ void __launch_bounds__(1024) k_pme_finish(PmeDesc D, PmePtrs P, int single) {
     __shared__ double red[16];
     double U[2] = {0.0, 0.0};
+    double direct0 = 0.0;
     for (int s = 0; s < (single ? 1 : 2); ++s) {
         const double* sl = P.eslot + (long long)s * D.nslot;
-        const int ranges[4] = {0, D.nslotDirect, D.nslotDirect + D.nslotEx, D.nslot};
+        const int first[3] = {0, D.nslotDirect, D.nslotDirect + D.nslotEx};
+        const int last[3] = {D.nslotUsed[s], D.nslotDirect + D.nslotEx, D.nslot};
         double parts[3];
         for (int r = 0; r < 3; ++r) {
             // four independent partial sums per thread (fixed order): their loads overlap
             double v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
-            int k = ranges[r] + (int)threadIdx.x;
-            for (; k + 3 * 1024 < ranges[r + 1]; k += 4 * 1024) {
+            int k = first[r] + (int)threadIdx.x;
+            for (; k + 3 * 1024 < last[r]; k += 4 * 1024) {
                 v0 += sl[k];
                 v1 += sl[k + 1024];
                 v2 += sl[k + 2 * 1024];
                 v3 += sl[k + 3 * 1024];
             }
-            for (; k < ranges[r + 1]; k += 1024) v0 += sl[k];
+            for (; k < last[r]; k += 1024) v0 += sl[k];
             parts[r] = block_sum<1024>((v0 + v1) + (v2 + v3), red);
         }
+        if (s == 0) direct0 = parts[0];
+        else if (D.delta) parts[0] += direct0;  // the slots hold the difference
         if (threadIdx.x == 0) {
             P.parts[5 * s + 0] = parts[0];
             P.parts[5 * s + 1] = parts[1];
@@ -682,8 +1008,9 @@ __global__ void k_pme_blend(PmeDesc D, PmePtrs P, int single, double* out) {
     if (k >= 3 * D.n) return;
     const SysResult r = *P.result;
     const double a = single ? 0.0 : (P.params->direction > 0.0 ? r.sp : 1.0 - r.sp);  // weight of state 2 (x + d)
-    const double f1 = (double)(long long)P.F[k] * (1.0 / kFix);
-    const double f2 = single ? 0.0 : (double)(long long)P.F[3ll * D.n + k] * (1.0 / kFix);
+    const unsigned long long both = P.F[6ll * D.n + k];
+    const double f1 = (double)(long long)(P.F[k] + both) * (1.0 / kFix);
+    const double f2 = single ? 0.0 : (double)(long long)(P.F[3ll * D.n + k] + both) * (1.0 / kFix);
     const int comp = k / D.n, i = k % D.n;
     out[3 * i + comp] = (1.0 - a) * f1 + a * f2;
 }
@@ -713,49 +1040,80 @@ hipError_t launch_pme_fill(unsigned long long* p, long long n, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_pme_state(const PmeDesc& D, const PmePtrs& P, int state, hipStream_t st) {
-    const double* x = state == 0 ? P.x : P.x2;
-    unsigned long long* F = P.F + 3ll * D.n * state;
-    double* es = P.eslot + (long long)D.nslot * state;
-    {
-        const long long nc = (D.ncell + 1) / 2, ng = D.ngrid, nf = 3ll * D.n;
-        k_pme_fill3<<<blocks_of(nc + ng + nf, 256), 256, 0, st>>>(reinterpret_cast<unsigned long long*>(P.cellCount), nc,
-                                                                  reinterpret_cast<unsigned long long*>(P.qgrid), ng, F, nf);
-    }
-    // 256 threads: the histogram loops assume it; state 1 forms x + d here
-    k_pme_bin<<<blocks_of(D.n, 256), 256, 0, st>>>(D, P, state == 1 ? P.x : x, state == 1 ? P.displ : nullptr);
-    k_pme_scan<<<1, 1024, 0, st>>>(D, P);
-    k_pme_scatter<<<blocks_of(D.n, 256), 256, 0, st>>>(D, P);
-    k_pme_cellsort<<<D.ncell, 256, 0, st>>>(D, P);
+hipError_t launch_pme_states(const PmeDesc& D, const PmePtrs& P, bool single, hipStream_t st) {
+    const int ns = single ? 1 : 2;
+    unsigned long long* q0 = reinterpret_cast<unsigned long long*>(P.qgrid);
+    const bool delta = D.delta && !single;
+    // cell list of the positions of `state`, its direct space into F
+    auto cells = [&](int state, bool first) {
+        if (first) {
+            const long long nc = (D.ncell + 1) / 2, ng = (long long)ns * D.ngrid, nf = 9ll * D.n;
+            k_pme_fill3<<<blocks_of(nc + ng + nf, 256), 256, 0, st>>>(reinterpret_cast<unsigned long long*>(P.cellCount), nc,
+                                                                      q0, ng, P.F, nf);
+        } else {
+            launch_pme_fill(reinterpret_cast<unsigned long long*>(P.cellCount), (D.ncell + 1) / 2, st);
+        }
+        // 256 threads: the histogram loops assume it; the first call forms x + d
+        k_pme_bin<<<blocks_of(D.n, 256), 256, 0, st>>>(D, P, P.x, single ? nullptr : P.displ, state);
+        k_pme_scan<<<1, 1024, 0, st>>>(D, P);
+        k_pme_scatter<<<blocks_of(D.n, 256), 256, 0, st>>>(D, P);
+        k_pme_cellsort<<<D.ncell, 256, 0, st>>>(D, P);
+    };
+    auto spread = [&](int state) {
+        unsigned long long* grid = q0 + (long long)state * D.ngrid;
+        const unsigned lb = delta && state == 0 ? blocks_of((long long)D.nlig * 2 * kOrder, 256) : 0u;
+        if (D.tileBytes > 0) {  // the cell's grid tile fits in LDS
+            k_pme_spread_tiles<<<D.ncell * kPmeSpreadSplit + lb, 256, D.tileBytes, st>>>(D, P, grid);
+        } else {
+            k_pme_spread<<<blocks_of(D.n, 256), 256, 0, st>>>(D, P, state ? P.x2 : P.x, grid);
+            if (lb) k_pme_spread_difference<<<lb, 256, 0, st>>>(D, P);
+        }
+    };
     // neighbour offset fastest, chunk slowest: consecutive workgroups (dealt round-robin to the
     // XCDs) carry comparable work, and the mostly empty late chunks come last
-    k_pme_direct<<<dim3(kPmeHalfShell * kPmeJSplit, D.ncell, D.chunks), 64, 0, st>>>(D, P, F, es);
-    k_pme_exceptions<<<blocks_of(D.nex, 256) > 0 ? blocks_of(D.nex, 256) : 1, 256, 0, st>>>(D, P, x, F,
-                                                                                               es + D.nslotDirect);
-    if (D.tileBytes > 0)  // the cell's grid tile fits in LDS
-        k_pme_spread_tiles<<<D.ncell * kPmeSpreadSplit, 256, D.tileBytes, st>>>(D, P);
-    else
-        k_pme_spread<<<blocks_of(D.n, 256), 256, 0, st>>>(D, P, x);
+    const dim3 gridDirect(kPmeHalfShell * kPmeJSplit, D.ncell, D.chunks);
+    cells(0, true);
+    k_pme_direct<<<gridDirect, 64, 0, st>>>(D, P, delta ? P.F + 6ll * D.n : P.F, P.eslot);
+    spread(0);
+    if (delta) {
+        if (D.nlig > 0) k_pme_displaced<<<dim3(54, D.nlig), 64, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot);
+    } else if (!single) {
+        cells(1, false);
+        k_pme_direct<<<gridDirect, 64, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot);
+        spread(1);
+    }
+    const unsigned gatherBlocks = blocks_of(8ll * D.n, 256);
+    const dim3 gridGather(gatherBlocks + D.nslotEx, ns);
+    double* erec = P.eslot + D.nslotDirect + D.nslotEx;
+    if (D.fused) {
+        const int Kp = D.K[D.pAx], Kq = D.K[D.qAx], Kl = D.K[D.lineAx];
+        const size_t ldsPlane = (size_t)(Kp * Kq + Kp + Kq) * sizeof(double2);
+        k_pme_planes<true><<<dim3(Kl, ns), kPmeFuseNT, ldsPlane, st>>>(D, P);
+        k_pme_lines<<<dim3(D.lineBlocks, ns), kPmeFuseNT, (size_t)(D.lineTile + 1) * Kl * sizeof(double2), st>>>(D, P, erec);
+        k_pme_planes<false><<<dim3(Kl, ns), kPmeFuseNT, ldsPlane, st>>>(D, P);
+        k_pme_gather<<<gridGather, 256, 0, st>>>(D, P, reinterpret_cast<const double*>(P.g1), 1, gatherBlocks);
+        return hipGetLastError();
+    }
     const unsigned gb = blocks_of(D.ngrid, 256);
     auto dft = [&](const double2* in, double2* out, int axis, double sign, const long long* qfix = nullptr) {
         const int K = D.K[axis];
         if (K <= kPmeDftLdsMax) {
-            k_pme_dft_lines<<<blocks_of(D.ngrid / K, 4), 256, 5 * K * sizeof(double2), st>>>(D, in, out, P.tw + D.twOff[axis],
-                                                                                          axis, sign, qfix);
+            k_pme_dft_lines<<<dim3(blocks_of(D.ngrid / K, 4), ns), 256, 5 * K * sizeof(double2), st>>>(
+                D, in, out, P.tw + D.twOff[axis], axis, sign, qfix);
         } else {
-            if (qfix) k_pme_q2c<<<gb, 256, 0, st>>>(D, P);  // into g0 = in
-            k_pme_dft<<<gb, 256, 0, st>>>(D, in, out, P.tw + D.twOff[axis], axis, sign);
+            if (qfix) k_pme_q2c<<<dim3(gb, ns), 256, 0, st>>>(D, P);  // into g0 = in
+            k_pme_dft<<<dim3(gb, ns), 256, 0, st>>>(D, in, out, P.tw + D.twOff[axis], axis, sign);
         }
     };
     // first pass straight from the fixed-point charge grid
-    dft(P.g0, P.g1, 2, -1.0, reinterpret_cast<const long long*>(P.qgrid));
+    dft(P.g0, P.g1, 2, -1.0, P.qgrid);
     dft(P.g1, P.g0, 1, -1.0);
     dft(P.g0, P.g1, 0, -1.0);
-    k_pme_convolve<<<gb, 256, 0, st>>>(D, P, P.g1, es + D.nslotDirect + D.nslotEx);
+    k_pme_convolve<<<dim3(gb, ns), 256, 0, st>>>(D, P, P.g1, erec);
     dft(P.g1, P.g0, 0, 1.0);
     dft(P.g0, P.g1, 1, 1.0);
     dft(P.g1, P.g0, 2, 1.0);
-    k_pme_gather<<<blocks_of(8ll * D.n, 256), 256, 0, st>>>(D, P, x, P.g0, F);
+    k_pme_gather<<<gridGather, 256, 0, st>>>(D, P, reinterpret_cast<const double*>(P.g0), 2, gatherBlocks);
     return hipGetLastError();
 }
 

@@ -84,7 +84,7 @@ struct PmeForce {
 
     DevBuf dX, dX2, dDispl, dCellOf, dRankOf, dCellCount, dCellStart, dCellAtoms, dWpos, dPrm, dPrm2, dExkey;
     DevBuf dCpos, dCprm, dCex, dExbits, dExpairs, dExprm, dQgrid, dG0, dG1, dTw, dBmod, dF, dEslot, dParts;
-    DevBuf dResult, dOverflow, dOut, dParams;
+    DevBuf dResult, dOverflow, dOut, dParams, dLig;
     PmeDesc D{};
     PmePtrs P{};
     std::vector<double> hOut;
@@ -213,6 +213,16 @@ void setup(PmeForce& S) {
     upload(st, S.dTw, tw.data(), sizeof(double2) * tw.size());
     upload(st, S.dBmod, bmod.data(), sizeof(double) * bmod.size());
     upload(st, S.dDispl, S.displ.data(), sizeof(double) * 3 * n);
+    std::vector<int> lig;
+    for (int i = 0; i < n; ++i)
+        if (S.displ[3 * (size_t)i] != 0.0 || S.displ[3 * (size_t)i + 1] != 0.0 || S.displ[3 * (size_t)i + 2] != 0.0)
+            lig.push_back(i);
+    S.D.nlig = (int)lig.size();
+    // x + d as the difference from x: each displaced atom costs 54 waves over its neighbour
+    // cells, so only while they are few (a wave per 64 atoms of a cell pair covers the rest)
+    S.D.delta = 16ll * S.D.nlig <= n && S.D.nlig <= 65535;
+    if (lig.empty()) lig.push_back(0);
+    upload(st, S.dLig, lig.data(), sizeof(int) * lig.size());
     HIPCHK(hipStreamSynchronize(st));
     const long long ng = (long long)S.K[0] * S.K[1] * S.K[2];
     S.dX.alloc(sizeof(double) * 3 * n);
@@ -224,10 +234,10 @@ void setup(PmeForce& S) {
     S.dCpos.alloc(sizeof(double4) * n);
     S.dCprm.alloc(sizeof(double2) * n);
     S.dCex.alloc(sizeof(int4) * n);
-    S.dQgrid.alloc(sizeof(long long) * ng);
-    S.dG0.alloc(sizeof(double2) * ng);
-    S.dG1.alloc(sizeof(double2) * ng);
-    S.dF.alloc(sizeof(unsigned long long) * 6 * n);
+    S.dQgrid.alloc(sizeof(long long) * 2 * ng);
+    S.dG0.alloc(sizeof(double2) * 2 * ng);
+    S.dG1.alloc(sizeof(double2) * 2 * ng);
+    S.dF.alloc(sizeof(unsigned long long) * 9 * n);
     S.dParts.alloc(sizeof(double) * 10);
     S.dResult.alloc(sizeof(SysResult));
     S.dParams.alloc(sizeof(AtmParamsDev) + 2 * sizeof(double));  // parameters, then the two energy offsets
@@ -237,7 +247,24 @@ void setup(PmeForce& S) {
     S.D.n = n;
     S.D.nex = nex;
     S.D.ngrid = (int)ng;
-    for (int d = 0; d < 3; ++d) S.D.K[d] = S.K[d];
+    for (int d = 0; d < 3; ++d) {
+        S.D.K[d] = S.K[d];
+        S.D.fA[d] = 1;  // the largest factor not above the square root
+        for (int a = 2; a * a <= S.K[d]; ++a)
+            if (S.K[d] % a == 0) S.D.fA[d] = a;
+    }
+    // fused transforms: lines along the longest axis, planes over the other two, when both fit
+    // the block's LDS (64 KiB) and registers
+    S.D.lineAx = 0;
+    for (int d = 1; d < 3; ++d)
+        if (S.K[d] > S.K[S.D.lineAx]) S.D.lineAx = d;
+    S.D.pAx = S.D.lineAx == 0 ? 1 : 0;
+    S.D.qAx = S.D.lineAx == 2 ? 1 : 2;
+    const int Kp = S.K[S.D.pAx], Kq = S.K[S.D.qAx], Kl = S.K[S.D.lineAx];
+    S.D.lineTile = kPmeLineTile;
+    while (S.D.lineTile > 1 && (S.D.lineTile * Kl > kPmeFuseMax || (S.D.lineTile + 1) * Kl * 16 > 64000)) S.D.lineTile /= 2;
+    S.D.lineBlocks = (Kp * Kq + S.D.lineTile - 1) / S.D.lineTile;
+    S.D.fused = Kp * Kq <= kPmeFuseMax && (Kp * Kq + Kp + Kq) * 16 <= 65536;
     S.D.alpha = S.alpha;
     S.D.twoAlphaSqrtPi = 2.0 * S.alpha / std::sqrt(kPi);
     S.D.pi2OverAlpha2 = kPi * kPi / (S.alpha * S.alpha);
@@ -270,9 +297,11 @@ void set_box(PmeForce& S, const double box[3]) {
     cap = std::min(kPmeCellMax, (cap + 63) / 64 * 64);
     S.D.cellCap = cap;
     S.D.chunks = cap / 64;
-    S.D.nslotDirect = S.D.chunks * kPmeHalfShell * kPmeJSplit * S.D.ncell;
+    S.D.nslotUsed[0] = S.D.nslotUsed[1] = S.D.chunks * kPmeHalfShell * kPmeJSplit * S.D.ncell;
+    if (S.D.delta) S.D.nslotUsed[1] = 54 * S.D.nlig;
+    S.D.nslotDirect = std::max(S.D.nslotUsed[0], S.D.nslotUsed[1]);
     S.D.nslotEx = std::max(1, (S.D.nex + 255) / 256);
-    S.D.nslot = S.D.nslotDirect + S.D.nslotEx + (S.D.ngrid + 255) / 256;
+    S.D.nslot = S.D.nslotDirect + S.D.nslotEx + (S.D.fused ? S.D.lineBlocks : (S.D.ngrid + 255) / 256);
     // charge-grid tile of one cell: grid indices [floor(c K/m) - 5, ... + ceil(K/m) + 7)
     long long tb = 8;
     for (int d = 0; d < 3; ++d) {
@@ -293,6 +322,7 @@ void set_box(PmeForce& S, const double box[3]) {
     P.x = S.dX.as<double>();
     P.x2 = S.dX2.as<double>();
     P.displ = S.dDispl.as<double>();
+    P.lig = S.dLig.as<int>();
     P.cellOf = S.dCellOf.as<int>();
     P.rankOf = S.dRankOf.as<int>();
     P.cellCount = S.dCellCount.as<int>();
@@ -524,8 +554,7 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
                 hipGraph_t graph = nullptr;
                 HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
                 hipError_t e = launch_pme_fill(reinterpret_cast<unsigned long long*>(S.dOverflow.p), 1, st);
-                if (e == hipSuccess) e = launch_pme_state(S.D, S.P, 0, st);
-                if (e == hipSuccess && !single) e = launch_pme_state(S.D, S.P, 1, st);
+                if (e == hipSuccess) e = launch_pme_states(S.D, S.P, single, st);
                 if (e == hipSuccess) e = launch_pme_finish(S.D, S.P, single, forces ? S.dOut.as<double>() : nullptr, st);
                 const hipError_t ee = hipStreamEndCapture(st, &graph);
                 HIPCHK(e);
