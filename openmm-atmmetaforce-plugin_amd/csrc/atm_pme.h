@@ -8,8 +8,13 @@
 namespace atm {
 
 constexpr int kPmeCellMax = 1024;  // atoms per cell the cell sort holds
-constexpr int kPmeJBatch = 64;     // neighbour-cell atoms staged in LDS per batch (direct kernel)
-constexpr int kPmeJSplit = 4;      // parts of a neighbour cell's atoms taken by separate waves
+// Block of the direct kernel: atoms of a cell, atoms of its neighbour cell staged at a time, waves.
+// 48 us for 8,479 atoms and 120 for 25,437 (cells of some 133); (64, 160, 8) 55 / 156,
+// (64, 160, 2) 70 / 133, (128, 160, 8) 73 / 151, (192, 192, 8) 74 / 152.
+constexpr int kPmeIBlock = 64;
+constexpr int kPmeJBlock = 160;
+constexpr int kPmeDirectWaves = 4;
+constexpr int kPmeExWords = 4;       // words of each i-atom's exclusion row it stages (groups of up to 128 atoms)
 constexpr int kPmeSpreadSplit = 4; // parts of a cell's atoms spread by separate blocks (own LDS tiles)
 constexpr int kPmeHalfShell = 14;  // the cell itself and its 13 forward neighbour cells
 constexpr int kPmeBinLds = 4096;   // cell grids up to this size are binned through LDS histograms
@@ -23,7 +28,7 @@ constexpr int kPmeLineTile = 16;   // grid lines per block of the fused line ker
 struct PmeDesc {
     int n;                       // atoms
     int m[3], ncell;             // cell grid (edge >= rc, at least 3 per axis)
-    int cellCap, chunks;         // atoms per cell the direct kernel covers (chunks of 64)
+    int cellCap, chunks;         // atoms per cell the direct kernel covers (chunks of kPmeBlockAtoms)
     int K[3], ngrid;             // PME grid
     int twOff[3];                // offset of each axis' twiddle table
     int nex;                     // exception pairs

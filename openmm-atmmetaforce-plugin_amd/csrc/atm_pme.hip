@@ -10,9 +10,8 @@
 //                    positions / parameters / exclusion keys gathered into
 //                    cell order
 //   k_pme_direct     erfc(alpha r)/r Coulomb + LJ over minimum-image pairs with
-//                    r < rc that are not exceptions; one wave per (64 atoms of
-//                    a cell, the cell or one of its 13 forward neighbours, a
-//                    quarter of that cell's atoms): each pair once
+//                    r < rc that are not exceptions; one block per (cell, the
+//                    cell or one of its 13 forward neighbours): each pair once
 //   k_pme_spread_tiles  order-5 B-spline charge spreading per cell into an LDS
 //                    tile of the grid, 64-bit fixed point (k_pme_spread: the
 //                    same straight into the grid, when a tile does not fit)
@@ -56,6 +55,33 @@ constexpr int kOrder = 5;
 
 __device__ __forceinline__ void add_fixed(unsigned long long* p, double f) {
     atomicAdd(p, (unsigned long long)__double2ll_rn(f * kFix));
+}
+
+// Integer add in LDS (workgroup scope, no result).
+__device__ __forceinline__ void lds_add(unsigned long long* p, unsigned long long v) {
+    typedef __attribute__((address_space(3))) unsigned long long LdsU64;
+    __hip_atomic_fetch_add((LdsU64*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// A whole number below 2^51 as an integer: the low bits of its sum with 1.5 2^52.
+__device__ __forceinline__ long long whole(double v) {
+    return __double_as_longlong(v + 6755399441055744.0) - 0x4338000000000000LL;
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Sum over each aligned octet of lanes (xor 1, xor 2, half-row mirror by DPP).
+__device__ __forceinline__ double oct_sum(double v) {
+    v += dpp_f64<0xB1>(v);
+    v += dpp_f64<0x4E>(v);
+    v += dpp_f64<0x141>(v);
+    return v;
 }
 
 // Grid index v in [-K, 2K) wrapped into [0, K) (no integer division).
@@ -209,7 +235,13 @@ __global__ void __launch_bounds__(256) k_pme_cellsort(PmeDesc D, PmePtrs P) {
 // e4 = 4 eps): the energy; fs, the force over the separation.
 __device__ __forceinline__ double direct_pair(const PmeDesc& D, double r2, double qq, double sg, double e4, double& fs) {
     const double a = D.alpha;
-    const double rinv = 1.0 / sqrt(r2);
+    // 1/r: hardware estimate and two Newton steps on the residual 1 - r2 y^2 (an FMA)
+    double rinv = __builtin_amdgcn_rsq(r2);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const double t = r2 * rinv;
+        rinv = fma(0.5 * rinv, fma(-t, rinv, 1.0), rinv);
+    }
     const double r = r2 * rinv, r2inv = rinv * rinv;
     const double ec = qq * erfc(a * r) * rinv;
     const double s2 = sg * sg * r2inv, s6 = s2 * s2 * s2;
@@ -219,32 +251,47 @@ __device__ __forceinline__ double direct_pair(const PmeDesc& D, double r2, doubl
     return ec + elj;
 }
 
-// Half shell: blockIdx.x = 0 is cell c = blockIdx.y itself (pairs with the
-// j slot above the i slot), 1..13 its forward neighbour cells (all pairs);
-// blockIdx.z = chunk of 64 atoms of c (one per lane).  Every pair is visited
-// once: +f on i, -f on j, the whole pair energy.
-//  test:  the wave walks the neighbour cell's atoms staged in LDS; each lane
-//         tests its atom against the common j (FP64 r^2, the image shift known
-//         from the cell offset, exclusion bitmap for atoms of one exclusion
-//         group) and the in-range pairs are appended to a ring in LDS
-//         (ballot + mbcnt, so the order is fixed);
+// Half shell: neighbour 0 is cell c itself (pairs with the j slot above the i slot), 1..13
+// its forward neighbour cells (all pairs).  Every pair is visited once: +f on i, -f on j,
+// the whole pair energy.
+//
+// One block of 4 waves per (cell c, fastest; kPmeIBlock atoms of c; neighbour): those atoms
+// and, kPmeJBlock at a time, the neighbour cell's are staged in LDS with their force sums.
+// Each wave takes its share of the staged j-atoms against every i-atom:
+//  test:  lane il + n2 jg tests i-atom il of a chunk of up to 64 against j-atom k G + jg (a
+//         chunk of n2 = 8, 16, 32 or 64 i-atoms takes G = 64 / n2 j-atoms a step, so the 5
+//         atoms left of a cell of 133 cost an eighth of a full chunk).  FP64 r^2, the
+//         image shift known from the cell offset, exclusion bitmap for atoms of one
+//         exclusion group; in-range pairs are appended to the wave's ring in LDS (ballot +
+//         mbcnt, so the order is fixed);
 //  dense: whenever 64 pairs are pending, each lane evaluates one of them
-//         (erfc Coulomb + LJ in FP64); forces go to per-atom LDS accumulators
-//         of the chunk (i) and of the staged batch (j) in 64-bit fixed point
-//         (integer atomics: order-independent), flushed to global memory.
-__global__ void __launch_bounds__(64) k_pme_direct(PmeDesc D, PmePtrs P, unsigned long long* F, double* eslot) {
-    __shared__ double4 sI[64];
-    __shared__ double2 sIp[64];
-    __shared__ unsigned long long sF[3][64];
-    __shared__ uint32_t sQ[128];
-    __shared__ double4 sJ[kPmeJBatch];  // the neighbour cell's atoms of the current batch
-    __shared__ double2 sJp[kPmeJBatch];
-    __shared__ int4 sJx[kPmeJBatch];    // exclusion group, rank, -, atom
-    __shared__ unsigned long long sJF[3][kPmeJBatch];
-    const int lane = threadIdx.x;
-    // x: neighbour offset (fastest) and part of the neighbour cell's atoms; y: cell; z: 64-atom chunk
-    const int nb = blockIdx.x % kPmeHalfShell, part = blockIdx.x / kPmeHalfShell;
-    const int c = blockIdx.y, chunk = blockIdx.z;
+//         (erfc Coulomb + LJ in FP64); forces go to the block's LDS sums in 64-bit fixed
+//         point (integer atomics: order-independent).
+// The dense steps bound it (some 230 VALU instructions and six 64-bit LDS adds each):
+// pairs of one j-atom sit in consecutive lanes and their adds queue on one address, so an
+// octet of lanes of one j-atom adds up first (LDS conflict cycles halved, 85 -> 73 us with
+// blocks of 8 waves).  59 -> 48 us for 8,479 atoms, 151 -> 120 for 25,437, against one wave
+// per (64 atoms, neighbour, quarter of its atoms) with its own sums.
+__global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc D, PmePtrs P, unsigned long long* F,
+                                                                       double* eslot) {
+    constexpr int IB = kPmeIBlock, JB = kPmeJBlock, W = kPmeDirectWaves, NT = 64 * W;
+    __shared__ double4 sI[IB], sJ[JB];       // x, y, z, q sqrt(k_e); i-atoms shifted to the neighbour's image
+    __shared__ double2 sIp[IB], sJp[JB];
+    __shared__ int4 sIx[IB], sJx[JB];        // exclusion group, rank, row offset, atom
+    __shared__ uint32_t sIw[kPmeExWords][IB]; // first words of the i-atoms' exclusion rows
+    __shared__ unsigned long long sIF[3][IB], sJF[3][JB];
+    __shared__ uint32_t sQ[W][128];
+    __shared__ double sE[W];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // the cell itself, its face, edge and corner neighbours: most pairs first
+    constexpr unsigned long long order = 0xDB75CA86429310ull;
+    const int nb = (int)((order >> (4 * blockIdx.z)) & 15ull), c = blockIdx.x;
+    const int i0 = P.cellStart[c] + blockIdx.y * IB, ni = min(P.cellStart[c + 1] - i0, IB);
+    const int blockSlot = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + c;
+    if (ni <= 0) {  // no atom in this part of the cell
+        if (threadIdx.x == 0) eslot[blockSlot] = 0.0;
+        return;
+    }
     const int cz = c % D.m[2], cy = (c / D.m[2]) % D.m[1], cx = c / (D.m[1] * D.m[2]);
     // forward offsets: (a, b, e) lexicographically above (0, 0, 0); nb = 0 is the cell itself
     int ox = 0, oy = 0, oz = 0;
@@ -258,116 +305,149 @@ __global__ void __launch_bounds__(64) k_pme_direct(PmeDesc D, PmePtrs P, unsigne
     if (ny < 0) { ny += D.m[1]; sy = -D.L[1]; } else if (ny >= D.m[1]) { ny -= D.m[1]; sy = D.L[1]; }
     if (nz < 0) { nz += D.m[2]; sz = -D.L[2]; } else if (nz >= D.m[2]) { nz -= D.m[2]; sz = D.L[2]; }
     const int cn = (nx * D.m[1] + ny) * D.m[2] + nz;
-    const int s0 = P.cellStart[c], s1 = P.cellStart[c + 1];
-    const int blockSlot = (chunk * gridDim.y + c) * gridDim.x + blockIdx.x;
-    if (s0 + chunk * 64 >= s1) {  // no atom in this chunk: the whole block leaves
-        if (lane == 0) eslot[blockSlot] = 0.0;
-        return;
+    const int jend = P.cellStart[cn + 1];
+    // in the cell itself only j slots above the block's first slot can pair with it
+    const int jstart = nb == 0 ? i0 + 1 : P.cellStart[cn];
+    for (int k = threadIdx.x; k < ni; k += NT) {
+        double4 p = P.cpos[i0 + k];
+        p.x -= sx; p.y -= sy; p.z -= sz;  // (x_i - s) - x_j = x_i - (x_j + s)
+        sI[k] = p;
+        sIp[k] = P.cprm[i0 + k];
+        const int4 xk = P.cex[i0 + k];
+        sIx[k] = xk;
+#pragma unroll
+        for (int w = 0; w < kPmeExWords; ++w) sIw[w][k] = P.exbits[xk.z + w];  // (padded past the last row)
+        sIF[0][k] = 0ull; sIF[1][k] = 0ull; sIF[2][k] = 0ull;
     }
-    const int si = s0 + chunk * 64 + lane;
-    const bool active = si < s1;
-    double4 pi = make_double4(0.0, 0.0, 0.0, 0.0);
-    int4 xi = make_int4(-1, 0, 0, -1);
-    uint32_t word0 = 0u;  // first word of this atom's exclusion row (groups of up to 32 atoms)
-    if (active) {
-        pi = P.cpos[si];
-        xi = P.cex[si];
-        sIp[lane] = P.cprm[si];
-        word0 = P.exbits[xi.z];
-    }
-    pi.x -= sx; pi.y -= sy; pi.z -= sz;  // (x_i - s) - x_j = x_i - (x_j + s)
-    sI[lane] = pi;
-    sF[0][lane] = 0ull; sF[1][lane] = 0ull; sF[2][lane] = 0ull;
-    const int j0 = P.cellStart[cn], j1 = P.cellStart[cn + 1];
-    // in the cell itself only j slots above the chunk's first slot can pair with it;
-    // this wave takes part `part` of kPmeJSplit contiguous parts of the j range
-    const int jall = nb == 0 ? s0 + chunk * 64 + 1 : j0;
-    const int jlen = max(0, j1 - jall);
-    const int jstart = jall + (jlen * part) / kPmeJSplit, jend = jall + (jlen * (part + 1)) / kPmeJSplit;
     const double rc2 = D.rc2;
     double e = 0.0;
-    int head = 0, tail = 0;  // ring [head, tail) of pending pairs (wave-uniform)
-    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    int head = 0, tail = 0;  // the wave's ring [head, tail) of pending pairs (wave-uniform)
+    uint32_t* Q = sQ[wave];
 
-    // evaluate `count` queued pairs, one per lane (j data from the staged batch)
-    auto dense = [&](int count) {
+    // evaluate `count` queued pairs, one per lane
+    auto dense = [&](int count) __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (lane < count) {
-            const uint32_t code = sQ[(head + lane) & 127];
-            const int il = code >> 16, k = (int)(code & 0xFFFFu);
-            const double4 p = sI[il];
-            const double2 ip = sIp[il];
+            const uint32_t code = Q[(head + lane) & 127];
+            const int i = code >> 16, k = (int)(code & 0xFFFFu);
+            const double4 p = sI[i];
+            const double2 ip = sIp[i];
             const double4 pj = sJ[k];
             const double2 jp = sJp[k];
             const double dx = p.x - pj.x, dy = p.y - pj.y, dz = p.z - pj.z;
             const double r2 = dx * dx + dy * dy + dz * dz;
             double fs;
             e += direct_pair(D, r2, p.w * pj.w, ip.x + jp.x, ip.y * jp.y, fs);
-            const long long fx = __double2ll_rn(fs * dx * kFix), fy = __double2ll_rn(fs * dy * kFix);
-            const long long fz = __double2ll_rn(fs * dz * kFix);
-            atomicAdd(&sF[0][il], (unsigned long long)fx);
-            atomicAdd(&sF[1][il], (unsigned long long)fy);
-            atomicAdd(&sF[2][il], (unsigned long long)fz);
-            atomicAdd(&sJF[0][k], (unsigned long long)(-fx));
-            atomicAdd(&sJF[1][k], (unsigned long long)(-fy));
-            atomicAdd(&sJF[2][k], (unsigned long long)(-fz));
+            const double vx = fs * dx * kFix, vy = fs * dy * kFix, vz = fs * dz * kFix;
+            const double mx = fmax(fabs(vx), fmax(fabs(vy), fabs(vz)));
+            // the pairs of one j-atom sit in consecutive lanes (up to 64 of them: the adds to its
+            // sums would queue on one address): an octet of one j-atom adds up first, exactly (whole
+            // numbers below 2^48, whose sum whole() takes), and issues one add per component
+            const int k0 = __shfl(k, lane & 56, 64);
+            uint64_t oct = __ballot(k == k0 && mx < 281474976710656.0);
+            oct &= oct >> 1; oct &= oct >> 2; oct &= oct >> 4;
+            oct &= 0x0101010101010101ull;
+            oct = (oct << 8) - oct;  // all 8 lanes of such octets
+            double rx = rint(vx), ry = rint(vy), rz = rint(vz);
+            const bool big = !(mx < 2251799813685248.0);
+            const long long fx = big ? __double2ll_rn(vx) : whole(rx);
+            const long long fy = big ? __double2ll_rn(vy) : whole(ry);
+            const long long fz = big ? __double2ll_rn(vz) : whole(rz);
+            lds_add(&sIF[0][i], (unsigned long long)fx);
+            lds_add(&sIF[1][i], (unsigned long long)fy);
+            lds_add(&sIF[2][i], (unsigned long long)fz);
+            rx = oct_sum(rx); ry = oct_sum(ry); rz = oct_sum(rz);
+            const bool full = __builtin_amdgcn_inverse_ballot_w64(oct);
+            const bool idle = full && (lane & 7) != 0;
+            const long long gx = idle ? 0ll : -(full ? whole(rx) : fx);
+            const long long gy = idle ? 0ll : -(full ? whole(ry) : fy);
+            const long long gz = idle ? 0ll : -(full ? whole(rz) : fz);
+            if (gx != 0) lds_add(&sJF[0][k], (unsigned long long)gx);
+            if (gy != 0) lds_add(&sJF[1][k], (unsigned long long)gy);
+            if (gz != 0) lds_add(&sJF[2][k], (unsigned long long)gz);
         }
         head += count;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
 
-    for (int jb = jstart; jb < jend; jb += kPmeJBatch) {
-        const int nbat = min(kPmeJBatch, jend - jb);
-        __syncthreads();  // the previous batch is fully evaluated and flushed
-        for (int k = lane; k < nbat; k += 64) {
+    for (int jb = jstart; jb < jend; jb += JB) {
+        const int nj = min(JB, jend - jb);
+        for (int k = threadIdx.x; k < nj; k += NT) {
             sJ[k] = P.cpos[jb + k];
             sJp[k] = P.cprm[jb + k];
             sJx[k] = P.cex[jb + k];
             sJF[0][k] = 0ull; sJF[1][k] = 0ull; sJF[2][k] = 0ull;
         }
         __syncthreads();
-        for (int k = 0; k < nbat; ++k) {
-            const int sj = jb + k;
-            const double4 pj = sJ[k];
-            const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            bool in = active && r2 < rc2 && (nb != 0 || sj > si);
-            if (__ballot(in) == 0ull) continue;
-            const int4 xj = sJx[k];
-            if (in && xj.x == xi.x) {  // same exclusion group: look the pair up
-                const uint32_t bits = (xj.y >> 5) == 0 ? word0 : P.exbits[xi.z + (xj.y >> 5)];
-                if ((bits >> (xj.y & 31)) & 1u) in = false;
-            }
-            const uint64_t m = __ballot(in);
-            if (in) sQ[(tail + __popcll(m & below)) & 127] = ((uint32_t)lane << 16) | (uint32_t)k;
-            tail += __popcll(m);
-            if (tail - head >= 64) {
-                __syncthreads();
-                dense(64);
-                __syncthreads();
+        const int ka = nj * wave / W, kb = nj * (wave + 1) / W;  // this wave's j-atoms
+        for (int ic = 0; ic < ni; ic += 64) {
+            const int cnt = min(64, ni - ic);
+            const int lg = cnt > 32 ? 6 : (cnt > 16 ? 5 : (cnt > 8 ? 4 : 3)), G = 64 >> lg;
+            const int il = lane & ((1 << lg) - 1), jg = lane >> lg;
+            const bool active = il < cnt;
+            const int i = ic + (active ? il : 0);
+            const double px = sI[i].x, py = sI[i].y, pz = sI[i].z;
+            const int4 xi = sIx[i];
+            const uint64_t act = __ballot(active);
+            const uint32_t codeI = (uint32_t)i << 16;
+            const int jself = jb - (i0 + i);  // the cell itself: j slots above the i slot only
+            for (int k0 = ka; k0 < kb; k0 += G) {
+                const int k = min(k0 + jg, kb - 1);
+                const double dx = px - sJ[k].x, dy = py - sJ[k].y, dz = pz - sJ[k].z;
+                const double r2 = dx * dx + dy * dy + dz * dz;
+                uint64_t m = __ballot(r2 < rc2) & act;
+                if (G > 1) m &= __ballot(k0 + jg < kb);
+                if (nb == 0) m &= __ballot(jself + k > 0);
+                if (m == 0ull) continue;
+                const uint64_t same = __ballot(sJx[k].x == xi.x) & m;
+                if (same != 0ull) {  // atoms of one exclusion group: look the pairs up
+                    bool ex = false;
+                    if (__builtin_amdgcn_inverse_ballot_w64(same)) {
+                        const int rank = sJx[k].y;
+                        uint32_t bits = sIw[min(rank >> 5, kPmeExWords - 1)][i];
+                        if (rank >= 32 * kPmeExWords) bits = P.exbits[xi.z + (rank >> 5)];
+                        ex = (bits >> (rank & 31)) & 1u;
+                    }
+                    m &= ~__ballot(ex);
+                }
+                const int at = tail + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                if (__builtin_amdgcn_inverse_ballot_w64(m)) Q[at & 127] = codeI | (uint32_t)k;
+                tail += __popcll(m);
+                if (tail - head >= 64) dense(64);
             }
         }
-        if (tail > head) {  // drain: the next batch replaces the staged j data
-            __syncthreads();
-            dense(tail - head);
-        }
+        if (tail > head) dense(tail - head);  // the staged j-atoms are replaced or flushed next
         __syncthreads();
-        for (int k = lane; k < nbat; k += 64) {  // j forces of the batch
+        for (int k = threadIdx.x; k < nj; k += NT) {  // j forces of the batch
             const int atom = sJx[k].w;
+#pragma unroll
             for (int q = 0; q < 3; ++q) {
                 const unsigned long long v = sJF[q][k];
                 if (v) atomicAdd(F + (long long)q * D.n + atom, v);
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
-    if (active) {
-        const int atom = xi.w;
-        for (int k = 0; k < 3; ++k) {
-            const unsigned long long v = sF[k][lane];
-            if (v) atomicAdd(F + (long long)k * D.n + atom, v);
+    for (int k = threadIdx.x; k < ni; k += NT) {
+        const int atom = sIx[k].w;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const unsigned long long v = sIF[q][k];
+            if (v) atomicAdd(F + (long long)q * D.n + atom, v);
         }
     }
     e = wave_sum(e);
-    if (lane == 0) eslot[blockSlot] = e;
+    if (lane == 0) sE[wave] = e;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < W; ++w) e += sE[w];
+        eslot[blockSlot] = e;
+    }
 }
 
 // Direct space of x + d as the difference from x (the displaced atoms are few): one
@@ -1069,17 +1149,17 @@ hipError_t launch_pme_states(const PmeDesc& D, const PmePtrs& P, bool single, hi
             if (lb) k_pme_spread_difference<<<lb, 256, 0, st>>>(D, P);
         }
     };
-    // neighbour offset fastest, chunk slowest: consecutive workgroups (dealt round-robin to the
-    // XCDs) carry comparable work, and the mostly empty late chunks come last
-    const dim3 gridDirect(kPmeHalfShell * kPmeJSplit, D.ncell, D.chunks);
+    // cell fastest, neighbour slowest and the fullest first (the cell itself holds three times
+    // the pairs of an edge neighbour): the launch ends on the short blocks
+    const dim3 gridDirect(D.ncell, D.chunks, kPmeHalfShell);
     cells(0, true);
-    k_pme_direct<<<gridDirect, 64, 0, st>>>(D, P, delta ? P.F + 6ll * D.n : P.F, P.eslot);
+    k_pme_direct<<<gridDirect, 64 * kPmeDirectWaves, 0, st>>>(D, P, delta ? P.F + 6ll * D.n : P.F, P.eslot);
     spread(0);
     if (delta) {
         if (D.nlig > 0) k_pme_displaced<<<dim3(54, D.nlig), 64, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot);
     } else if (!single) {
         cells(1, false);
-        k_pme_direct<<<gridDirect, 64, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot);
+        k_pme_direct<<<gridDirect, 64 * kPmeDirectWaves, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot);
         spread(1);
     }
     const unsigned gatherBlocks = blocks_of(8ll * D.n, 256);

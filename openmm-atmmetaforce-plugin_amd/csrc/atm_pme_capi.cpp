@@ -179,7 +179,7 @@ void setup(PmeForce& S) {
         }
     }
     if (words > (1ll << 31) - 1) fail(ATM_ERR_INVALID_ARGUMENT, "exclusion bitmaps too large");
-    std::vector<uint32_t> bits((size_t)words, 0u);
+    std::vector<uint32_t> bits((size_t)words + kPmeExWords, 0u);  // (padding: rows are read kPmeExWords at a time)
     std::vector<int2> expairs(std::max(nex, 1));
     std::vector<double4> exprm(std::max(nex, 1));
     for (int k = 0; k < nex; ++k) {
@@ -296,8 +296,8 @@ void set_box(PmeForce& S, const double box[3]) {
     int cap = S.cellCap > 0 ? S.cellCap : (int)std::ceil(1.5 * mean + 64.0);  // grown on overflow
     cap = std::min(kPmeCellMax, (cap + 63) / 64 * 64);
     S.D.cellCap = cap;
-    S.D.chunks = cap / 64;
-    S.D.nslotUsed[0] = S.D.nslotUsed[1] = S.D.chunks * kPmeHalfShell * kPmeJSplit * S.D.ncell;
+    S.D.chunks = (cap + kPmeIBlock - 1) / kPmeIBlock;
+    S.D.nslotUsed[0] = S.D.nslotUsed[1] = S.D.chunks * kPmeHalfShell * S.D.ncell;
     if (S.D.delta) S.D.nslotUsed[1] = 54 * S.D.nlig;
     S.D.nslotDirect = std::max(S.D.nslotUsed[0], S.D.nslotUsed[1]);
     S.D.nslotEx = std::max(1, (S.D.nex + 255) / 256);

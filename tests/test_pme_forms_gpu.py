@@ -47,3 +47,33 @@ def test_forms(gpu, form, grid):
     # clashes at x + d leave forces of up to 1e9 in one state: relative where it is larger
     assert np.all(np.abs(F - Fref) < F_ABS + 1e-12 * np.abs(Fref).max())
     assert np.abs(F1 - po.nonbonded_pme(x, q, sig, eps, L, 1.0, pairs, qq, es, ee, grid=grid)[1]).max() < F_ABS
+
+
+@pytest.mark.parametrize("n,chain", [(30, 0), (300, 140), (1700, 300), (3600, 0), (6000, 40)])
+def test_direct_cells(gpu, n, chain):
+    """Cells of 1 to 222 atoms (short and full chunks of 64, more than one staged batch of the
+    neighbour cell) and exclusion groups longer than the staged rows of 128 atoms."""
+    rng = np.random.default_rng(n)
+    L = np.array([3.05, 3.1, 3.2])
+    g = int(np.ceil(n ** (1 / 3)))
+    lat = np.array([(i, j, k) for i in range(g) for j in range(g) for k in range(g)][:n], dtype=float)
+    x = (lat + 0.5) * (L / g) + rng.uniform(-0.03, 0.03, (n, 3))
+    q = rng.normal(0, 0.5, n)
+    q -= q.mean()
+    sig, eps = rng.uniform(0.15, 0.2, n), rng.uniform(0.1, 0.6, n)
+    pairs = np.array([(i, i + 1) for i in range(5, 5 + chain)] + [(5, 5 + chain)] * (chain > 1)).reshape(-1, 2)
+    zero = np.zeros(len(pairs))
+    d = np.zeros((n, 3))
+    # between lattice sites: the closest pairs at x + d stay below 1e7 kJ/mol/nm.  A shift off the lattice
+    # (0.8, 0.9, 1.0) leaves a pair at 0.032 nm and 1.2e12 among 3600 atoms, past the 2^63 / 2^24 =
+    # 5.5e11 that the forces' fixed-point sums hold.
+    d[:max(1, n // 40)] = (L / g) * (2.5 if g > 4 else 0.5)
+    print(f"[pme] {n} atoms, chain of {chain}", flush=True)
+    with pme.ATMPMEForce(q, sig, eps, d, L, 1.0, exceptions=(pairs, zero, zero + 0.1, zero), params=PARAMS) as f:
+        r, F, _ = f.evaluate(x)
+    ref, Fref, p1, _ = _oracle_atm(x, q, sig, eps, L, pairs, zero, zero + 0.1, zero, d, PARAMS)
+    # the sums' magnitudes (the self energy stands for the reciprocal sum, whose charges are rounded to 2^-36 e)
+    scale = sum(abs(p1[k]) for k in ("direct_coulomb", "direct_lj", "exclusion_correction", "self"))
+    assert abs(r["state1_energy"] - ref["U1"]) <= E_REL * max(1.0, scale)
+    assert abs(r["energy"] - ref["W"]) <= E_REL * max(1.0, scale)
+    assert np.abs(F - Fref).max() < F_ABS + 1e-12 * np.abs(Fref).max()
