@@ -59,7 +59,11 @@ class ATMEnergyFunction(torch.autograd.Function):
         else:
             atoms = (_np(charges), _np(sigmas), _np(epsilons))
         grads = any(t.requires_grad for t in (charges, sigmas, epsilons))
-        state = (on_gpu, atoms, [_np(t) for t in scal], grads)
+        if all(t.is_cuda and t.device == scal[0].device for t in scal):
+            rows = list(torch.stack([_dev64(t) for t in scal]).cpu().numpy())  # one copy for all five
+        else:
+            rows = [_np(t) for t in scal]
+        state = (on_gpu, atoms, rows, grads)
         _upload(batch, state)
         W = np.array([batch.result(k)["energy"] for k in range(S)])
         ctx.batch = batch

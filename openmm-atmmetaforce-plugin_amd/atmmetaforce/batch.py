@@ -231,7 +231,7 @@ class ATMBatch:
         return [self.result(k) for k in range(len(self.systems))]
 
     def forces(self, k) -> np.ndarray:
-        out = np.zeros((self.num_atoms[k], 3))
+        out = np.empty((self.num_atoms[k], 3))
         C.check(self._lib.atm_get_forces(self._h, k, _dptr(out)))
         return out
 

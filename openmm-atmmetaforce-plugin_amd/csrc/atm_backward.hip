@@ -57,11 +57,30 @@ __global__ void k_set_positions(float4* posq, const float* xyz, long long n) {
     posq[i] = p;
 }
 
+// The same from page-locked host memory: each block's 768 floats are read as whole 16-byte
+// words (the memory is not cached on the device: three reads of every third float would cross
+// the link three times) and handed out through LDS.  xyz: 16-byte aligned, padded to a
+// multiple of 4 floats.
+__global__ void __launch_bounds__(256) k_upload_positions(float4* posq, const float4* xyz, int n) {
+    __shared__ float4 row4[192];
+    const int base = blockIdx.x * 256, words = (3 * n + 3) / 4;
+    const int w = blockIdx.x * 192 + threadIdx.x;
+    if (threadIdx.x < 192 && w < words) row4[threadIdx.x] = xyz[w];
+    __syncthreads();
+    const int i = base + threadIdx.x;
+    if (i >= n) return;
+    const float* row = reinterpret_cast<const float*>(row4) + 3 * threadIdx.x;
+    float4 p = posq[i];
+    p.x = row[0]; p.y = row[1]; p.z = row[2];
+    posq[i] = p;
+}
+
 // Per-atom parameters of every atom of a context from device doubles, converted
 // as atm_set_particles converts host ones: posq.w = q sqrt(k_e), ljp = (sigma/2,
 // 2 sqrt(eps)) in FP32, prm64 = (sigma/2, 2 sqrt(eps), q sqrt(k_e), w) in FP64 (w, 1 for a
 // displaced atom, is kept).
-// k_check_particles counts the entries atm_set_particles would reject.
+// k_check_particles counts the entries atm_set_particles would reject; k_set_particles then
+// changes nothing if there are any, and leaves the count for the host.
 __global__ void k_check_particles(const double* q, const double* sig, const double* eps, long long n, int* bad) {
     const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -70,9 +89,12 @@ __global__ void k_check_particles(const double* q, const double* sig, const doub
 }
 
 __global__ void k_set_particles(float4* posq, float2* ljp, double4* prm64, const double* q, const double* sig,
-                                const double* eps, long long n, double sqk) {
+                                const double* eps, long long n, double sqk, const int* bad, int* hostBad) {
     const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (i >= n) return;
+    const int nbad = *bad;
+    if (i == 0) *hostBad = nbad;
+    if (nbad) return;
     const double qi = q[i], si = sig[i], ei = eps[i];
     posq[i].w = (float)(qi * sqk);
     ljp[i] = make_float2((float)(0.5 * si), (float)(2.0 * sqrt(ei)));
@@ -100,10 +122,10 @@ hipError_t launch_check_particles(const double* q, const double* sig, const doub
 }
 
 hipError_t launch_set_particles(const DevPtrs& P, const double* q, const double* sig, const double* eps, long long n,
-                                double sqk, hipStream_t st) {
+                                double sqk, const int* bad, int* hostBad, hipStream_t st) {
     if (n <= 0) return hipSuccess;
     k_set_particles<<<cdivb(n, 256), 256, 0, st>>>(const_cast<float4*>(P.posq), const_cast<float2*>(P.ljp),
-                                                   const_cast<double4*>(P.prm64), q, sig, eps, n, sqk);
+                                                   const_cast<double4*>(P.prm64), q, sig, eps, n, sqk, bad, hostBad);
     return hipGetLastError();
 }
 
@@ -126,6 +148,12 @@ hipError_t launch_backward_gather(const DevPtrs& P, int sysBegin, int nsys, int 
 hipError_t launch_set_positions(DevPtrs P, float4* posq, const float* xyz, long long n, hipStream_t st) {
     if (n <= 0) return hipSuccess;
     k_set_positions<<<cdivb(n, 256), 256, 0, st>>>(posq, xyz, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_upload_positions(float4* posq, const float* xyz, int n, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    k_upload_positions<<<cdivb(n, 256), 256, 0, st>>>(posq, reinterpret_cast<const float4*>(xyz), n);
     return hipGetLastError();
 }
 

@@ -62,4 +62,59 @@ struct DevBuf {
     template <typename T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Page-locked host memory that kernels read and write in place (coherent: a kernel's
+// stores are seen by the host once its stream has been waited for).  A copy to or from
+// ordinary host memory is staged by the runtime and waited for, 20 to 85 us each; a
+// kernel's own stores to this memory cost only their bytes over the link.
+struct HostBuf {
+    void* p = nullptr;
+    size_t bytes = 0;
+    void alloc(size_t n) {
+        release();
+        n = std::max<size_t>(n, 256);
+        HIPCHK(hipHostMalloc(&p, n, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
+        bytes = n;
+    }
+    void release() {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
+    HostBuf() = default;
+    HostBuf(const HostBuf&) = delete;
+    HostBuf& operator=(const HostBuf&) = delete;
+    ~HostBuf() { release(); }
+    template <typename T> T* as() const { return static_cast<T*>(p); }
+};
+
+// Host data on its way to a kernel that reads it in place, without a wait after the
+// launch: begin() waits for the kernel that still reads the previous contents (and
+// refuses a stream under capture, whose replays would read whatever is here by then),
+// end() marks the launch of the reader.
+struct Upload {
+    HostBuf buf;
+    hipEvent_t done = nullptr;
+    bool used = false;
+    void* begin(size_t bytes, hipStream_t st) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(st, &cap));
+        if (cap != hipStreamCaptureStatusNone) fail(ATM_ERR_DEVICE, "host data cannot be set on a stream under capture");
+        if (used) HIPCHK(hipEventSynchronize(done));
+        used = false;
+        if (!done) HIPCHK(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+        if (buf.bytes < bytes) buf.alloc(bytes);
+        return buf.p;
+    }
+    void end(hipStream_t st) {
+        used = true;
+        HIPCHK(hipEventRecord(done, st));
+    }
+    Upload() = default;
+    Upload(const Upload&) = delete;
+    Upload& operator=(const Upload&) = delete;
+    ~Upload() {
+        if (done) (void)hipEventDestroy(done);
+    }
+};
+
 }  // namespace atm

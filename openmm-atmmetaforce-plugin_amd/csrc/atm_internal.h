@@ -96,6 +96,12 @@ struct SysResult {
     double W, usc, U1, U2, u, fp, bfp, sp;
 };
 
+// What a batched evaluation leaves for the host, one per system (page-locked memory).
+struct HostRecord {
+    SysResult res;
+    int overflow[2], maxEntries[2], maxAtoms[2];  // of the two sets' SetRuntime
+};
+
 struct AtmParamsDev {
     double lambda1, lambda2, alpha, u0, w0, umax, ubcore, acore, direction;
 };

@@ -18,6 +18,7 @@ struct DevPtrs {
     const double4* prm64;  // (sigma/2, 2 sqrt(eps), q sqrt(k_e), 0) in FP64
     const AtmParamsDev* params;  // [S]
     SysResult* res;        // [S]
+    HostRecord* host;      // [S] results and list lengths for the host (page-locked memory; may be null)
     double* outF;          // accumulated ATM force (kJ/mol/nm), SoA per system at 3*atomOff
     // per set, unsorted order (setAtomOff)
     float4* bpos;
@@ -146,6 +147,9 @@ hipError_t launch_displaced_dump(const DevPtrs& P, int sys, int state, int nLig,
                                  unsigned long long* ctr, hipStream_t st);
 hipError_t launch_fill_i64(long long* p, long long n, hipStream_t st);
 hipError_t launch_fill_zero(void* p, long long n8, hipStream_t st);
+hipError_t launch_copy8(void* dst, const void* src, long long n8, hipStream_t st);
+// The force of one system (SoA, n atoms) into out (AoS, page-locked host memory).
+hipError_t launch_export_forces(const double* F, int n, double* out, hipStream_t st);
 hipError_t launch_pairs_dump(const DevPtrs& P, int c, int maxGroups, int2* out, long long cap,
                              unsigned long long* counters, hipStream_t st);
 

@@ -2586,6 +2586,19 @@ __global__ void __launch_bounds__(256) k_energy(DevPtrs P, int sysBegin, int est
         SysResult r;
         atm_combine(P.params[s], U[0], U[1], r);
         P.res[s] = r;
+        if (P.host) {
+            // the list lengths are final here (this kernel follows every list kernel): the host
+            // reads this record after one wait instead of copying two device arrays
+            HostRecord h;
+            h.res = r;
+            for (int st = 0; st < 2; ++st) {
+                const SetRuntime& rt = P.rt[2 * s + st];
+                h.overflow[st] = rt.overflow;
+                h.maxEntries[st] = rt.maxEntries;
+                h.maxAtoms[st] = rt.maxAtoms;
+            }
+            P.host[s] = h;
+        }
     }
 }
 
@@ -2673,6 +2686,20 @@ __global__ void k_blend(DevPtrs P, int sysBegin, int nsys, int gx, int hostMode,
     F[i] = ox + (w1 * f1x + w2 * f2x);
     F[N + i] = oy + (w1 * f1y + w2 * f2y);
     F[2 * N + i] = oz + (w1 * f1z + w2 * f2z);
+}
+
+// Consecutive lanes write consecutive doubles (whole lines over the link to the host); the
+// gathered reads are the L2's, which the blend has just filled.
+__global__ void k_export_forces(const double* F, int n, double* out) {
+    const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (k >= 3ll * n) return;
+    const long long i = k / 3;
+    out[k] = F[(k - 3 * i) * n + i];
+}
+
+__global__ void k_copy8(unsigned long long* dst, const unsigned long long* src, long long n) {
+    const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (k < n) dst[k] = src[k];
 }
 
 __global__ void k_fill_i64(long long* p, long long n) {
@@ -2810,6 +2837,19 @@ hipError_t launch_pairs(const DevPtrs& P, int setBegin, int nsets, int maxGroups
 
 hipError_t launch_energy(const DevPtrs& P, int sysBegin, int nsys, int estride, hipStream_t st, bool delta) {
     k_energy<<<nsys, 256, 0, st>>>(P, sysBegin, estride, delta ? 1 : 0);
+    return hipGetLastError();
+}
+
+hipError_t launch_export_forces(const double* F, int n, double* out, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    k_export_forces<<<cdiv(3ll * n, 256), 256, 0, st>>>(F, n, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy8(void* dst, const void* src, long long n8, hipStream_t st) {
+    if (n8 <= 0) return hipSuccess;
+    k_copy8<<<cdiv(n8, 256), 256, 0, st>>>(static_cast<unsigned long long*>(dst),
+                                          static_cast<const unsigned long long*>(src), n8);
     return hipGetLastError();
 }
 

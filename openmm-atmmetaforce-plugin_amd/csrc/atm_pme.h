@@ -77,9 +77,23 @@ struct PmePtrs {
     double* eslot;          // [2][nslot]
     double* parts;          // [2][5]
     SysResult* result;
-    const AtmParamsDev* params;  // the nine ATM parameters (uploaded before each evaluation)
-    const double* eoff;          // [2] energies of other variable-group forces added to U1, U2 (uploaded with params)
+    const AtmParamsDev* params;  // the nine ATM parameters (in the input block)
+    const double* eoff;          // [2] energies of other variable-group forces added to U1, U2 (in the input block)
     int* overflow;
+    // page-locked host memory the kernels read and write in place: the parameters, offsets and
+    // positions of this evaluation, copied by the first kernel to `in`, and its results
+    const double* hostIn;   // [kPmeInHead + 3n]
+    double* in;             // [kPmeInHead + 3n] (params, eoff and x point into it)
+    struct PmeHostRecord* record;
+};
+
+// The head of the input block: the nine ATM parameters and the two offsets, padded.
+constexpr int kPmeInHead = 16;
+
+struct PmeHostRecord {
+    SysResult result;
+    double parts[10];
+    int overflow;
 };
 
 struct BondedPtrs {
@@ -97,6 +111,7 @@ struct BondedPtrs {
 hipError_t launch_pme_fill(unsigned long long* p, long long n, hipStream_t st);
 // Every kernel of one evaluation (single: state 0 only) up to the energy sums.
 hipError_t launch_pme_states(const PmeDesc& D, const PmePtrs& P, bool single, hipStream_t st);
+// forcesOut: page-locked host memory, or null
 hipError_t launch_pme_finish(const PmeDesc& D, const PmePtrs& P, bool single, double* forcesOut, hipStream_t st);
 hipError_t launch_bonded(const BondedPtrs& B, double* eslot, int nblocks, hipStream_t st);
 

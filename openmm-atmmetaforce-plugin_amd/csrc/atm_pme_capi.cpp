@@ -82,12 +82,13 @@ struct PmeForce {
     int cellCap = 0;
     int ncellAlloc = 0, nslotAlloc = 0;
 
-    DevBuf dX, dX2, dDispl, dCellOf, dRankOf, dCellCount, dCellStart, dCellAtoms, dWpos, dPrm, dPrm2, dExkey;
+    DevBuf dIn, dX2, dDispl, dCellOf, dRankOf, dCellCount, dCellStart, dCellAtoms, dWpos, dPrm, dPrm2, dExkey;
     DevBuf dCpos, dCprm, dCex, dExbits, dExpairs, dExprm, dQgrid, dG0, dG1, dTw, dBmod, dF, dEslot, dParts;
-    DevBuf dResult, dOverflow, dOut, dParams, dLig;
+    DevBuf dResult, dOverflow, dLig;
     PmeDesc D{};
     PmePtrs P{};
-    std::vector<double> hOut;
+    // page-locked memory the evaluation's kernels use in place: inputs, results, force (atom by atom)
+    HostBuf hIn, hRecord, hOut;
     // captured evaluation per (state 1 only, forces) and the descriptors it was captured with
     hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     PmeDesc graphD[2][2];
@@ -225,7 +226,10 @@ void setup(PmeForce& S) {
     upload(st, S.dLig, lig.data(), sizeof(int) * lig.size());
     HIPCHK(hipStreamSynchronize(st));
     const long long ng = (long long)S.K[0] * S.K[1] * S.K[2];
-    S.dX.alloc(sizeof(double) * 3 * n);
+    S.dIn.alloc(sizeof(double) * (kPmeInHead + 3 * (size_t)n));
+    S.hIn.alloc(sizeof(double) * (kPmeInHead + 3 * (size_t)n));
+    S.hRecord.alloc(sizeof(PmeHostRecord));
+    S.hOut.alloc(sizeof(double) * 3 * (size_t)n);
     S.dX2.alloc(sizeof(double) * 3 * n);
     S.dCellOf.alloc(sizeof(int) * n);
     S.dRankOf.alloc(sizeof(int) * n);
@@ -240,10 +244,7 @@ void setup(PmeForce& S) {
     S.dF.alloc(sizeof(unsigned long long) * 9 * n);
     S.dParts.alloc(sizeof(double) * 10);
     S.dResult.alloc(sizeof(SysResult));
-    S.dParams.alloc(sizeof(AtmParamsDev) + 2 * sizeof(double));  // parameters, then the two energy offsets
     S.dOverflow.alloc(sizeof(int) * 2);
-    S.dOut.alloc(sizeof(double) * 3 * n);
-    S.hOut.assign(3 * (size_t)n, 0.0);
     S.D.n = n;
     S.D.nex = nex;
     S.D.ngrid = (int)ng;
@@ -319,7 +320,10 @@ void set_box(PmeForce& S, const double box[3]) {
         S.nslotAlloc = S.D.nslot;
     }
     PmePtrs& P = S.P;
-    P.x = S.dX.as<double>();
+    P.hostIn = S.hIn.as<double>();
+    P.in = S.dIn.as<double>();
+    P.record = S.hRecord.as<PmeHostRecord>();
+    P.x = P.in + kPmeInHead;
     P.x2 = S.dX2.as<double>();
     P.displ = S.dDispl.as<double>();
     P.lig = S.dLig.as<int>();
@@ -347,8 +351,9 @@ void set_box(PmeForce& S, const double box[3]) {
     P.eslot = S.dEslot.as<double>();
     P.parts = S.dParts.as<double>();
     P.result = S.dResult.as<SysResult>();
-    P.params = S.dParams.as<AtmParamsDev>();
-    P.eoff = reinterpret_cast<const double*>(S.dParams.as<char>() + sizeof(AtmParamsDev));
+    static_assert(sizeof(AtmParamsDev) == 9 * sizeof(double), "the nine parameters, then the two offsets");
+    P.params = reinterpret_cast<const AtmParamsDev*>(P.in);
+    P.eoff = P.in + 9;
     P.overflow = S.dOverflow.as<int>();
 }
 
@@ -529,16 +534,14 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
         HIPCHK(hipSetDevice(S.device));
         if (!S.setupDone) setup(S);
         const hipStream_t st = S.stream;
-        HIPCHK(hipMemcpyAsync(S.dX.p, positions, sizeof(double) * 3 * S.n, hipMemcpyHostToDevice, st));
-        struct {
-            AtmParamsDev prm;
-            double eoff[2];
-        } up{{S.params.lambda1, S.params.lambda2, S.params.alpha, S.params.u0, S.params.w0, S.params.umax,
-              S.params.ubcore, S.params.acore, S.params.direction},
-             {S.eoff[0], S.eoff[1]}};
-        static_assert(sizeof(up) == sizeof(AtmParamsDev) + 2 * sizeof(double), "parameters and offsets packed");
+        // the graph's first kernel reads these in place; every evaluation is waited for before it returns
+        const double head[kPmeInHead] = {S.params.lambda1, S.params.lambda2, S.params.alpha, S.params.u0,
+                                         S.params.w0, S.params.umax, S.params.ubcore, S.params.acore,
+                                         S.params.direction, S.eoff[0], S.eoff[1]};
+        std::memcpy(S.hIn.p, head, sizeof(head));
+        std::memcpy(S.hIn.as<double>() + kPmeInHead, positions, sizeof(double) * 3 * S.n);
         const bool single = (flags & ATM_EVAL_STATE1_ONLY) != 0;
-        HIPCHK(hipMemcpyAsync(S.dParams.p, &up, sizeof(up), hipMemcpyHostToDevice, st));
+        PmeHostRecord rec;
         for (int attempt = 0; attempt < 2; ++attempt) {
             set_box(S, box ? box : S.box);
             // one captured graph per (state 1 only, forces); captured again when the
@@ -553,9 +556,8 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
             if (!g) {
                 hipGraph_t graph = nullptr;
                 HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-                hipError_t e = launch_pme_fill(reinterpret_cast<unsigned long long*>(S.dOverflow.p), 1, st);
-                if (e == hipSuccess) e = launch_pme_states(S.D, S.P, single, st);
-                if (e == hipSuccess) e = launch_pme_finish(S.D, S.P, single, forces ? S.dOut.as<double>() : nullptr, st);
+                hipError_t e = launch_pme_states(S.D, S.P, single, st);
+                if (e == hipSuccess) e = launch_pme_finish(S.D, S.P, single, forces ? S.hOut.as<double>() : nullptr, st);
                 const hipError_t ee = hipStreamEndCapture(st, &graph);
                 HIPCHK(e);
                 HIPCHK(ee);
@@ -566,24 +568,19 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
                 gP = S.P;
             }
             HIPCHK(hipGraphLaunch(g, st));
-            int ovf[2] = {0, 0};
-            HIPCHK(hipMemcpyAsync(ovf, S.dOverflow.p, sizeof(int) * 2, hipMemcpyDeviceToHost, st));
             HIPCHK(hipStreamSynchronize(st));
-            if (!ovf[0]) break;
+            rec = *S.hRecord.as<PmeHostRecord>();
+            if (!rec.overflow) break;
             if (S.D.cellCap >= kPmeCellMax)
                 fail(ATM_ERR_CAPACITY, "a cell holds more than " + std::to_string(kPmeCellMax) + " atoms");
             S.cellCap = kPmeCellMax;
         }
-        SysResult r;
-        double hp[10];
-        HIPCHK(hipMemcpyAsync(&r, S.dResult.p, sizeof(SysResult), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(hp, S.dParts.p, sizeof(hp), hipMemcpyDeviceToHost, st));
-        if (forces)
-            HIPCHK(hipMemcpyAsync(S.hOut.data(), S.dOut.p, sizeof(double) * 3 * S.n, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        if (forces)
-            for (size_t k = 0; k < 3 * (size_t)S.n; ++k) forces[k] += S.hOut[k];
-        if (parts) std::memcpy(parts, hp, sizeof(hp));
+        const SysResult& r = rec.result;
+        if (forces) {
+            const double* F = S.hOut.as<double>();
+            for (size_t k = 0; k < 3 * (size_t)S.n; ++k) forces[k] += F[k];
+        }
+        if (parts) std::memcpy(parts, rec.parts, sizeof(rec.parts));
         if (result) {
             result->energy = r.W;
             result->perturbation_energy = r.usc;
