@@ -638,8 +638,7 @@ void enqueue_batched(Context& C, int flags, hipEvent_t* ev = nullptr) {
     if (ev) HIPCHK(hipEventRecord(ev[0], st));
     // with forces, the blend writes the cleared force itself
     const bool clearHere = (flags & ATM_EVAL_CLEAR_FORCES) && !forces;
-    HIPCHK(launch_zero_counts(P, 0, nsets, C.maxCells, P.outF, clearHere ? 3 * C.totalAtoms : 0, st));
-    HIPCHK(launch_build(P, 0, nsets, C.maxAtoms, C.maxCells, C.maxSlots, st));
+    HIPCHK(launch_build(P, 0, nsets, C.maxAtoms, C.maxCells, C.maxSlots, P.outF, clearHere ? 3 * C.totalAtoms : 0, st));
     if (ev) HIPCHK(hipEventRecord(ev[1], st));
     // the displaced-atom kernels need only the x sets' cells and clusters: without stage
     // events they run on the side stream beside the pair list and pair kernel (not with
@@ -736,8 +735,7 @@ void eval_plain(Context& C, int flags) {
             const int c = 2 * s + stt;
             const SetDesc& D = C.sets[c];
             const int split = launch_split(C, c, 1, 1);
-            HIPCHK(launch_zero_counts(P, c, 1, D.nx * D.ny * D.nz, nullptr, 0, st));
-            HIPCHK(launch_build(P, c, 1, D.natoms, D.nx * D.ny * D.nz, D.slotCap, st));
+            HIPCHK(launch_build(P, c, 1, D.natoms, D.nx * D.ny * D.nz, D.slotCap, nullptr, 0, st));
             HIPCHK(launch_pairlist(P, c, 1, D.groupCap, 4, st));
             if (uses_atom_lists(C, flags)) HIPCHK(launch_alist(P, c, 1, D.groupCap, st));
             HIPCHK(launch_pairs(P, c, 1, D.groupCap, C.tuning.pairWaves, true, (flags & ATM_EVAL_FP32_PAIRS) == 0,
@@ -769,8 +767,7 @@ void eval_state1(Context& C, int flags) {
         const SetDesc& D = C.sets[2 * s];
         const int c = 2 * s, split = launch_split(C, c, 1, 1);
         if (flags & ATM_EVAL_CLEAR_FORCES) HIPCHK(launch_fill_zero(P.outF + 3ll * D.atomOff, 3ll * D.natoms, st));
-        HIPCHK(launch_zero_counts(P, c, 1, D.nx * D.ny * D.nz, nullptr, 0, st));
-        HIPCHK(launch_build(P, c, 1, D.natoms, D.nx * D.ny * D.nz, D.slotCap, st));
+        HIPCHK(launch_build(P, c, 1, D.natoms, D.nx * D.ny * D.nz, D.slotCap, nullptr, 0, st));
         HIPCHK(launch_pairlist(P, c, 1, D.groupCap, 4, st));
         if (uses_atom_lists(C, flags)) HIPCHK(launch_alist(P, c, 1, D.groupCap, st));
         HIPCHK(launch_pairs(P, c, 1, D.groupCap, C.tuning.pairWaves, (flags & ATM_EVAL_FORCES) != 0,

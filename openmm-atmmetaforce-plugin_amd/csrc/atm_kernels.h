@@ -79,12 +79,11 @@ struct DevPtrs {
     double* geps;
 };
 
-// Clears the cell counters and pair counters of sets setBegin + k P.setStride, k < nsets
-// (maxCells: the largest cell count among them) and, when nf > 0, the doubles f[0, nf).
-hipError_t launch_zero_counts(const DevPtrs& P, int setBegin, int nsets, int maxCells, double* f, long long nf,
-                              hipStream_t st);
-hipError_t launch_build(const DevPtrs& P, int setBegin, int nsets, int maxAtoms, int maxCells, int maxSlots,
-                        hipStream_t st);
+// Clears the counters of sets setBegin + k P.setStride, k < nsets, bins and sorts their atoms into
+// clusters (maxAtoms, maxCells, maxSlots: the largest among them) and, when nf > 0, clears the
+// doubles f[0, nf).
+hipError_t launch_build(const DevPtrs& P, int setBegin, int nsets, int maxAtoms, int maxCells, int maxSlots, double* f,
+                        long long nf, hipStream_t st);
 hipError_t launch_pairlist(const DevPtrs& P, int setBegin, int nsets, int maxGroups, int listWaves, hipStream_t st);
 // atom-level j lists from the cluster list (needed by pair kernel variant kPairKernelAtomLists)
 constexpr int kPairKernelAtomLists = 5;

@@ -349,6 +349,22 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
 
 // ---------------------------------------------------------------- binning
 
+// The counters of set c that an evaluation starts from.
+__device__ __forceinline__ void reset_set(const DevPtrs& P, int c) {
+    // the overflow flag stays set until the host has seen it (it relays out and clears it)
+    P.rt[c].npairs = 0ull;
+    P.rt[c].maxEntries = 0;
+    P.rt[c].maxAtoms = 0;
+    P.rt[c].lpairs[0] = 0ull;
+    P.rt[c].lpairs[1] = 0ull;
+    if (P.setStride == 2 && (c & 1) == 0) {
+        // state difference: the state-1 set's counters hold the derived state-1 values
+        P.rt[c + 1].npairs = 0ull;
+        P.rt[c + 1].maxEntries = 0;
+        P.rt[c + 1].maxAtoms = 0;
+    }
+}
+
 __global__ void k_zero_counts(DevPtrs P, int setBegin, double* f, long long nf) {
     // blockIdx.y: set setBegin + blockIdx.y * setStride (its cell counters and pair counters)
     const int c = setBegin + (int)blockIdx.y * P.setStride;
@@ -359,27 +375,11 @@ __global__ void k_zero_counts(DevPtrs P, int setBegin, double* f, long long nf) 
     // outF (when the evaluation clears it without a blend): the blocks of the first set
     if (blockIdx.y == 0)
         for (long long k = i; k < nf; k += (long long)gridDim.x * blockDim.x) f[k] = 0.0;
-    // the overflow flag stays set until the host has seen it (it relays out and clears it)
-    if (i == 0) {
-        P.rt[c].npairs = 0ull;
-        P.rt[c].maxEntries = 0;
-        P.rt[c].maxAtoms = 0;
-        P.rt[c].lpairs[0] = 0ull;
-        P.rt[c].lpairs[1] = 0ull;
-        if (P.setStride == 2 && (c & 1) == 0) {
-            // state difference: the state-1 set's counters hold the derived state-1 values
-            P.rt[c + 1].npairs = 0ull;
-            P.rt[c + 1].maxEntries = 0;
-            P.rt[c + 1].maxAtoms = 0;
-        }
-    }
+    if (i == 0) reset_set(P, c);
 }
 
-__global__ void k_bin(DevPtrs P, int setBegin) {
-    const int c = setBegin + (int)blockIdx.y * P.setStride;
-    const SetDesc& D = P.desc[c];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= D.natoms) return;
+// Atom i of set c: its wrapped position to bpos; returns its fine cell.
+__device__ __forceinline__ int bin_atom(const DevPtrs& P, const SetDesc& D, int c, int i) {
     float4 p = P.posq[D.atomOff + i];
     if (D.state) {
         float4 d = P.displ[D.atomOff + i];
@@ -396,12 +396,7 @@ __global__ void k_bin(DevPtrs P, int setBegin) {
     const int cx = (int)fminf(fmaxf(p.x * D.invCe[0], 0.f), (float)(D.nx - 1));
     const int cy = (int)fminf(fmaxf(p.y * D.invCe[1], 0.f), (float)(D.ny - 1));
     const int cz = (int)fminf(fmaxf(p.z * D.invZe, 0.f), (float)(D.nz - 1));
-    int cell = (cx * D.ny + cy) * D.nz + cz;
-    int r = atomicAdd(P.cellCount + D.cellOff + cell, 1);
-    const int k = D.setAtomOff + i;
-    P.bpos[k] = p;
-    P.bcell[k] = cell;
-    P.brank[k] = r;
+    P.bpos[D.setAtomOff + i] = p;
     if (P.setStride == 2 && (c & 1) == 0) {
         // state difference: clear dF of atom i (the state-1 set's sums, by atom) and,
         // after an evaluation that used them, its FP64 side sums and their mask word
@@ -417,6 +412,17 @@ __global__ void k_bin(DevPtrs P, int setBegin) {
         }
         P.sf[k2] = 0; P.sf[P.sfn + k2] = 0; P.sf[2 * P.sfn + k2] = 0;
     }
+    return (cx * D.ny + cy) * D.nz + cz;
+}
+
+__global__ void k_bin(DevPtrs P, int setBegin) {
+    const int c = setBegin + (int)blockIdx.y * P.setStride;
+    const SetDesc& D = P.desc[c];
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= D.natoms) return;
+    const int cell = bin_atom(P, D, c, i);
+    P.bcell[D.setAtomOff + i] = cell;
+    P.brank[D.setAtomOff + i] = atomicAdd(P.cellCount + D.cellOff + cell, 1);
 }
 
 __device__ __forceinline__ int wave_incl_scan(int v) {
@@ -436,10 +442,11 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 //     scan joins the chunks; column starts, dummy slots and the group table
 //     are written.
 // A cell's first slot is colStart[column] + cellStart[cell].
-__global__ void __launch_bounds__(1024) k_scan(DevPtrs P, int setBegin) {
+// LDS: the cell counts are in cells (left as the cell starts) and cols has a word per column
+// (left as the column starts); the counts go to memory here as well.
+template <bool LDS>
+__device__ __forceinline__ void scan_set(const DevPtrs& P, const SetDesc& D, int c, int* cells, int* cols) {
     constexpr int NT = 1024, NW = NT / 64;
-    const int c = setBegin + (int)blockIdx.x * P.setStride;
-    const SetDesc& D = P.desc[c];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int ncols = D.nx * D.ny, nz = D.nz;
     if (nz <= 64) {
@@ -451,31 +458,49 @@ __global__ void __launch_bounds__(1024) k_scan(DevPtrs P, int setBegin) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int col = col0 + u * NW;
-                v[u] = (col < ncols && lane < nz) ? P.cellCount[D.cellOff + (size_t)col * nz + lane] : 0;
+                v[u] = (col < ncols && lane < nz) ? (LDS ? cells[col * nz + lane] : P.cellCount[D.cellOff + (size_t)col * nz + lane]) : 0;
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int col = col0 + u * NW;
                 const int incl = wave_incl_scan(v[u]);  // lane 63: the column count (lanes >= nz add 0)
                 if (col < ncols) {
-                    if (lane < nz) P.cellStart[D.cellOff + (size_t)col * nz + lane] = incl - v[u];
-                    if (lane == 63) P.colCount[D.colOff + col] = incl;
+                    if (lane < nz) {
+                        P.cellStart[D.cellOff + (size_t)col * nz + lane] = incl - v[u];
+                        if (LDS) {
+                            cells[col * nz + lane] = incl - v[u];
+                            P.cellCount[D.cellOff + (size_t)col * nz + lane] = v[u];
+                        }
+                    }
+                    if (lane == 63) {
+                        P.colCount[D.colOff + col] = incl;
+                        if (LDS) cols[col] = incl;
+                    }
                 }
             }
         }
     }
     for (int col = nz <= 64 ? ncols : wave; col < ncols; col += NW) {
-        const int* cnt = P.cellCount + D.cellOff + (size_t)col * nz;
+        int* cnt = P.cellCount + D.cellOff + (size_t)col * nz;
         int* st = P.cellStart + D.cellOff + (size_t)col * nz;
         int run = 0;
         for (int z0 = 0; z0 < nz; z0 += 64) {
             const int z = z0 + lane;
-            const int v = z < nz ? cnt[z] : 0;
+            const int v = z < nz ? (LDS ? cells[col * nz + z] : cnt[z]) : 0;
             const int incl = wave_incl_scan(v);
-            if (z < nz) st[z] = run + incl - v;
+            if (z < nz) {
+                st[z] = run + incl - v;
+                if (LDS) {
+                    cells[col * nz + z] = run + incl - v;
+                    cnt[z] = v;
+                }
+            }
             run += __shfl(incl, 63, 64);
         }
-        if (lane == 0) P.colCount[D.colOff + col] = run;
+        if (lane == 0) {
+            P.colCount[D.colOff + col] = run;
+            if (LDS) cols[col] = run;
+        }
     }
     // the column counts written above by other waves of this block: the barrier
     // orders them (workgroup scope covers global memory of the same block)
@@ -486,7 +511,7 @@ __global__ void __launch_bounds__(1024) k_scan(DevPtrs P, int setBegin) {
     __shared__ int sS[NW], sG[NW];
     int accS = 0, accG = 0;
     for (int col = b; col < e; ++col) {
-        const int n = colCount[col];
+        const int n = LDS ? cols[col] : colCount[col];
         const int padded = (n + 7) & ~7;
         accS += padded;
         accG += ((padded >> 3) + kGroupClusters - 1) / kGroupClusters;
@@ -503,11 +528,12 @@ __global__ void __launch_bounds__(1024) k_scan(DevPtrs P, int setBegin) {
     }
     int offS = baseS + inS - accS, offG = baseG + inG - accG;
     for (int col = b; col < e; ++col) {
-        const int cnt = colCount[col];
+        const int cnt = LDS ? cols[col] : colCount[col];
         const int padded = (cnt + 7) & ~7;
         const int ncl = padded >> 3;
         const int ng = (ncl + kGroupClusters - 1) / kGroupClusters;
         P.colStart[D.colOff + col] = offS;
+        if (LDS) cols[col] = offS;
         for (int s2 = offS + cnt; s2 < offS + padded; ++s2) P.sslot[D.slotOff + s2] = make_int2(-1, -1);
         for (int gg = 0; gg < ng; ++gg)
             P.ginfo[D.groupOff + offG + gg] =
@@ -525,6 +551,11 @@ __global__ void __launch_bounds__(1024) k_scan(DevPtrs P, int setBegin) {
     }
 }
 
+__global__ void __launch_bounds__(1024) k_scan(DevPtrs P, int setBegin) {
+    const int c = setBegin + (int)blockIdx.x * P.setStride;
+    scan_set<false>(P, P.desc[c], c, nullptr, nullptr);
+}
+
 // Counting-sort scatter: each atom's (index, cell) into its provisional slot
 // (cell start + the atomic rank of k_bin, whose order is not deterministic).
 __global__ void k_scatter_idx(DevPtrs P, int setBegin) {
@@ -536,6 +567,48 @@ __global__ void k_scatter_idx(DevPtrs P, int setBegin) {
     const int cell = P.bcell[k];
     const int slot = P.colStart[D.colOff + cell / D.nz] + P.cellStart[D.cellOff + cell] + P.brank[k];
     P.sslot[D.slotOff + slot] = make_int2(i, cell);
+}
+
+// k_zero_counts, k_bin, k_scan and k_scatter_idx of one set in one block: the counts and starts
+// stay in LDS (cell | rank of a thread's atoms in registers) and three launches with the gaps
+// between them go.  One CU per set: bound by the chain of one block's barriers and loads, so
+// only for sets of few atoms.  Stage times with events, four kernels against this one: 4 sets
+// of 2,501 atoms 26.8 / 21.0 us (the whole call 190 / 175), 5 of 7,003 30.2 / 35.2 (266 / 269),
+// 6 of 9,001 31.9 / 41.4.
+constexpr int kBuildPerThread = 4, kBuildAtoms = kBuildPerThread * 1024;
+constexpr int kBuildCells = 8000;  // two words a cell stay below 64 KiB
+__global__ void __launch_bounds__(1024) k_build_set(DevPtrs P, int setBegin, double* f, long long nf) {
+    extern __shared__ int lds[];
+    const int c = setBegin + (int)blockIdx.x * P.setStride;
+    const SetDesc& D = P.desc[c];
+    const int t = threadIdx.x, n = D.natoms, nz = D.nz;
+    const int ncells = D.nx * D.ny * nz;
+    int* cells = lds;
+    int* cols = lds + ncells;
+    for (int k = t; k < ncells; k += 1024) cells[k] = 0;
+    for (long long k = blockIdx.x * 1024ll + t; k < nf; k += gridDim.x * 1024ll) f[k] = 0.0;
+    if (t == 0) reset_set(P, c);
+    __syncthreads();
+    uint32_t at[kBuildPerThread];
+#pragma unroll
+    for (int k = 0; k < kBuildPerThread; ++k) {
+        const int i = t + k * 1024;
+        if (i < n) {
+            const int cell = bin_atom(P, D, c, i);
+            at[k] = (uint32_t)cell | (uint32_t)atomicAdd(cells + cell, 1) << 16;
+        }
+    }
+    __syncthreads();
+    scan_set<true>(P, D, c, cells, cols);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kBuildPerThread; ++k) {
+        const int i = t + k * 1024;
+        if (i < n) {
+            const int cell = (int)(at[k] & 0xFFFFu);
+            P.sslot[D.slotOff + cols[cell / nz] + cells[cell] + (int)(at[k] >> 16)] = make_int2(i, cell);
+        }
+    }
 }
 
 // The atom that belongs at rank r of its fine cell: the cell's atoms ordered
@@ -2710,20 +2783,20 @@ __global__ void k_fill_i64(long long* p, long long n) {
 
 static inline unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
 
-hipError_t launch_zero_counts(const DevPtrs& P, int setBegin, int nsets, int maxCells, double* f, long long nf,
-                              hipStream_t st) {
-    const long long per = std::max<long long>(maxCells, cdiv(nf, std::max(nsets, 1)));
-    unsigned blocks = (unsigned)std::min<long long>(std::max<long long>(cdiv(per, 256), 1), 1024);
-    k_zero_counts<<<dim3(blocks, nsets), 256, 0, st>>>(P, setBegin, f, nf);
-    return hipGetLastError();
-}
-
-hipError_t launch_build(const DevPtrs& P, int setBegin, int nsets, int maxAtoms, int maxCells, int maxSlots,
-                        hipStream_t st) {
-    dim3 ga(cdiv(maxAtoms, 256), nsets);
-    k_bin<<<ga, 256, 0, st>>>(P, setBegin);
-    k_scan<<<nsets, 1024, 0, st>>>(P, setBegin);
-    k_scatter_idx<<<ga, 256, 0, st>>>(P, setBegin);
+hipError_t launch_build(const DevPtrs& P, int setBegin, int nsets, int maxAtoms, int maxCells, int maxSlots, double* f,
+                        long long nf, hipStream_t st) {
+    if (maxAtoms <= kBuildAtoms && maxCells <= kBuildCells) {
+        const size_t lds = sizeof(int) * 2 * (size_t)maxCells;  // a column holds at least one cell
+        k_build_set<<<nsets, 1024, lds, st>>>(P, setBegin, f, nf);
+    } else {
+        const long long per = std::max<long long>(maxCells, cdiv(nf, std::max(nsets, 1)));
+        const unsigned blocks = (unsigned)std::min<long long>(std::max<long long>(cdiv(per, 256), 1), 1024);
+        const dim3 ga(cdiv(maxAtoms, 256), nsets);
+        k_zero_counts<<<dim3(blocks, nsets), 256, 0, st>>>(P, setBegin, f, nf);
+        k_bin<<<ga, 256, 0, st>>>(P, setBegin);
+        k_scan<<<nsets, 1024, 0, st>>>(P, setBegin);
+        k_scatter_idx<<<ga, 256, 0, st>>>(P, setBegin);
+    }
     k_gather_bbox<<<dim3(cdiv(maxSlots, 256), nsets), 256, 0, st>>>(P, setBegin);
     return hipGetLastError();
 }
