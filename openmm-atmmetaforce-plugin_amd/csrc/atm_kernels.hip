@@ -102,32 +102,52 @@ __device__ __forceinline__ void pair_image(const SetDesc& D, float& dx, float& d
     dz = min_image(dz, D.L[2], D.invL[2]);
 }
 
-// Two boxes with centre difference d and summed half-extents h hold points closer
-// than sqrt(r2) under some lattice image n_a a + n_b b + n_c c of a triclinic box
-// (every image whose shifted box can reach is tested, so the pair kernel's image
-// of any pair inside the cutoff is among them).
-__device__ __forceinline__ bool tri_boxes_near(const SetDesc& D, float dx, float dy, float dz, float hx, float hy,
-                                               float hz, float r, float r2) {
-    const int c0 = (int)floorf((dz - hz - r) * D.invL[2]), c1 = (int)ceilf((dz + hz + r) * D.invL[2]);
+// The images n of one lattice direction (edge 1 / invL) under which |d - n L| - h < r can hold:
+// [n0, n1], often empty or one.  1e-4 of the edge of slack covers the rounding here; the
+// caller's test of each image decides.
+__device__ __forceinline__ void image_range(float d, float reach, float invL, int& n0, int& n1) {
+    n0 = (int)ceilf(fmaf(d - reach, invL, -1e-4f));
+    n1 = (int)floorf(fmaf(d + reach, invL, 1e-4f));
+}
+
+// f(dx, dy, dz) for every lattice image n_a a + n_b b + n_c c of a triclinic box under which
+// two boxes with centre difference d and summed half-extents h hold points closer than
+// sqrt(r2): the centre difference under that image.  f returns true to end the walk.
+template <class F>
+__device__ __forceinline__ void tri_each_image(const SetDesc& D, float dx, float dy, float dz, float hx, float hy,
+                                               float hz, float r, float r2, F f) {
+    int c0, c1, b0, b1, a0, a1;
+    image_range(dz, hz + r, D.invL[2], c0, c1);
     for (int nc = c0; nc <= c1; ++nc) {
-        const float az = fmaxf(0.f, fabsf(fmaf(-D.L[2], (float)nc, dz)) - hz);
+        const float dz1 = fmaf(-D.L[2], (float)nc, dz);
+        const float az = fmaxf(0.f, fabsf(dz1) - hz);
         const float remz = r2 - az * az;
         if (remz <= 0.f) continue;
         const float dy1 = fmaf(-D.tilt[2], (float)nc, dy), dx1 = fmaf(-D.tilt[1], (float)nc, dx);
-        const int b0 = (int)floorf((dy1 - hy - r) * D.invL[1]), b1 = (int)ceilf((dy1 + hy + r) * D.invL[1]);
+        image_range(dy1, hy + r, D.invL[1], b0, b1);
         for (int nb = b0; nb <= b1; ++nb) {
-            const float ay = fmaxf(0.f, fabsf(fmaf(-D.L[1], (float)nb, dy1)) - hy);
+            const float dy2 = fmaf(-D.L[1], (float)nb, dy1);
+            const float ay = fmaxf(0.f, fabsf(dy2) - hy);
             const float remy = remz - ay * ay;
             if (remy <= 0.f) continue;
             const float dx2 = fmaf(-D.tilt[0], (float)nb, dx1);
-            const int a0 = (int)floorf((dx2 - hx - r) * D.invL[0]), a1 = (int)ceilf((dx2 + hx + r) * D.invL[0]);
+            image_range(dx2, hx + r, D.invL[0], a0, a1);
             for (int na = a0; na <= a1; ++na) {
-                const float ax = fmaxf(0.f, fabsf(fmaf(-D.L[0], (float)na, dx2)) - hx);
-                if (ax * ax < remy) return true;
+                const float dx3 = fmaf(-D.L[0], (float)na, dx2);
+                const float ax = fmaxf(0.f, fabsf(dx3) - hx);
+                if (ax * ax < remy && f(dx3, dy2, dz1)) return;
             }
         }
     }
-    return false;
+}
+
+// The two boxes are near under some image (every image whose shifted box can reach is tested,
+// so the pair kernel's image of any pair inside the cutoff is among them).
+__device__ __forceinline__ bool tri_boxes_near(const SetDesc& D, float dx, float dy, float dz, float hx, float hy,
+                                               float hz, float r, float r2) {
+    bool near = false;
+    tri_each_image(D, dx, dy, dz, hx, hy, hz, r, r2, [&](float, float, float) { return near = true; });
+    return near;
 }
 
 // A column's x-y rectangle and a group's x-y box (centre difference d, summed
@@ -139,13 +159,14 @@ __device__ __forceinline__ bool tri_rect_near(const SetDesc& D, float dx, float 
     for (int nc = -ncSpan; nc <= ncSpan; ++nc) {
         if (skip0 && nc == 0) continue;
         const float dy1 = fmaf(-D.tilt[2], (float)nc, dy), dx1 = fmaf(-D.tilt[1], (float)nc, dx);
-        const int b0 = (int)floorf((dy1 - hy - r) * D.invL[1]), b1 = (int)ceilf((dy1 + hy + r) * D.invL[1]);
+        int b0, b1, a0, a1;
+        image_range(dy1, hy + r, D.invL[1], b0, b1);
         for (int nb = b0; nb <= b1; ++nb) {
             const float ay = fmaxf(0.f, fabsf(fmaf(-D.L[1], (float)nb, dy1)) - hy);
             const float remy = r2 - ay * ay;
             if (remy <= 0.f) continue;
             const float dx2 = fmaf(-D.tilt[0], (float)nb, dx1);
-            const int a0 = (int)floorf((dx2 - hx - r) * D.invL[0]), a1 = (int)ceilf((dx2 + hx + r) * D.invL[0]);
+            image_range(dx2, hx + r, D.invL[0], a0, a1);
             for (int na = a0; na <= a1; ++na) {
                 const float ax = fmaxf(0.f, fabsf(fmaf(-D.L[0], (float)na, dx2)) - hx);
                 if (ax * ax < remy) return true;
@@ -790,6 +811,7 @@ __global__ void __launch_bounds__(64 * W) k_pairlist(DevPtrs P, int setBegin) {
     // list cutoff of the group's x-y box under every image is dropped before its
     // clusters are tested.  A z-window inside [0, L2) admits only c-images n_c = 0.
     float gcx = 0.f, gcy = 0.f, ghx = 0.f, ghy = 0.f;
+    const float gcz = 0.5f * (zlo + zhi), ghz = 0.5f * (zhi - zlo);
     const int ncSpan = (zwrap || zall) ? 1 : 0;
     if (TRI && D.tri) {
         float xlo = sIc[wave][0].x - sIh[wave][0].x, xhi = sIc[wave][0].x + sIh[wave][0].x;
@@ -908,13 +930,21 @@ __global__ void __launch_bounds__(64 * W) k_pairlist(DevPtrs P, int setBegin) {
                 const float sy = D.shiftOK ? (syc == 1 ? D.L[1] : (syc == 2 ? -D.L[1] : 0.f)) : 0.f;
                 const float4 jc = P.bbc[D.clusterOff + J], jh = P.bbh[D.clusterOff + J];
                 if (TRI && D.tri) {
-                    // triclinic: every lattice image the boxes can reach (one loop copy, not unrolled)
-                    for (int q = 0; q < ncl && g0 + q <= J; ++q) {
-                        const float4 ic = sIc[wave][q], ih = sIh[wave][q];
-                        if (tri_boxes_near(D, jc.x - ic.x, jc.y - ic.y, jc.z - ic.z, ih.x + jh.x, ih.y + jh.y,
-                                           ih.z + jh.z, rcl, D.rcList2))
-                            mask |= 1u << q;
-                    }
+                    // triclinic: the images under which the j-cluster reaches the group's box (1e-3 nm
+                    // wider: the clusters' own tests round otherwise), mostly none or one, and the
+                    // group's clusters under each.  Every image of every cluster instead, from bounds
+                    // one image wider on each side, took 80 us for 6 x 9,001 atoms; this 29.
+                    tri_each_image(D, jc.x - gcx, jc.y - gcy, jc.z - gcz, ghx + jh.x + 1e-3f, ghy + jh.y + 1e-3f,
+                                   ghz + jh.z + 1e-3f, rcl, D.rcList2, [&](float dx, float dy, float dz) {
+                        for (int q = 0; q < ncl && g0 + q <= J; ++q) {
+                            const float4 ic = sIc[wave][q], ih = sIh[wave][q];
+                            const float ax = fmaxf(0.f, fabsf(dx + (gcx - ic.x)) - ih.x - jh.x);
+                            const float ay = fmaxf(0.f, fabsf(dy + (gcy - ic.y)) - ih.y - jh.y);
+                            const float az = fmaxf(0.f, fabsf(dz + (gcz - ic.z)) - ih.z - jh.z);
+                            if (ax * ax + ay * ay + az * az < D.rcList2) mask |= 1u << q;
+                        }
+                        return false;
+                    });
                 } else {
 #pragma unroll
                     for (int q = 0; q < kGroupClusters; ++q) {

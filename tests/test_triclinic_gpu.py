@@ -203,3 +203,36 @@ def test_triclinic_runs_the_tile_kernel_for_every_variant(gpu, variant, split):
         b.set_tuning(1.3, 2, 4, variant, pair_split=split)
         b.compute()
         check_system(b, 0, s, tag=f"tri variant {variant} split {split}")
+
+
+@pytest.mark.parametrize("frac", [(0.5, 0.5, 0.5), (-0.5, 0.5, -0.5), (0.5, -0.5, 0.5), (0.0, 0.5, 0.0), (-0.5, 0.0, 0.25)])
+@pytest.mark.parametrize("n,edges", [(260, (1.875, 2.0, 1.875)), (900, (1.875, 3.5, 2.5)), (1500, (3.75, 1.875, 2.0))])
+def test_images_of_small_boxes(gpu, n, edges, frac):
+    """Edges just above twice the cutoff and the largest tilts: several images of a cluster reach
+    a group.  A pair missed or taken twice changes the energy by far more than the bound."""
+    L = np.array(edges)
+    tilt = np.array([frac[0] * L[0], frac[1] * L[0], frac[2] * L[1]])
+    rng = np.random.default_rng(n)
+    g = np.ceil(L / 0.19).astype(int)
+    lat = np.array([(i, j, k) for i in range(g[0]) for j in range(g[1]) for k in range(g[2])], dtype=float)
+    u = (lat[rng.permutation(len(lat))[:n]] + 0.5) / g
+    H = np.array([[L[0], 0, 0], [tilt[0], L[1], 0], [tilt[1], tilt[2], L[2]]])
+    x = np.round((u @ H + rng.uniform(-0.02, 0.02, (len(u), 3))) * 2.0 ** 20) / 2.0 ** 20
+    x += np.round(rng.integers(-1, 2, (len(u), 3)) @ H * 2.0 ** 20) / 2.0 ** 20  # whole cells away
+    n = len(x)
+    d = np.zeros((n, 3))
+    d[:n // 20] = (np.array([1.5, 0.5, 0.5]) / g) @ H  # between lattice sites
+    d = np.round(d * 2.0 ** 20) / 2.0 ** 20
+    q = rng.normal(0, 0.3, n)
+    p = W.ATMParams(0.2, 0.4, 0.1, 110.0, 0.0, 200.0, 100.0, 0.0625, 1.0)
+    s = W.System(positions=x, charges=q - q.mean(), sigmas=rng.uniform(0.15, 0.2, n), epsilons=rng.uniform(0.1, 0.6, n),
+                 displacements=d, box=L, cutoff=0.9, params=p, tilt=tilt)
+    ref, Fref = oracle.atm_eval(s)
+    with ATMBatch([s]) as b:
+        b.compute()
+        r = b.result(0)
+        assert np.array_equal(b.pairs(0, 0), oracle.pairs(x, L, 0.9, tilt=tilt))
+        # FP64 pair energies in another order: 1e-13 of the sum of their magnitudes
+        assert abs(r["state1_energy"] - ref["U1"]) <= 1e-13 * max(ref["abs1"], 1.0)
+        # FP32 force vectors (2^-24 each) and per-lane sums of up to ~100 of them
+        assert np.linalg.norm(b.forces(0) - Fref) <= 1e-6 * np.linalg.norm(Fref)
