@@ -316,7 +316,8 @@ class ATMBatch:
         per batch, copies of the j-force sums, drain after every test step) = (4, 2, yes), (4, 2, no),
         (4, 4, yes), (8, 2, yes); 5: atom-level j lists per i-cluster, 8 i x 8 j lanes per step;
         6: filtered atom queues.  list_capacity: list entries per group to start from (0: sized from
-        the density).  pair_split: waves sharing one group's list in the tile kernel (1, 2, 4, 8).
+        the density).  pair_split: least number of waves sharing one group's list in the tile
+        kernel (1, 2, 4, 8; a launch of few groups takes more, up to 16).
         full_state2: bin and pair x + d in full instead of as the difference from x at the
         displaced atoms (used when every system displaces at most a quarter of its atoms).
         pair_order: the tile kernel's group order (0 launch order, 1 longest lists first over all

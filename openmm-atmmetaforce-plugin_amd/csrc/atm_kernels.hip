@@ -6,14 +6,15 @@
 //   k_bin          x (+ d for state 1), wrap into the box, fine-cell id and rank
 //   k_scan         per-set column/cell scans, dummy padding, group table
 //   k_scatter_idx  counting-sort scatter of (atom, cell) into provisional slots
+//   k_build_set    the four above in one block, for sets of few atoms
 //   k_gather_bbox  order each fine cell by atom index (deterministic results),
 //                  gather positions/parameters into cluster order, clear the
 //                  set's force accumulators, per-cluster bounding boxes
 //   k_pairlist     per group of 8 clusters: j-clusters (from the group's
 //                  z-window) whose boxes are within the cutoff of at least one
 //                  i-cluster (half shell, i <= j)
-//   k_pairs        LJ + reaction-field pair kernel, one wave64 per group,
-//                  lanes = 8 j-atoms x 8 i-atoms, FP32 geometry, FP64 pair
+//   k_pairs        LJ + reaction-field pair kernel, one block of 2 to 16 waves
+//                  per group, lanes = 8 j-atoms x 8 i-atoms, FP32 geometry, FP64 pair
 //                  function (or FP32), FP64 energy, 64-bit fixed-point forces;
 //                  k_pairs_f: one wave per i-cluster over its atom-filtered j
 //                  atoms

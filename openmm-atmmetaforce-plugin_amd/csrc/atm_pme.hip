@@ -2,7 +2,7 @@
 // particle-mesh Ewald evaluated on x and on x + d, then the ATM combine.
 //
 // Direct space and charge spreading of x:
-//   k_pme_fill3      clear the cell counts, charge grids and force sums
+//   k_pme_begin      inputs from the host's memory; clear the cell counts, charge grids and force sums
 //   k_pme_bin        (form x + d) wrap into the box, cell of edge >= rc, rank in the cell
 //   k_pme_scan       cell starts (one block)
 //   k_pme_scatter    atom indices into cell order
