@@ -33,8 +33,10 @@ struct PmeDesc {
     int twOff[3];                // offset of each axis' twiddle table
     int nex;                     // exception pairs
     int nslot, nslotDirect, nslotEx;  // energy slots per state (direct | exceptions | reciprocal)
-    int nslotUsed[2];            // direct slots in use per state (delta: state 1 holds the displaced atoms' differences)
-    int delta;                   // direct space and charges of x + d as the difference from x (few displaced atoms)
+    int nslotPairs;              // direct slots of the cell pairs (delta: of state 0, for both states); the displaced
+                                 // atoms' own follow in each state
+    int delta;                   // x + d shares the direct space that d leaves alone, and its charges are the difference
+                                 // from x (few displaced atoms)
     int nlig;                    // displaced atoms
     // fused transforms (fused != 0): planes over axes pAx, qAx in LDS, then lines along lineAx with the
     // convolution; every axis length K = fA (K / fA) in two short steps
@@ -64,6 +66,8 @@ struct PmePtrs {
     double4* cpos;          // [n] cell order: wrapped x, y, z, q sqrt(k_e)
     double2* cprm;          // [n] cell order: sigma/2, 2 sqrt(eps)
     int4* cex;              // [n] cell order: group, rank, row offset, atom
+    const int* dcls;        // [n] displacement class: 0 not displaced, the same for atoms displaced alike
+    int* ccls;              // [n] cell order: displacement class
     const uint32_t* exbits; // exclusion bitmaps
     const int2* expairs;    // [nex]
     const double4* exprm;   // [nex] (k_e qq', sigma', 4 eps', k_e q_i q_j)

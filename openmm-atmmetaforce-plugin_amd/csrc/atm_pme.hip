@@ -7,8 +7,8 @@
 //   k_pme_scan       cell starts (one block)
 //   k_pme_scatter    atom indices into cell order
 //   k_pme_cellsort   each cell ordered by atom index (deterministic sums), and
-//                    positions / parameters / exclusion keys gathered into
-//                    cell order
+//                    positions / parameters / exclusion keys / displacement
+//                    classes gathered into cell order
 //   k_pme_direct     erfc(alpha r)/r Coulomb + LJ over minimum-image pairs with
 //                    r < rc that are not exceptions; one block per (cell, the
 //                    cell or one of its 13 forward neighbours): each pair once
@@ -16,7 +16,8 @@
 //                    tile of the grid, 64-bit fixed point (k_pme_spread: the
 //                    same straight into the grid, when a tile does not fit)
 // x + d differs from x at the displaced atoms only.  When they are few (at most one in
-// 16) k_pme_displaced adds what their pairs change, and their charges move on a
+// 16) k_pme_direct takes the pairs whose separation d leaves alone, once for both
+// states, k_pme_displaced the others at x and at x + d, and the charges move on a
 // difference grid; otherwise the same kernels run on x + d.  Then for both states at
 // once (blockIdx.y):
 //   k_pme_planes     two axes of the forward transform per plane of the grid, in LDS
@@ -53,9 +54,9 @@ constexpr double kFix = 16777216.0;          // 2^24 force units per kJ/mol/nm
 constexpr double kGridFix = 68719476736.0;   // 2^36 charge-grid units per e
 constexpr int kOrder = 5;
 
-__device__ __forceinline__ void add_fixed(unsigned long long* p, double f) {
-    atomicAdd(p, (unsigned long long)__double2ll_rn(f * kFix));
-}
+__device__ __forceinline__ unsigned long long fixed_force(double f) { return (unsigned long long)__double2ll_rn(f * kFix); }
+
+__device__ __forceinline__ void add_fixed(unsigned long long* p, double f) { atomicAdd(p, fixed_force(f)); }
 
 // Integer add in LDS (workgroup scope, no result).
 __device__ __forceinline__ void lds_add(unsigned long long* p, unsigned long long v) {
@@ -90,7 +91,8 @@ __device__ __forceinline__ int wrap_index(int v, int K) {
     return v >= K ? v - K : v;
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
+template <class T>
+__device__ __forceinline__ T wave_sum(T v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     return v;
 }
@@ -228,6 +230,7 @@ __global__ void __launch_bounds__(256) k_pme_cellsort(PmeDesc D, PmePtrs P) {
         P.cprm[slot] = make_double2(P.prm2[a].x, P.prm2[a].y);
         const int4 ex = P.exkey[a];
         P.cex[slot] = make_int4(ex.x, ex.y, ex.z, a);
+        P.ccls[slot] = P.dcls[a];
     }
 }
 
@@ -263,7 +266,8 @@ __device__ __forceinline__ double direct_pair(const PmeDesc& D, double r2, doubl
 //         atoms left of a cell of 133 cost an eighth of a full chunk).  FP64 r^2, the
 //         image shift known from the cell offset, exclusion bitmap for atoms of one
 //         exclusion group; in-range pairs are appended to the wave's ring in LDS (ballot +
-//         mbcnt, so the order is fixed);
+//         mbcnt, so the order is fixed);  shared: pairs of atoms displaced differently are left
+//         out (looked up only where a wave's atoms hold a displaced one);
 //  dense: whenever 64 pairs are pending, each lane evaluates one of them
 //         (erfc Coulomb + LJ in FP64); forces go to the block's LDS sums in 64-bit fixed
 //         point (integer atomics: order-independent).
@@ -273,11 +277,13 @@ __device__ __forceinline__ double direct_pair(const PmeDesc& D, double r2, doubl
 // blocks of 8 waves).  59 -> 48 us for 8,479 atoms, 151 -> 120 for 25,437, against one wave
 // per (64 atoms, neighbour, quarter of its atoms) with its own sums.
 __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc D, PmePtrs P, unsigned long long* F,
-                                                                       double* eslot) {
+                                                                       double* eslot, int shared) {
     constexpr int IB = kPmeIBlock, JB = kPmeJBlock, W = kPmeDirectWaves, NT = 64 * W;
+    static_assert(JB + W - 1 <= 64 * W, "a wave's j-atoms are looked over one per lane");
     __shared__ double4 sI[IB], sJ[JB];       // x, y, z, q sqrt(k_e); i-atoms shifted to the neighbour's image
     __shared__ double2 sIp[IB], sJp[JB];
     __shared__ int4 sIx[IB], sJx[JB];        // exclusion group, rank, row offset, atom
+    __shared__ int sIc[IB], sJc[JB];         // displacement classes
     __shared__ uint32_t sIw[kPmeExWords][IB]; // first words of the i-atoms' exclusion rows
     __shared__ unsigned long long sIF[3][IB], sJF[3][JB];
     __shared__ uint32_t sQ[W][128];
@@ -315,6 +321,7 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
         sIp[k] = P.cprm[i0 + k];
         const int4 xk = P.cex[i0 + k];
         sIx[k] = xk;
+        sIc[k] = P.ccls[i0 + k];
 #pragma unroll
         for (int w = 0; w < kPmeExWords; ++w) sIw[w][k] = P.exbits[xk.z + w];  // (padded past the last row)
         sIF[0][k] = 0ull; sIF[1][k] = 0ull; sIF[2][k] = 0ull;
@@ -380,6 +387,7 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
             sJ[k] = P.cpos[jb + k];
             sJp[k] = P.cprm[jb + k];
             sJx[k] = P.cex[jb + k];
+            sJc[k] = P.ccls[jb + k];
             sJF[0][k] = 0ull; sJF[1][k] = 0ull; sJF[2][k] = 0ull;
         }
         __syncthreads();
@@ -395,6 +403,8 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
             const uint64_t act = __ballot(active);
             const uint32_t codeI = (uint32_t)i << 16;
             const int jself = jb - (i0 + i);  // the cell itself: j slots above the i slot only
+            const int clsI = sIc[i];
+            const bool mixed = shared && __ballot((active && clsI != 0) || (ka + lane < kb && sJc[ka + lane] != 0)) != 0ull;
             for (int k0 = ka; k0 < kb; k0 += G) {
                 const int k = min(k0 + jg, kb - 1);
                 const double dx = px - sJ[k].x, dy = py - sJ[k].y, dz = pz - sJ[k].z;
@@ -402,6 +412,7 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
                 uint64_t m = __ballot(r2 < rc2) & act;
                 if (G > 1) m &= __ballot(k0 + jg < kb);
                 if (nb == 0) m &= __ballot(jself + k > 0);
+                if (mixed) m &= __ballot(sJc[k] == clsI);
                 if (m == 0ull) continue;
                 const uint64_t same = __ballot(sJx[k].x == xi.x) & m;
                 if (same != 0ull) {  // atoms of one exclusion group: look the pairs up
@@ -450,18 +461,21 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
     }
 }
 
-// Direct space of x + d as the difference from x (the displaced atoms are few): one
-// wave per (displaced atom k, neighbour cell, state): the pairs of atom k at that
-// state with the cell's atoms that are not displaced, at x (-) and at x + d (+); the
-// first cell's wave also takes the displaced atoms after k that are displaced
-// differently (atoms displaced alike keep their separation).  Energies into the
-// state-1 direct slots, forces into state 1's sums.  10 us for the 21-atom ligand of an
-// 8,479-atom system, where a second cell list and direct pass took 79; one wave per
-// neighbour cell because a wave walking all 27 waits on memory 50 times in a row.
-__global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P, unsigned long long* F, double* eslot) {
+// The pairs that d changes, at each state by themselves (the displaced atoms are few): one
+// wave per (displaced atom k, neighbour cell, state): the pairs of atom k at that state
+// with the cell's atoms that are not displaced; the first cell's wave also takes the
+// displaced atoms after k that are displaced differently.  Energies and forces go to the
+// state's own sums (per pair in fixed point, as k_pme_direct adds them), so nothing cancels:
+// a pair that clashes at x, up to the last bit it has, leaves x + d alone.  (k_pme_direct with
+// these pairs at x and this kernel taking them off again for x + d left 1e-16 of the clash in
+// U2 and, past the fixed-point range of a force, thousands of kJ/mol/nm.)  10 us for the
+// 21-atom ligand of an 8,479-atom system, where a second cell list and direct pass took 79;
+// one wave per neighbour cell because a wave walking all 27 waits on memory 50 times in a row.
+__global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P) {
     const int lane = threadIdx.x, cellOff = blockIdx.x >> 1, st = blockIdx.x & 1, k = blockIdx.y;
     const int a = P.lig[k];
     const double* X = st ? P.x2 : P.x;
+    unsigned long long* F = P.F + 3ll * D.n * st;
     double w[3];
     const int c0 = wrap_cell(X[3 * a], D.L[0], D.invL[0], D.m[0], &w[0]);
     const int c1 = wrap_cell(X[3 * a + 1], D.L[1], D.invL[1], D.m[1], &w[1]);
@@ -475,18 +489,18 @@ __global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P, unsi
     const int4 xa = P.exkey[a];
     const double2 pa = P.prm2[a];
     const double qa = P.prm[a].x;
-    const double dax = P.displ[3 * a], day = P.displ[3 * a + 1], daz = P.displ[3 * a + 2];
-    const double sgn = st ? 1.0 : -1.0;
-    double e = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+    const int clsA = P.dcls[a];
+    double e = 0.0;
+    unsigned long long fx = 0ull, fy = 0ull, fz = 0ull;
     auto pair = [&](int b, double dx, double dy, double dz, double r2, int grp, int rank, double qb, double2 pb) {
         if (grp == xa.x && ((P.exbits[xa.z + (rank >> 5)] >> (rank & 31)) & 1u)) return;
         double fs;
         e += direct_pair(D, r2, qa * qb, pa.x + pb.x, pa.y * pb.y, fs);
-        const double gx = sgn * fs * dx, gy = sgn * fs * dy, gz = sgn * fs * dz;
+        const unsigned long long gx = fixed_force(fs * dx), gy = fixed_force(fs * dy), gz = fixed_force(fs * dz);
         fx += gx; fy += gy; fz += gz;
-        add_fixed(F + b, -gx);
-        add_fixed(F + D.n + b, -gy);
-        add_fixed(F + 2ll * D.n + b, -gz);
+        atomicAdd(F + b, 0ull - gx);
+        atomicAdd(F + D.n + b, 0ull - gy);
+        atomicAdd(F + 2ll * D.n + b, 0ull - gz);
     };
     const int j0 = P.cellStart[cn], j1 = min(P.cellStart[cn + 1], j0 + kPmeCellMax);
     for (int j = j0 + lane; j < j1; j += 64) {
@@ -494,16 +508,14 @@ __global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P, unsi
         const double dx = px - pj.x, dy = py - pj.y, dz = pz - pj.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
         if (!(r2 < D.rc2)) continue;
+        if (P.ccls[j] != 0) continue;  // displaced itself: below
         const int4 xj = P.cex[j];
-        const double* db = P.displ + 3ll * xj.w;
-        if (db[0] != 0.0 || db[1] != 0.0 || db[2] != 0.0) continue;  // displaced itself: below
         pair(xj.w, dx, dy, dz, r2, xj.x, xj.y, pj.w, P.cprm[j]);
     }
     if (cellOff == 0)
         for (int q = k + 1 + lane; q < D.nlig; q += 64) {
             const int b = P.lig[q];
-            const double* db = P.displ + 3ll * b;
-            if (db[0] == dax && db[1] == day && db[2] == daz) continue;
+            if (P.dcls[b] == clsA) continue;  // displaced alike: in the shared sums
             double v[3];
             wrap_cell(X[3 * b], D.L[0], D.invL[0], D.m[0], &v[0]);
             wrap_cell(X[3 * b + 1], D.L[1], D.invL[1], D.m[1], &v[1]);
@@ -520,10 +532,10 @@ __global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P, unsi
     e = wave_sum(e);
     fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
     if (lane == 0) {
-        eslot[(27 * k + cellOff) * 2 + st] = sgn * e;
-        if (fx != 0.0) add_fixed(F + a, fx);
-        if (fy != 0.0) add_fixed(F + D.n + a, fy);
-        if (fz != 0.0) add_fixed(F + 2ll * D.n + a, fz);
+        P.eslot[(long long)D.nslot * st + D.nslotPairs + 27 * k + cellOff] = e;
+        if (fx != 0ull) atomicAdd(F + a, fx);
+        if (fy != 0ull) atomicAdd(F + D.n + a, fy);
+        if (fz != 0ull) atomicAdd(F + 2ll * D.n + a, fz);
     }
 }
 
@@ -1042,27 +1054,27 @@ __global__ void __launch_bounds__(256) k_pme_gather(PmeDesc D, PmePtrs P, const 
 __global__ void __launch_bounds__(1024) k_pme_finish(PmeDesc D, PmePtrs P, int single) {
     __shared__ double red[16];
     double U[2] = {0.0, 0.0};
-    double direct0 = 0.0;
+    auto sum = [&](const double* sl, int first, int last) {
+        // four independent partial sums per thread (fixed order): their loads overlap
+        double v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
+        int k = first + (int)threadIdx.x;
+        for (; k + 3 * 1024 < last; k += 4 * 1024) {
+            v0 += sl[k];
+            v1 += sl[k + 1024];
+            v2 += sl[k + 2 * 1024];
+            v3 += sl[k + 3 * 1024];
+        }
+        for (; k < last; k += 1024) v0 += sl[k];
+        return block_sum<1024>((v0 + v1) + (v2 + v3), red);
+    };
+    const bool own = D.delta && !single;  // the pairs of both states in state 0's slots, then each state's own
+    const double shared = own ? sum(P.eslot, 0, D.nslotPairs) : 0.0;
     for (int s = 0; s < (single ? 1 : 2); ++s) {
         const double* sl = P.eslot + (long long)s * D.nslot;
-        const int first[3] = {0, D.nslotDirect, D.nslotDirect + D.nslotEx};
-        const int last[3] = {D.nslotUsed[s], D.nslotDirect + D.nslotEx, D.nslot};
         double parts[3];
-        for (int r = 0; r < 3; ++r) {
-            // four independent partial sums per thread (fixed order): their loads overlap
-            double v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
-            int k = first[r] + (int)threadIdx.x;
-            for (; k + 3 * 1024 < last[r]; k += 4 * 1024) {
-                v0 += sl[k];
-                v1 += sl[k + 1024];
-                v2 += sl[k + 2 * 1024];
-                v3 += sl[k + 3 * 1024];
-            }
-            for (; k < last[r]; k += 1024) v0 += sl[k];
-            parts[r] = block_sum<1024>((v0 + v1) + (v2 + v3), red);
-        }
-        if (s == 0) direct0 = parts[0];
-        else if (D.delta) parts[0] += direct0;  // the slots hold the difference
+        parts[0] = own ? shared + sum(sl, D.nslotPairs, D.nslotDirect) : sum(sl, 0, D.nslotPairs);
+        parts[1] = sum(sl, D.nslotDirect, D.nslotDirect + D.nslotEx);
+        parts[2] = sum(sl, D.nslotDirect + D.nslotEx, D.nslot);
         if (threadIdx.x == 0) {
             P.parts[5 * s + 0] = parts[0];
             P.parts[5 * s + 1] = parts[1];
@@ -1165,13 +1177,13 @@ hipError_t launch_pme_states(const PmeDesc& D, const PmePtrs& P, bool single, hi
     // the pairs of an edge neighbour): the launch ends on the short blocks
     const dim3 gridDirect(D.ncell, D.chunks, kPmeHalfShell);
     cells(0, true);
-    k_pme_direct<<<gridDirect, 64 * kPmeDirectWaves, 0, st>>>(D, P, delta ? P.F + 6ll * D.n : P.F, P.eslot);
+    k_pme_direct<<<gridDirect, 64 * kPmeDirectWaves, 0, st>>>(D, P, delta ? P.F + 6ll * D.n : P.F, P.eslot, delta ? 1 : 0);
     spread(0);
     if (delta) {
-        if (D.nlig > 0) k_pme_displaced<<<dim3(54, D.nlig), 64, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot);
+        if (D.nlig > 0) k_pme_displaced<<<dim3(54, D.nlig), 64, 0, st>>>(D, P);
     } else if (!single) {
         cells(1, false);
-        k_pme_direct<<<gridDirect, 64 * kPmeDirectWaves, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot);
+        k_pme_direct<<<gridDirect, 64 * kPmeDirectWaves, 0, st>>>(D, P, P.F + 3ll * D.n, P.eslot + D.nslot, 0);
         spread(1);
     }
     const unsigned gatherBlocks = blocks_of(8ll * D.n, 256);

@@ -9,6 +9,7 @@
 // x + d and combines them (platforms/reference/src/ReferenceATMMetaForceKernels.cpp:56-110).
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <functional>
@@ -84,7 +85,7 @@ struct PmeForce {
 
     DevBuf dIn, dX2, dDispl, dCellOf, dRankOf, dCellCount, dCellStart, dCellAtoms, dWpos, dPrm, dPrm2, dExkey;
     DevBuf dCpos, dCprm, dCex, dExbits, dExpairs, dExprm, dQgrid, dG0, dG1, dTw, dBmod, dF, dEslot, dParts;
-    DevBuf dResult, dOverflow, dLig;
+    DevBuf dResult, dOverflow, dLig, dDcls, dCcls;
     PmeDesc D{};
     PmePtrs P{};
     // page-locked memory the evaluation's kernels use in place: inputs, results, force (atom by atom)
@@ -214,16 +215,23 @@ void setup(PmeForce& S) {
     upload(st, S.dTw, tw.data(), sizeof(double2) * tw.size());
     upload(st, S.dBmod, bmod.data(), sizeof(double) * bmod.size());
     upload(st, S.dDispl, S.displ.data(), sizeof(double) * 3 * n);
-    std::vector<int> lig;
-    for (int i = 0; i < n; ++i)
-        if (S.displ[3 * (size_t)i] != 0.0 || S.displ[3 * (size_t)i + 1] != 0.0 || S.displ[3 * (size_t)i + 2] != 0.0)
-            lig.push_back(i);
+    // displaced atoms and their displacement classes (1, 2, ... by first appearance)
+    std::vector<int> lig, dcls(n, 0);
+    std::map<std::array<double, 3>, int> classOf;
+    for (int i = 0; i < n; ++i) {
+        const std::array<double, 3> d = {S.displ[3 * (size_t)i], S.displ[3 * (size_t)i + 1], S.displ[3 * (size_t)i + 2]};
+        if (d[0] == 0.0 && d[1] == 0.0 && d[2] == 0.0) continue;
+        lig.push_back(i);
+        dcls[i] = classOf.emplace(d, (int)classOf.size() + 1).first->second;
+    }
     S.D.nlig = (int)lig.size();
-    // x + d as the difference from x: each displaced atom costs 54 waves over its neighbour
-    // cells, so only while they are few (a wave per 64 atoms of a cell pair covers the rest)
+    // the displaced atoms' pairs by themselves: each costs 54 waves over its neighbour cells, so
+    // only while they are few.  Whole call in us with 21 atoms, n/64, n/32 and n/16 displaced: 201, 217,
+    // 229, 249 (8,479 atoms; both states in full 260 to 265) and 363, 398, 435, 504 (25,437; 503)
     S.D.delta = 16ll * S.D.nlig <= n && S.D.nlig <= 65535;
     if (lig.empty()) lig.push_back(0);
     upload(st, S.dLig, lig.data(), sizeof(int) * lig.size());
+    upload(st, S.dDcls, dcls.data(), sizeof(int) * n);
     HIPCHK(hipStreamSynchronize(st));
     const long long ng = (long long)S.K[0] * S.K[1] * S.K[2];
     S.dIn.alloc(sizeof(double) * (kPmeInHead + 3 * (size_t)n));
@@ -238,6 +246,7 @@ void setup(PmeForce& S) {
     S.dCpos.alloc(sizeof(double4) * n);
     S.dCprm.alloc(sizeof(double2) * n);
     S.dCex.alloc(sizeof(int4) * n);
+    S.dCcls.alloc(sizeof(int) * n);
     S.dQgrid.alloc(sizeof(long long) * 2 * ng);
     S.dG0.alloc(sizeof(double2) * 2 * ng);
     S.dG1.alloc(sizeof(double2) * 2 * ng);
@@ -298,9 +307,8 @@ void set_box(PmeForce& S, const double box[3]) {
     cap = std::min(kPmeCellMax, (cap + 63) / 64 * 64);
     S.D.cellCap = cap;
     S.D.chunks = (cap + kPmeIBlock - 1) / kPmeIBlock;
-    S.D.nslotUsed[0] = S.D.nslotUsed[1] = S.D.chunks * kPmeHalfShell * S.D.ncell;
-    if (S.D.delta) S.D.nslotUsed[1] = 54 * S.D.nlig;
-    S.D.nslotDirect = std::max(S.D.nslotUsed[0], S.D.nslotUsed[1]);
+    S.D.nslotPairs = S.D.chunks * kPmeHalfShell * S.D.ncell;
+    S.D.nslotDirect = S.D.nslotPairs + (S.D.delta ? 27 * S.D.nlig : 0);
     S.D.nslotEx = std::max(1, (S.D.nex + 255) / 256);
     S.D.nslot = S.D.nslotDirect + S.D.nslotEx + (S.D.fused ? S.D.lineBlocks : (S.D.ngrid + 255) / 256);
     // charge-grid tile of one cell: grid indices [floor(c K/m) - 5, ... + ceil(K/m) + 7)
@@ -339,6 +347,8 @@ void set_box(PmeForce& S, const double box[3]) {
     P.cpos = S.dCpos.as<double4>();
     P.cprm = S.dCprm.as<double2>();
     P.cex = S.dCex.as<int4>();
+    P.dcls = S.dDcls.as<int>();
+    P.ccls = S.dCcls.as<int>();
     P.exbits = S.dExbits.as<uint32_t>();
     P.expairs = S.dExpairs.as<int2>();
     P.exprm = S.dExprm.as<double4>();

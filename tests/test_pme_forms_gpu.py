@@ -77,3 +77,31 @@ def test_direct_cells(gpu, n, chain):
     assert abs(r["state1_energy"] - ref["U1"]) <= E_REL * max(1.0, scale)
     assert abs(r["energy"] - ref["W"]) <= E_REL * max(1.0, scale)
     assert np.abs(F - Fref).max() < F_ABS + 1e-12 * np.abs(Fref).max()
+
+
+# an LJ pair passes the range of the fixed-point forces (5.5e11 kJ/mol/nm) below 0.05 nm
+@pytest.mark.parametrize("dist", [0.05, 0.03, 0.01, 0.0])
+@pytest.mark.parametrize("partner", ["stays", "displaced differently"])
+def test_clash_at_x_leaves_the_other_state_alone(gpu, dist, partner):
+    """A displaced atom on top of another at x, at the end of a leg where x + d is the physical
+    state (direction -1, weight 0 for x): the energy and force of x + d are exact."""
+    x, q, sig, eps, L, pairs, qq, es, ee, d = _small_system(seed=23)
+    d[40:60] = (1.1, 1.2, 1.3)
+    other = 200
+    if partner != "stays":
+        d[other] = (-0.55, 0.8, 0.3)
+    x[50] = x[other] + dist * np.array([0.48, 0.6, 0.64])
+    sig[[50, other]], eps[[50, other]] = 0.3, 0.5
+    params = dict(PARAMS, lambda1=0.0, lambda2=0.0, alpha=0.0, w0=0.0, direction=-1.0)
+    print(f"[pme] pair at {dist} nm, partner {partner}", flush=True)
+    with pme.ATMPMEForce(q, sig, eps, d, L, 1.0, exceptions=(pairs, qq, es, ee), params=params) as f:
+        r, F, _ = f.evaluate(x)
+    U2, F2, p2 = po.nonbonded_pme(x + d, q, sig, eps, L, 1.0, pairs, qq, es, ee)
+    # the sums' magnitudes (pairs of x + d may be close too), as the tests above
+    scale = sum(abs(p2[k]) for k in ("direct_coulomb", "direct_lj", "exclusion_correction", "self"))
+    assert abs(r["state2_energy"] - U2) <= E_REL * max(1.0, scale)
+    if dist > 0.0:  # (two atoms in one place have no energy at x)
+        U1, _, _ = po.nonbonded_pme(x, q, sig, eps, L, 1.0, pairs, qq, es, ee, forces=False)
+        assert abs(r["state1_energy"] - U1) <= E_REL * abs(U1)
+        assert abs(r["energy"] - U2) <= E_REL * max(1.0, scale)
+        assert np.abs(F - F2).max() < F_ABS + 1e-12 * np.abs(F2).max()
