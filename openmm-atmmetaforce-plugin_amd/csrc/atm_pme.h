@@ -85,10 +85,12 @@ struct PmePtrs {
     const double* eoff;          // [2] energies of other variable-group forces added to U1, U2 (in the input block)
     int* overflow;
     // page-locked host memory the kernels read and write in place: the parameters, offsets and
-    // positions of this evaluation, copied by the first kernel to `in`, and its results
+    // positions of this evaluation, copied by the first kernel to `in`, and its results (every address
+    // the kernels use is in here: a captured evaluation is made again when one of them changes)
     const double* hostIn;   // [kPmeInHead + 3n]
     double* in;             // [kPmeInHead + 3n] (params, eoff and x point into it)
     struct PmeHostRecord* record;
+    double* hostF;          // [3n] the force, atom by atom
 };
 
 // The head of the input block: the nine ATM parameters and the two offsets, padded.
@@ -115,8 +117,8 @@ struct BondedPtrs {
 hipError_t launch_pme_fill(unsigned long long* p, long long n, hipStream_t st);
 // Every kernel of one evaluation (single: state 0 only) up to the energy sums.
 hipError_t launch_pme_states(const PmeDesc& D, const PmePtrs& P, bool single, hipStream_t st);
-// forcesOut: page-locked host memory, or null
-hipError_t launch_pme_finish(const PmeDesc& D, const PmePtrs& P, bool single, double* forcesOut, hipStream_t st);
+// Energy sums and combine; forces: the hybrid force into P.hostF
+hipError_t launch_pme_finish(const PmeDesc& D, const PmePtrs& P, bool single, bool forces, hipStream_t st);
 hipError_t launch_bonded(const BondedPtrs& B, double* eslot, int nblocks, hipStream_t st);
 
 }  // namespace atm

@@ -1102,7 +1102,7 @@ __global__ void __launch_bounds__(1024) k_pme_finish(PmeDesc D, PmePtrs P, int s
 // Writes straight to the host's page-locked memory, consecutive lanes consecutive doubles;
 // with the inputs' copy in k_pme_begin and the record of k_pme_finish this replaces two copies in
 // and four out, 274 -> 208 us (8k atoms) and 435 -> 360 us (25k).
-__global__ void k_pme_blend(PmeDesc D, PmePtrs P, int single, double* out) {
+__global__ void k_pme_blend(PmeDesc D, PmePtrs P, int single) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= 3 * D.n) return;
     const int i = j / 3, k = (j - 3 * i) * D.n + i;  // the sums are SoA
@@ -1111,7 +1111,7 @@ __global__ void k_pme_blend(PmeDesc D, PmePtrs P, int single, double* out) {
     const unsigned long long both = P.F[6ll * D.n + k];
     const double f1 = (double)(long long)(P.F[k] + both) * (1.0 / kFix);
     const double f2 = single ? 0.0 : (double)(long long)(P.F[3ll * D.n + k] + both) * (1.0 / kFix);
-    out[j] = (1.0 - a) * f1 + a * f2;
+    P.hostF[j] = (1.0 - a) * f1 + a * f2;
 }
 
 __global__ void k_pme_fill(unsigned long long* p, long long n) {
@@ -1221,9 +1221,9 @@ hipError_t launch_pme_states(const PmeDesc& D, const PmePtrs& P, bool single, hi
     return hipGetLastError();
 }
 
-hipError_t launch_pme_finish(const PmeDesc& D, const PmePtrs& P, bool single, double* forcesOut, hipStream_t st) {
+hipError_t launch_pme_finish(const PmeDesc& D, const PmePtrs& P, bool single, bool forces, hipStream_t st) {
     k_pme_finish<<<1, 1024, 0, st>>>(D, P, single ? 1 : 0);
-    if (forcesOut) k_pme_blend<<<blocks_of(3ll * D.n, 256), 256, 0, st>>>(D, P, single ? 1 : 0, forcesOut);
+    if (forces) k_pme_blend<<<blocks_of(3ll * D.n, 256), 256, 0, st>>>(D, P, single ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -331,6 +331,7 @@ void set_box(PmeForce& S, const double box[3]) {
     P.hostIn = S.hIn.as<double>();
     P.in = S.dIn.as<double>();
     P.record = S.hRecord.as<PmeHostRecord>();
+    P.hostF = S.hOut.as<double>();
     P.x = P.in + kPmeInHead;
     P.x2 = S.dX2.as<double>();
     P.displ = S.dDispl.as<double>();
@@ -567,7 +568,7 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
                 hipGraph_t graph = nullptr;
                 HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
                 hipError_t e = launch_pme_states(S.D, S.P, single, st);
-                if (e == hipSuccess) e = launch_pme_finish(S.D, S.P, single, forces ? S.hOut.as<double>() : nullptr, st);
+                if (e == hipSuccess) e = launch_pme_finish(S.D, S.P, single, forces != nullptr, st);
                 const hipError_t ee = hipStreamEndCapture(st, &graph);
                 HIPCHK(e);
                 HIPCHK(ee);

@@ -2,10 +2,12 @@
 (each line axis, prime lengths, the largest planes) and axis by axis, and x + d as the
 difference from x (none displaced, displaced alike, displaced differently, exceptions
 across) or in full (many displaced)."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from atmmetaforce import pme
+from atmmetaforce import _capi as C, pme
 from oracle import pme_oracle as po
 from test_pme_gpu import E_REL, F_ABS, PARAMS, _oracle_atm, _small_system
 
@@ -105,3 +107,33 @@ def test_clash_at_x_leaves_the_other_state_alone(gpu, dist, partner):
         assert abs(r["state1_energy"] - U1) <= E_REL * abs(U1)
         assert abs(r["energy"] - U2) <= E_REL * max(1.0, scale)
         assert np.abs(F - F2).max() < F_ABS + 1e-12 * np.abs(F2).max()
+
+
+def _set_particles(f, *arrays):
+    C.check(f._lib.atm_pme_set_particles(f._h, *[np.ascontiguousarray(a, dtype=np.float64).ctypes.data_as(
+        ctypes.POINTER(ctypes.c_double)) for a in arrays]))
+
+
+def test_changed_particles_and_exceptions(gpu):
+    """A change of the particles, displacements or exceptions gives the object new buffers, the one
+    its forces are written to among them: what it computes next is what a new object computes."""
+    x, q, sig, eps, L, pairs, qq, es, ee, d = _small_system(seed=29)
+    rng = np.random.default_rng(5)
+    kinds = (dict(), dict(state1_only=True), dict(forces=False))
+    with pme.ATMPMEForce(q, sig, eps, d, L, 1.0, exceptions=(pairs, qq, es, ee), params=PARAMS) as f:
+        for step in range(6):
+            for kind in kinds:  # an evaluation of each kind captured before the change
+                f.evaluate(x, **kind)
+            d = np.where(rng.random((len(q), 1)) < 0.05 + 0.05 * (step % 2), rng.uniform(-1, 1, (len(q), 3)), 0.0)
+            keep = rng.random(len(pairs)) < 0.8
+            exc = (pairs[keep], qq[keep], es[keep], ee[keep])
+            if step % 3 != 2:
+                q = rng.permutation(q)
+            _set_particles(f, q, sig, eps, d)
+            f.set_exceptions(*exc)
+            print(f"[pme] change {step}", flush=True)
+            with pme.ATMPMEForce(q, sig, eps, d, L, 1.0, exceptions=exc, params=PARAMS) as new:
+                for kind in kinds + kinds:
+                    (r, F, p), (rn, Fn, pn) = f.evaluate(x, **kind), new.evaluate(x, **kind)
+                    assert r == rn and (F is None or np.array_equal(F, Fn))
+                    assert kind.get("state1_only") or p == pn
