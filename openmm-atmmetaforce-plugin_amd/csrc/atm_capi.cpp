@@ -48,6 +48,8 @@ std::string& last_error() {
 using namespace atm;
 
 namespace {
+constexpr int kForceWindow = 4;  // systems whose forces one read sends at most
+
 struct Context {
     int device = 0;
     hipStream_t own = nullptr;
@@ -76,10 +78,10 @@ struct Context {
     DevBuf dGq, dGsig, dGeps, dWset, dDq, dDsig, dDeps;
     DevBuf dFlag;  // validation counter
     // page-locked host memory that kernels use in place (see HostBuf): the evaluations' records,
-    // the counter of atm_set_particles_device, one system's force on its way out (two in turn), and on
-    // their way in one system's FP32 positions (two in turn), the parameters and the gradient weights
-    HostBuf hRecord, hFlag, hForce[2];
-    int forceLast = -1, forceAhead = -1;  // the system last read, the one sent ahead of being asked for
+    // the counter of atm_set_particles_device, the forces of up to kForceWindow systems on their way
+    // out, and on their way in one system's FP32 positions (two in turn), the parameters and the weights
+    HostBuf hRecord, hFlag, hForce;
+    int forceLo = 0, forceHi = 0;  // the systems whose force hForce holds
     Upload upPos[2], upParams, upWset;
     int upNext = 0;
     // exceptions (atm_set_exceptions): per system, near masks, far partner lists and
@@ -792,7 +794,7 @@ void fetch_results(Context& C) {
     if (!C.evaluated) fail(ATM_ERR_STATE, "no evaluation has been run");
     HIPCHK(hipStreamSynchronize(C.stream));
     if (C.resultsValid) return;
-    C.forceLast = C.forceAhead = -1;
+    C.forceLo = C.forceHi = 0;
     struct Lists {
         int overflow, maxEntries, maxAtoms;
     };
@@ -847,31 +849,27 @@ void fetch_results(Context& C) {
 }
 
 // One system's force, atom by atom, in page-locked memory (valid until the next call; after
-// fetch_results, which waits for the stream).  A caller that reads system after system has
-// the next one sent while it takes this one away: 22 systems of 23,000 atoms 670 us instead
-// of 830 us.  Only from the second of two successive systems on, so that a caller of single
-// systems sends nothing that it does not ask for.
+// fetch_results, which waits for the stream).  Each wait costs some 8 us beside the bytes, so a
+// caller that reads system after system gets 1, 2, then kForceWindow of them sent at a time: what
+// has not been asked for is at most as much again as what has.  The stream is waited for here:
+// nothing is in flight when the call returns.  Until the force changes (fetch_results after an
+// evaluation, atm_clear_forces) the systems sent are served from this memory.
 const double* fetch_force(Context& C, int s) {
-    for (HostBuf& b : C.hForce)
-        if (!b.p) b.alloc(sizeof(double) * 3 * C.maxAtoms);
-    auto send = [&](int sys, int half) {
-        HIPCHK(launch_export_forces(C.dOutF.as<double>() + 3ll * C.atomOff[sys], C.sys[sys].num_atoms,
-                                    C.hForce[half].as<double>(), C.stream));
-    };
-    const int half = s & 1;
-    if (C.forceAhead != s) {
-        C.forceAhead = -1;
-        send(s, half);
+    if (!C.hForce.p) C.hForce.alloc(sizeof(double) * 3 * C.maxAtoms * std::min(C.nsys, kForceWindow));
+    if (s < C.forceLo || s >= C.forceHi) {
+        const int sent = C.forceHi - C.forceLo, run = sent > 0 && s == C.forceHi ? std::min(2 * sent, kForceWindow) : 1;
+        C.forceLo = C.forceHi = 0;
+        const int hi = std::min(s + run, C.nsys);
+        double* out = C.hForce.as<double>();
+        for (int k = s; k < hi; ++k) {
+            HIPCHK(launch_export_forces(C.dOutF.as<double>() + 3ll * C.atomOff[k], C.sys[k].num_atoms, out, C.stream));
+            out += 3ll * C.sys[k].num_atoms;
+        }
         HIPCHK(hipStreamSynchronize(C.stream));
+        C.forceLo = s;
+        C.forceHi = hi;
     }
-    const bool successive = s > 0 && C.forceLast == s - 1;
-    C.forceAhead = -1;
-    C.forceLast = s;
-    if (successive && s + 1 < C.nsys) {
-        send(s + 1, half ^ 1);
-        C.forceAhead = s + 1;
-    }
-    return C.hForce[half].as<double>();
+    return C.hForce.as<double>() + 3ll * (C.atomOff[s] - C.atomOff[C.forceLo]);
 }
 
 void upload_system(Context& C, int s) {
@@ -1304,7 +1302,7 @@ int atm_clear_forces(void* context) {
         HIPCHK(hipSetDevice(C.device));
         HIPCHK(launch_fill_zero(C.P.outF, 3 * C.totalAtoms, C.stream));
         HIPCHK(hipStreamSynchronize(C.stream));
-        C.forceLast = C.forceAhead = -1;
+        C.forceLo = C.forceHi = 0;
     });
 }
 

@@ -62,3 +62,21 @@ def test_device_parameters_refused_unchanged(gpu):
             b.set_particles_device(*[c.data_ptr() for c in cols])
         b.compute()
         assert [b.result(k) for k in range(2)] == before[0] and np.array_equal(b.forces(1), before[1])
+
+
+def test_reads_leave_the_stream_idle(gpu):
+    """A force read returns with its work done: nothing of another system is still on its way on
+    the caller's stream."""
+    systems = _systems((40000, 30001, 40000, 39999, 7, 40000, 20000))
+    stream = torch.cuda.Stream()
+    with ATMBatch(systems) as b:
+        b.set_stream(stream.cuda_stream)
+        b.compute()
+        first = []
+        for k in range(len(systems)):
+            first.append(b.forces(k))
+            assert stream.query(), k
+        for k in (3, 4, 0, 1, 6, 5, 2):
+            assert np.array_equal(b.forces(k), first[k])
+            assert stream.query(), k
+        b.set_stream(None)
