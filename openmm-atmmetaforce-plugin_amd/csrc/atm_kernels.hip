@@ -1178,9 +1178,11 @@ __device__ __forceinline__ void flush_component_u(const DevPtrs& P, int c, float
 // 27 us with 16; 6 x 9,001 triclinic (1,000 groups) 285 -> 69 us with 8; 6 x 23,000
 // (2,400 groups) 171 -> 95 us with 4; 22 x 23,000 (8,800 groups) 342 -> 302 us with 2.
 // Registers: 5 waves per SIMD (96 VGPRs) for 2 and 4 waves per group (6 waves spill
-// inside the entry loop: 353 against 312 us on 22 x 23,000), 4 for the longer blocks.
+// inside the entry loop: 353 against 312 us on 22 x 23,000), 4 for the longer blocks.  FP32
+// pairs: 6 (80 VGPRs, a few values spilled outside the loop); whole evaluations with 5 / 6 / 7
+// waves per SIMD: 22 x 23,000 418 / 413 / 427 us, 64 of 5,000 to 60,000 1104 / 1050 / 1091.
 template <int W, bool FORCES, bool F64, bool BWD, bool EXC>
-__global__ void __launch_bounds__(64 * W, W >= 8 ? 4 : 5) k_pairs(DevPtrs P, int setBegin, const double* wset) {
+__global__ void __launch_bounds__(64 * W, W >= 8 ? 4 : (F64 ? 5 : 6)) k_pairs(DevPtrs P, int setBegin, const double* wset) {
     static_assert(!BWD || (F64 && !FORCES), "the backward mode is FP64 and computes no forces");
     constexpr bool JSUMS = FORCES || BWD;  // per-atom j sums flushed every kJFlush entries
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
