@@ -33,41 +33,25 @@
 #include "atm_internal.h"
 #include "atm_kernels.h"
 #include "atm_math.h"
+#include "atm_wrap.h"
 
 namespace atm {
 
 // ---------------------------------------------------------------- helpers
 
-__device__ __forceinline__ float wrap_coord(float x, float L, float invL) {
-    // x - L floor(x/L) is exact on the 2^-20 grid (single rounding of an
-    // exactly representable result); one correction step fixes floor() misses.
-    float w = fmaf(-L, floorf(x * invL), x);
-    if (w < 0.0f) w += L;
-    if (w >= L) w -= L;
-    return w;
-}
-
 __device__ __forceinline__ float min_image(float d, float L, float invL) {
     return fmaf(-L, rintf(d * invL), d);
 }
 
-// Triclinic box in OpenMM's reduced form (a = (L0, 0, 0), b = (tilt0, L1, 0),
-// c = (tilt1, tilt2, L2)): wrap a position into the brick [0, L0) x [0, L1) x
-// [0, L2), which tiles space under the lattice -- by c to 0 <= z < L2, then by b
-// to 0 <= y < L1, then by a.  Each step is exact on the 2^-20 grid below 16 nm.
-__device__ __forceinline__ void wrap_tri(const SetDesc& D, float4& p) {
-    float n = floorf(p.z * D.invL[2]);
-    const float z = fmaf(-D.L[2], n, p.z);
-    n += z < 0.f ? -1.f : (z >= D.L[2] ? 1.f : 0.f);
-    p.z = fmaf(-D.L[2], n, p.z);
-    p.y = fmaf(-D.tilt[2], n, p.y);
-    p.x = fmaf(-D.tilt[1], n, p.x);
-    n = floorf(p.y * D.invL[1]);
-    const float y = fmaf(-D.L[1], n, p.y);
-    n += y < 0.f ? -1.f : (y >= D.L[1] ? 1.f : 0.f);
-    p.y = fmaf(-D.L[1], n, p.y);
-    p.x = fmaf(-D.tilt[0], n, p.x);
-    p.x = wrap_coord(p.x, D.L[0], D.invL[0]);
+// The position p wrapped into set D's box.
+__device__ __forceinline__ void wrap_position(const SetDesc& D, float4& p) {
+    if (D.tri) {
+        wrap_tri(D.L, D.invL, D.tilt, p.x, p.y, p.z);
+    } else {
+        p.x = wrap_coord(p.x, D.L[0], D.invL[0]);
+        p.y = wrap_coord(p.y, D.L[1], D.invL[1]);
+        p.z = wrap_coord(p.z, D.L[2], D.invL[2]);
+    }
 }
 
 // The x and y parts of OpenMM's triclinic image of a pair difference (shift by c
@@ -407,13 +391,7 @@ __device__ __forceinline__ int bin_atom(const DevPtrs& P, const SetDesc& D, int 
         float4 d = P.displ[D.atomOff + i];
         p.x += d.x; p.y += d.y; p.z += d.z;  // exact on the 2^-20 grid
     }
-    if (D.tri) {
-        wrap_tri(D, p);
-    } else {
-        p.x = wrap_coord(p.x, D.L[0], D.invL[0]);
-        p.y = wrap_coord(p.y, D.L[1], D.invL[1]);
-        p.z = wrap_coord(p.z, D.L[2], D.invL[2]);
-    }
+    wrap_position(D, p);
     // clamp in float before the conversion: every index stays inside the grid
     const int cx = (int)fminf(fmaxf(p.x * D.invCe[0], 0.f), (float)(D.nx - 1));
     const int cy = (int)fminf(fmaxf(p.y * D.invCe[1], 0.f), (float)(D.ny - 1));
@@ -2347,13 +2325,7 @@ __device__ __forceinline__ float4 displaced_position(const DevPtrs& P, const Set
         const float4 d = P.displ[D.atomOff + a];
         p.x += d.x; p.y += d.y; p.z += d.z;  // exact on the 2^-20 grid
     }
-    if (D.tri) {
-        wrap_tri(D, p);
-    } else {
-        p.x = wrap_coord(p.x, D.L[0], D.invL[0]);
-        p.y = wrap_coord(p.y, D.L[1], D.invL[1]);
-        p.z = wrap_coord(p.z, D.L[2], D.invL[2]);
-    }
+    wrap_position(D, p);
     return p;
 }
 
@@ -2494,11 +2466,8 @@ __global__ void __launch_bounds__(256) k_displaced(DevPtrs P, int sysBegin, int 
                 const int* ccs = P.cellStart + D.cellOff + (long long)col * D.nz;
                 const int* ccn = P.cellCount + D.cellOff + (long long)col * D.nz;
                 const float hz = sqrtf(lim2 - rho2);
-                int za0 = (int)floorf((p.z - hz) * D.invZe) - 1, za1 = (int)floorf((p.z + hz) * D.invZe) + 1;
-                int zb0 = 1, zb1 = 0;
-                if (za1 - za0 + 1 >= D.nz) { za0 = 0; za1 = D.nz - 1; }
-                else if (za0 < 0) { zb0 = za0 + D.nz; zb1 = D.nz - 1; za0 = 0; }
-                else if (za1 >= D.nz) { zb0 = 0; zb1 = za1 - D.nz; za1 = D.nz - 1; }
+                int za0, za1, zb0, zb1;
+                z_bins(p.z, hz, D.invZe, D.L[2], D.nz, za0, za1, zb0, zb1);
                 // slot ranges -> cluster ranges (clusters never straddle columns)
                 const int s0 = cs + ccs[za0], e0 = cs + ccs[za1] + ccn[za1];
                 b0 = s0 >> 3;

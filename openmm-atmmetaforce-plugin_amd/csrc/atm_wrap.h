@@ -1,0 +1,76 @@
+// Periodic images of one FP32 position: wrapping into the box, the lattice images of a
+// box pair and the z-bins of a cutoff, for the kernels of atm_kernels.hip (and for the
+// host program that tests them).  Positions may be any float: what is made from a
+// wrapped position (cell and bin indices, cluster boxes, image counts) relies on
+// 0 <= w <= L, so a coordinate too large for one FP32 step to bring home is folded again
+// and, past that, put on the edge.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <cmath>
+
+namespace atm {
+
+__host__ __device__ inline float fold_coord(float x, float L, float invL) {
+    // x - L floor(x/L) is exact on the 2^-20 grid (single rounding of an
+    // exactly representable result); one correction step fixes floor() misses.
+    float w = fmaf(-L, floorf(x * invL), x);
+    if (w < 0.0f) w += L;
+    if (w >= L) w -= L;
+    return w;
+}
+
+__host__ __device__ inline float clamp_coord(float w, float L) { return w < 0.0f ? 0.0f : (w > L ? L : w); }  // (NaN stays)
+
+__host__ __device__ inline float wrap_coord(float x, float L, float invL) {
+    float w = fold_coord(x, L, invL);
+    if (w < 0.0f || w > L) w = clamp_coord(fold_coord(w, L, invL), L);  // floor() missed by more than one (x beyond 4e6 L)
+    return w;
+}
+
+// Triclinic box in OpenMM's reduced form (a = (L0, 0, 0), b = (tilt0, L1, 0),
+// c = (tilt1, tilt2, L2)): wrap a position into the brick [0, L0) x [0, L1) x
+// [0, L2), which tiles space under the lattice -- by c to 0 <= z < L2, then by b
+// to 0 <= y < L1, then by a.  Each step is exact on the 2^-20 grid below 16 nm.
+__host__ __device__ inline void fold_tri(const float* L, const float* invL, const float* tilt, float& px, float& py,
+                                         float& pz) {
+    float n = floorf(pz * invL[2]);
+    const float z = fmaf(-L[2], n, pz);
+    n += z < 0.f ? -1.f : (z >= L[2] ? 1.f : 0.f);
+    pz = fmaf(-L[2], n, pz);
+    py = fmaf(-tilt[2], n, py);
+    px = fmaf(-tilt[1], n, px);
+    n = floorf(py * invL[1]);
+    const float y = fmaf(-L[1], n, py);
+    n += y < 0.f ? -1.f : (y >= L[1] ? 1.f : 0.f);
+    py = fmaf(-L[1], n, py);
+    px = fmaf(-tilt[0], n, px);
+    px = fold_coord(px, L[0], invL[0]);
+}
+
+__host__ __device__ inline void wrap_tri(const float* L, const float* invL, const float* tilt, float& px, float& py,
+                                         float& pz) {
+    fold_tri(L, invL, tilt, px, py, pz);
+    if (px < 0.f || px > L[0] || py < 0.f || py > L[1] || pz < 0.f || pz > L[2]) {
+        fold_tri(L, invL, tilt, px, py, pz);
+        px = clamp_coord(px, L[0]);
+        py = clamp_coord(py, L[1]);
+        pz = clamp_coord(pz, L[2]);
+    }
+}
+
+// The z-bins (nz of them, 1 / invZe wide, over [0, Lz]) within hz of z and one more on each
+// side, as [za0, za1] and, where they wrap, [zb0, zb1] (empty: zb0 > zb1): every bin at most
+// once, every index in [0, nz), whatever z, for 0 <= hz <= Lz.
+__host__ __device__ inline void z_bins(float z, float hz, float invZe, float Lz, int nz, int& za0, int& za1, int& zb0,
+                                       int& zb1) {
+    z = fminf(fmaxf(z, 0.f), Lz);  // (NaN: 0)
+    za0 = (int)floorf((z - hz) * invZe) - 1;
+    za1 = (int)floorf((z + hz) * invZe) + 1;
+    zb0 = 1;
+    zb1 = 0;
+    if (za1 - za0 + 1 >= nz) { za0 = 0; za1 = nz - 1; }
+    else if (za0 < 0) { zb0 = za0 + nz; zb1 = nz - 1; za0 = 0; }
+    else if (za1 >= nz) { zb0 = 0; zb1 = za1 - nz; za1 = nz - 1; }
+}
+
+}  // namespace atm
