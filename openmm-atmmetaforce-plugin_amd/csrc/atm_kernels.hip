@@ -87,14 +87,6 @@ __device__ __forceinline__ void pair_image(const SetDesc& D, float& dx, float& d
     dz = min_image(dz, D.L[2], D.invL[2]);
 }
 
-// The images n of one lattice direction (edge 1 / invL) under which |d - n L| - h < r can hold:
-// [n0, n1], often empty or one.  1e-4 of the edge of slack covers the rounding here; the
-// caller's test of each image decides.
-__device__ __forceinline__ void image_range(float d, float reach, float invL, int& n0, int& n1) {
-    n0 = (int)ceilf(fmaf(d - reach, invL, -1e-4f));
-    n1 = (int)floorf(fmaf(d + reach, invL, 1e-4f));
-}
-
 // f(dx, dy, dz) for every lattice image n_a a + n_b b + n_c c of a triclinic box under which
 // two boxes with centre difference d and summed half-extents h hold points closer than
 // sqrt(r2): the centre difference under that image.  f returns true to end the walk.
@@ -911,8 +903,9 @@ __global__ void __launch_bounds__(64 * W) k_pairlist(DevPtrs P, int setBegin) {
                 if (TRI && D.tri) {
                     // triclinic: the images under which the j-cluster reaches the group's box (1e-3 nm
                     // wider: the clusters' own tests round otherwise), mostly none or one, and the
-                    // group's clusters under each.  Every image of every cluster instead, from bounds
-                    // one image wider on each side, took 80 us for 6 x 9,001 atoms; this 29.
+                    // group's clusters under each, until all of them are in.  Every image of every cluster
+                    // instead, from bounds one image wider on each side, took 80 us for 6 x 9,001 atoms;
+                    // this 29.
                     tri_each_image(D, jc.x - gcx, jc.y - gcy, jc.z - gcz, ghx + jh.x + 1e-3f, ghy + jh.y + 1e-3f,
                                    ghz + jh.z + 1e-3f, rcl, D.rcList2, [&](float dx, float dy, float dz) {
                         for (int q = 0; q < ncl && g0 + q <= J; ++q) {

@@ -58,6 +58,18 @@ __host__ __device__ inline void wrap_tri(const float* L, const float* invL, cons
     }
 }
 
+// The images n of one lattice direction (edge 1 / invL) under which |d - n L| - h < r can hold
+// (reach = h + r): [n0, n1], often empty or one.  1e-4 of the edge of slack covers the rounding
+// here; the caller's test of each image decides.  Boxes of wrapped positions reach at most 5
+// edges over (the tilts add half an edge per image of the direction before): bounds past 8 come
+// from no position, and a walk over them would not end.
+constexpr float kMaxImages = 8.f;
+__host__ __device__ inline void image_range(float d, float reach, float invL, int& n0, int& n1) {
+    // (NaN: none)
+    n0 = (int)ceilf(fmaxf(fminf(fmaf(d - reach, invL, -1e-4f), kMaxImages), -kMaxImages));
+    n1 = (int)floorf(fminf(fmaxf(fmaf(d + reach, invL, 1e-4f), -kMaxImages), kMaxImages));
+}
+
 // The z-bins (nz of them, 1 / invZe wide, over [0, Lz]) within hz of z and one more on each
 // side, as [za0, za1] and, where they wrap, [zb0, zb1] (empty: zb0 > zb1): every bin at most
 // once, every index in [0, nz), whatever z, for 0 <= hz <= Lz.

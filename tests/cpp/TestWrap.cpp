@@ -64,6 +64,16 @@ int main() {
                 }
             }
         }
+        for (size_t k = 0; k + 1 < x.size(); ++k) {
+            const float d = x[k], reach = std::fabs(x[k + 1]);
+            int n0, n1;
+            image_range(d, reach, invL, n0, n1);
+            CHECK(n0 >= -8 && n1 <= 8, "d %g reach %g: %d..%d", d, reach, n0, n1);
+            if (!(std::fabs(d) <= 3 * L && reach <= 2 * L)) continue;  // differences and boxes inside the cell
+            for (int n = -20; n <= 20; ++n)
+                CHECK(std::fabs((double)d - n * (double)L) >= reach || (n >= n0 && n <= n1), "d %g reach %g: image %d missed (%d..%d)",
+                      d, reach, n, n0, n1);
+        }
         for (int nz : {1, 2, 3, 5, 17, 64, 333, 4096}) {
             const float invZe = (float)(nz / (double)L);
             for (size_t k = 0; k < x.size(); k += 11) {
