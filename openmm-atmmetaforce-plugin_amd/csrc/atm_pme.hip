@@ -45,6 +45,7 @@
 #include <stdint.h>
 #include "atm_pme.h"
 #include "atm_math.h"
+#include "atm_wrap.h"
 
 namespace atm {
 
@@ -109,15 +110,6 @@ __device__ double block_sum(double v, double* red) {
         for (int k = 0; k < NT / 64; ++k) s += red[k];
     __syncthreads();
     return s;
-}
-
-__device__ __forceinline__ int wrap_cell(double x, double L, double invL, int m, double* w) {
-    double v = x - L * floor(x * invL);
-    if (v < 0.0) v += L;
-    if (v >= L) v -= L;
-    *w = v;
-    int c = (int)(v * invL * m);
-    return c < 0 ? 0 : (c >= m ? m - 1 : c);
 }
 
 // Order-5 cardinal B-spline weights M5(w + j) and derivatives M5'(w + j),
@@ -547,9 +539,7 @@ __device__ __forceinline__ double grid_coord(const PmeDesc& D, double x, int d, 
         wrap_cell(x, D.L[d], D.invL[d], D.m[d], &w);
         return w * D.invL[d] * D.K[d];
     }
-    double f = x * D.invL[d];
-    f -= floor(f);
-    return f * D.K[d];
+    return grid_fraction(x, D.invL[d]) * D.K[d];
 }
 
 // The displaced atoms' charges off the grid at x and onto it at x + d, into the
@@ -593,9 +583,7 @@ __global__ void k_pme_spread(PmeDesc D, PmePtrs P, const double* x, unsigned lon
     double th[3][kOrder], dth[kOrder];
     int g0[3];
     for (int d = 0; d < 3; ++d) {
-        double f = x[3 * i + d] * D.invL[d];
-        f -= floor(f);
-        const double u = f * D.K[d];
+        const double u = grid_fraction(x[3 * i + d], D.invL[d]) * D.K[d];
         int g = (int)floor(u);
         const double w = u - g;
         g0[d] = g;
@@ -959,9 +947,7 @@ __device__ __forceinline__ void gather_forces(const PmeDesc& D, const PmePtrs& P
         double th[3][kOrder], dth[3][kOrder];
         int g0[3];
         for (int d = 0; d < 3; ++d) {
-            double f = x[3 * i + d] * D.invL[d];
-            f -= floor(f);
-            const double u = f * D.K[d];
+            const double u = grid_fraction(x[3 * i + d], D.invL[d]) * D.K[d];
             const int g = (int)floor(u);
             g0[d] = g;
             bspline5(u - g, th[d], dth[d]);

@@ -1,6 +1,6 @@
-// Periodic images of one FP32 position: wrapping into the box, the lattice images of a
-// box pair and the z-bins of a cutoff, for the kernels of atm_kernels.hip (and for the
-// host program that tests them).  Positions may be any float: what is made from a
+// Periodic images of one position: wrapping into the box, the lattice images of a box pair
+// and the z-bins of a cutoff (FP32), cells and grid points (FP64), for the kernels of
+// atm_kernels.hip and atm_pme.hip (and for the host program that tests them).  Positions may be any float: what is made from a
 // wrapped position (cell and bin indices, cluster boxes, image counts) relies on
 // 0 <= w <= L, so a coordinate too large for one FP32 step to bring home is folded again
 // and, past that, put on the edge.
@@ -68,6 +68,29 @@ __host__ __device__ inline void image_range(float d, float reach, float invL, in
     // (NaN: none)
     n0 = (int)ceilf(fmaxf(fminf(fmaf(d - reach, invL, -1e-4f), kMaxImages), -kMaxImages));
     n1 = (int)floorf(fminf(fmaxf(fmaf(d + reach, invL, 1e-4f), -kMaxImages), kMaxImages));
+}
+
+// The same for the FP64 positions of the PME evaluation.
+//
+// x wrapped into [0, L) and its cell of m.  Past some 4e15 L the step to the box leaves more than
+// it can take off, and x has no place in the box: 0 (grid points are made from w).
+__host__ __device__ inline int wrap_cell(double x, double L, double invL, int m, double* w) {
+    double v = x - L * floor(x * invL);
+    if (v < 0.0) v += L;
+    if (v >= L) v -= L;
+    if (!(v >= 0.0 && v < L)) v = 0.0;
+    *w = v;
+    int c = (int)(v * invL * m);
+    return c < 0 ? 0 : (c >= m ? m - 1 : c);
+}
+
+// x / L without its whole part, in [0, 1] but for the rounding: the fused step keeps the half unit
+// that the product lost, 1e-16 either way for a position in the box and 64 for one at 1e18 L.  Up
+// to 1/2048 past either end (x of some 1e12 L) the grid point, times K <= 1024, stays in [-1, K];
+// further out x has no place on the grid: 0.
+__host__ __device__ inline double grid_fraction(double x, double invL) {
+    const double f = fma(x, invL, -floor(x * invL));
+    return f > -1.0 / 2048 && f < 1.0 + 1.0 / 2048 ? f : 0.0;
 }
 
 // The z-bins (nz of them, 1 / invZe wide, over [0, Lz]) within hz of z and one more on each

@@ -1,4 +1,4 @@
-// Wrapping, z-bins and lattice images of any float (csrc/atm_wrap.h), on the host.
+// Wrapping, z-bins, lattice images and grid points of any position (csrc/atm_wrap.h), on the host.
 #include <cstdio>
 #include <cstring>
 #include <random>
@@ -92,6 +92,30 @@ int main() {
                         }
                         CHECK(!near || (q >= a0 && q <= a1) || (q >= b0 && q <= b1), "z %g hz %g nz %d: bin %d missed", z, hz, nz, q);
                     }
+                }
+            }
+        }
+    }
+    for (double L : {3.05, 4.217, 41.37}) {
+        const double invL = 1.0 / L;
+        for (int k = 0; k < 200000; ++k) {
+            double v;
+            uint64_t bits = (uint64_t)rng() << 32 | rng();
+            std::memcpy(&v, &bits, 8);  // every exponent and sign
+            if (k & 1) v = std::ldexp((double)rng() / 4294967296.0 - 0.5, (int)(rng() % 90) - 10);
+            const double f = grid_fraction(v, invL);
+            for (int K : {5, 27, 35, 1024}) {
+                const int g = (int)std::floor(f * K);
+                CHECK(g >= -1 && g <= K, "%g: grid point %d of %d", v, g, K);
+            }
+            for (int m : {3, 4, 40}) {
+                double w;
+                const int c = wrap_cell(v, L, invL, m, &w);
+                CHECK(c >= 0 && c < m && w >= 0.0 && w < L, "%g: cell %d of %d, %g", v, c, m, w);
+                if (std::fabs(v) < 1e6) {
+                    CHECK(std::fabs(std::remainder(v - w, L)) < 1e-9, "%.17g -> %.17g in %g", v, w, L);
+                    const double df = f * L - w;
+                    CHECK(std::fabs(std::remainder(df, L)) < 1e-9, "%.17g -> %.17g in %g: fraction %.17g", v, w, L, f);
                 }
             }
         }

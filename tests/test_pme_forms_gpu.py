@@ -137,3 +137,19 @@ def test_changed_particles_and_exceptions(gpu):
                     (r, F, p), (rn, Fn, pn) = f.evaluate(x, **kind), new.evaluate(x, **kind)
                     assert r == rn and (F is None or np.array_equal(F, Fn))
                     assert kind.get("state1_only") or p == pn
+
+
+def test_far_positions(gpu):
+    """Charged atoms at coordinates that no FP64 step brings back into the box: the evaluation ends
+    inside its grids, and the next one is as it was."""
+    x, q, sig, eps, L, pairs, qq, es, ee, d = _small_system(seed=31)
+    far = x.copy()
+    far[[7, 50, 399]] = [3e16, -1e17, 2e18], [-4e200, 1.0, 1e300], [2.0, -1e19, 1e25]  # atom 50 is displaced
+    with pme.ATMPMEForce(q, sig, eps, d, L, 1.0, exceptions=(pairs, qq, es, ee), params=PARAMS) as f:
+        r, F, _ = f.evaluate(x)
+        for grid_state in (dict(), dict(state1_only=True)):
+            print(f"[pme] far positions {grid_state}", flush=True)
+            rf, Ff, _ = f.evaluate(far, **grid_state)
+            assert np.isfinite(rf["state1_energy"]) and np.isfinite(Ff).all()
+        r2, F2, _ = f.evaluate(x)
+    assert r2 == r and np.array_equal(F2, F)

@@ -1,4 +1,4 @@
-"""Wrapping, z-bins and lattice images of any FP32 position (csrc/atm_wrap.h), on the host."""
+"""Wrapping, z-bins, lattice images and grid points of any position (csrc/atm_wrap.h), on the host."""
 import os
 import subprocess
 
