@@ -48,7 +48,9 @@ std::string& last_error() {
 using namespace atm;
 
 namespace {
-constexpr int kForceWindow = 4;  // systems whose forces one read sends at most
+constexpr int kForceWindow = 4;             // systems whose forces one read sends at most ...
+constexpr long long kForceStage = 1 << 19;  // ... and doubles (4 MiB)
+constexpr int kPosStage = 1 << 16;          // atoms whose positions one upload sends
 
 struct Context {
     int device = 0;
@@ -77,12 +79,18 @@ struct Context {
     DevBuf dLptItems;  // the tile kernel's longest-first group order
     DevBuf dGq, dGsig, dGeps, dWset, dDq, dDsig, dDeps;
     DevBuf dFlag;  // validation counter
-    // page-locked host memory that kernels use in place (see HostBuf): the evaluations' records,
-    // the counter of atm_set_particles_device, the forces of up to kForceWindow systems on their way
-    // out, and on their way in one system's FP32 positions (two in turn), the parameters and the weights
-    HostBuf hRecord, hFlag, hForce;
+    // page-locked host memory that kernels use in place (see HostBuf), one block taken at creation
+    // (each block costs some 40 us to take and give back, the first of a size 350): the evaluations'
+    // records, the counter of atm_set_particles_device, forces on their way out, and on their way
+    // in FP32 positions (two in turn), the parameters and the gradient weights
+    HostBuf hBlock;
+    HostRecord* hRecord = nullptr;
+    int* hFlag = nullptr;
+    double* hForce = nullptr;
+    long long forceCap = 0;        // doubles of hForce
     int forceLo = 0, forceHi = 0;  // the systems whose force hForce holds
     Upload upPos[2], upParams, upWset;
+    int posCap = 0;                // atoms of each of upPos
     int upNext = 0;
     // exceptions (atm_set_exceptions): per system, near masks, far partner lists and
     // the terms with a nonzero charge product or epsilon; batch arrays on the device
@@ -451,7 +459,7 @@ void alloc_layout(Context& C) {
     P.prm64 = C.dPrm64.as<double4>();
     P.params = C.dParams.as<AtmParamsDev>();
     P.res = C.dRes.as<SysResult>();
-    P.host = C.hRecord.as<HostRecord>();
+    P.host = C.hRecord;
     P.outF = C.dOutF.as<double>();
     P.bpos = C.dBpos.as<float4>();
     P.bcell = C.dBcell.as<int>();
@@ -601,7 +609,7 @@ void flush_params(Context& C) {
     }
     if (!C.paramsDirty) return;
     const size_t bytes = sizeof(AtmParamsDev) * C.nsys;
-    void* stage = C.upParams.begin(bytes, C.stream);
+    void* stage = C.upParams.begin(C.stream);
     std::memcpy(stage, C.params.data(), bytes);
     HIPCHK(launch_copy8(C.dParams.p, stage, (long long)(bytes / 8), C.stream));
     C.upParams.end(C.stream);
@@ -799,7 +807,7 @@ void fetch_results(Context& C) {
         int overflow, maxEntries, maxAtoms;
     };
     std::vector<Lists> rt(2 * C.nsys);
-    const HostRecord* rec = C.hRecord.as<HostRecord>();  // left by the batched evaluation's k_energy
+    const HostRecord* rec = C.hRecord;  // left by the batched evaluation's k_energy
     if (C.resultsOnHost) {
         std::vector<SetRuntime> dev(2 * C.nsys);
         to_host(C, dev.data(), C.dRt.p, sizeof(SetRuntime) * dev.size());
@@ -848,28 +856,44 @@ void fetch_results(Context& C) {
     }
 }
 
-// One system's force, atom by atom, in page-locked memory (valid until the next call; after
-// fetch_results, which waits for the stream).  Each wait costs some 8 us beside the bytes, so a
-// caller that reads system after system gets 1, 2, then kForceWindow of them sent at a time: what
-// has not been asked for is at most as much again as what has.  The stream is waited for here:
-// nothing is in flight when the call returns.  Until the force changes (fetch_results after an
-// evaluation, atm_clear_forces) the systems sent are served from this memory.
-const double* fetch_force(Context& C, int s) {
-    if (!C.hForce.p) C.hForce.alloc(sizeof(double) * 3 * C.maxAtoms * std::min(C.nsys, kForceWindow));
+// One system's force, atom by atom, through page-locked memory: take(k0, F, m) for its doubles
+// k0 .. k0 + m - 1 in order (after fetch_results, which waits for the stream).  Each wait costs
+// some 8 us beside the bytes, so a caller that reads system after system gets 1, 2, then
+// kForceWindow of them sent at a time: what has not been asked for is at most as much again as
+// what has.  The stream is waited for here: nothing is in flight when the call returns.  Until
+// the force changes (fetch_results after an evaluation, atm_clear_forces) the systems sent are
+// served from this memory.  A system that it does not hold comes in pieces.
+template <class Take>
+void take_force(Context& C, int s, Take take) {
+    auto send = [&](int sys, long long k0, long long m, double* out) {
+        HIPCHK(launch_export_forces(C.dOutF.as<double>() + 3ll * C.atomOff[sys], C.sys[sys].num_atoms, k0, m, out, C.stream));
+    };
+    const long long n3 = 3ll * C.sys[s].num_atoms;
+    if (n3 > C.forceCap) {
+        C.forceLo = C.forceHi = 0;
+        for (long long k0 = 0; k0 < n3; k0 += C.forceCap) {
+            const long long m = std::min(C.forceCap, n3 - k0);
+            send(s, k0, m, C.hForce);
+            HIPCHK(hipStreamSynchronize(C.stream));
+            take(k0, C.hForce, m);
+        }
+        return;
+    }
     if (s < C.forceLo || s >= C.forceHi) {
         const int sent = C.forceHi - C.forceLo, run = sent > 0 && s == C.forceHi ? std::min(2 * sent, kForceWindow) : 1;
         C.forceLo = C.forceHi = 0;
-        const int hi = std::min(s + run, C.nsys);
-        double* out = C.hForce.as<double>();
-        for (int k = s; k < hi; ++k) {
-            HIPCHK(launch_export_forces(C.dOutF.as<double>() + 3ll * C.atomOff[k], C.sys[k].num_atoms, out, C.stream));
-            out += 3ll * C.sys[k].num_atoms;
+        const long long at = 3ll * C.atomOff[s];
+        int hi = s;
+        for (; hi < C.nsys && hi < s + run; ++hi) {
+            const long long m = 3ll * C.sys[hi].num_atoms, to = 3ll * C.atomOff[hi] - at;
+            if (to + m > C.forceCap) break;
+            send(hi, 0, m, C.hForce + to);
         }
         HIPCHK(hipStreamSynchronize(C.stream));
         C.forceLo = s;
         C.forceHi = hi;
     }
-    return C.hForce.as<double>() + 3ll * (C.atomOff[s] - C.atomOff[C.forceLo]);
+    take(0, C.hForce + 3ll * (C.atomOff[s] - C.atomOff[C.forceLo]), n3);
 }
 
 void upload_system(Context& C, int s) {
@@ -967,7 +991,29 @@ int atm_create(const atm_system_desc* systems, int32_t num_systems, int32_t devi
         C->dPrm64.alloc(sizeof(double4) * off);
         C->dParams.alloc(sizeof(AtmParamsDev) * num_systems);
         C->dRes.alloc(sizeof(SysResult) * num_systems);
-        C->hRecord.alloc(sizeof(HostRecord) * num_systems);
+        {
+            C->posCap = std::min(C->maxAtoms, kPosStage);
+            C->forceCap = std::min(3ll * C->maxAtoms * std::min<int>(num_systems, kForceWindow), kForceStage);
+            size_t at = 0;
+            auto take = [&](size_t bytes) {
+                const size_t here = at;
+                at += (bytes + 255) & ~size_t(255);
+                return here;
+            };
+            const size_t rec = take(sizeof(HostRecord) * num_systems), flag = take(sizeof(int));
+            const size_t prm = take(sizeof(AtmParamsDev) * num_systems), wset = take(sizeof(double) * 2 * num_systems);
+            const size_t row = sizeof(float) * ((3ll * C->posCap + 3) / 4 * 4), pos0 = take(row), pos1 = take(row);
+            const size_t force = take(sizeof(double) * C->forceCap);
+            C->hBlock.alloc(at);
+            char* h = C->hBlock.as<char>();
+            C->hRecord = reinterpret_cast<HostRecord*>(h + rec);
+            C->hFlag = reinterpret_cast<int*>(h + flag);
+            C->upParams.create(h + prm);
+            C->upWset.create(h + wset);
+            C->upPos[0].create(h + pos0);
+            C->upPos[1].create(h + pos1);
+            C->hForce = reinterpret_cast<double*>(h + force);
+        }
         C->dOutF.alloc(sizeof(double) * 3 * off);
         zero_on_stream(*C, C->dPosq.p, sizeof(float4) * off);
         zero_on_stream(*C, C->dDispl.p, sizeof(float4) * off);
@@ -1122,15 +1168,19 @@ int atm_set_positions(void* context, int32_t sys, const double* x) {
             p.x = (float)x[3 * i]; p.y = (float)x[3 * i + 1]; p.z = (float)x[3 * i + 2];
         }
         // x, y, z only: the device may hold charges that the host mirror does not.  Two staging
-        // buffers in turn, so the next system's conversion runs beside this one's upload
-        Upload& up = C.upPos[C.upNext];
-        C.upNext ^= 1;
-        float* xyz = static_cast<float*>(up.begin(sizeof(float) * ((3ll * C.maxAtoms + 3) / 4 * 4), C.stream));
-        for (int i = 0; i < n; ++i) {
-            xyz[3 * i] = C.hPosq[off + i].x; xyz[3 * i + 1] = C.hPosq[off + i].y; xyz[3 * i + 2] = C.hPosq[off + i].z;
+        // buffers in turn, so the next conversion runs beside this one's upload
+        for (int i0 = 0; i0 < n; i0 += C.posCap) {
+            Upload& up = C.upPos[C.upNext];
+            C.upNext ^= 1;
+            const int m = std::min(C.posCap, n - i0);
+            const float4* p = C.hPosq.data() + off + i0;
+            float* xyz = static_cast<float*>(up.begin(C.stream));
+            for (int i = 0; i < m; ++i) {
+                xyz[3 * i] = p[i].x; xyz[3 * i + 1] = p[i].y; xyz[3 * i + 2] = p[i].z;
+            }
+            HIPCHK(launch_upload_positions(C.dPosq.as<float4>() + off + i0, xyz, m, C.stream));
+            up.end(C.stream);
         }
-        HIPCHK(launch_upload_positions(C.dPosq.as<float4>() + off, xyz, n, C.stream));
-        up.end(C.stream);
     });
 }
 
@@ -1149,13 +1199,12 @@ int atm_set_particles_device(void* context, const double* charges, const double*
         if (!charges || !sigmas || !epsilons) fail(ATM_ERR_INVALID_ARGUMENT, "null device array");
         HIPCHK(hipSetDevice(C.device));
         if (!C.dFlag.p) C.dFlag.alloc(sizeof(int));
-        if (!C.hFlag.p) C.hFlag.alloc(sizeof(int));
         zero_on_stream(C, C.dFlag.p, sizeof(int));
         HIPCHK(launch_check_particles(charges, sigmas, epsilons, C.totalAtoms, C.dFlag.as<int>(), C.stream));
         HIPCHK(launch_set_particles(C.P, charges, sigmas, epsilons, C.totalAtoms, std::sqrt(ATM_ONE_4PI_EPS0),
-                                    C.dFlag.as<int>(), C.hFlag.as<int>(), C.stream));
+                                    C.dFlag.as<int>(), C.hFlag, C.stream));
         HIPCHK(hipStreamSynchronize(C.stream));
-        const int bad = *C.hFlag.as<int>();
+        const int bad = *C.hFlag;
         if (bad) fail(ATM_ERR_INVALID_ARGUMENT, std::to_string(bad) + " atoms with a non-finite parameter or a negative "
                                                 "sigma or epsilon (nothing was changed)");
         C.chargesOnDevice = true;
@@ -1276,12 +1325,12 @@ int atm_get_forces_fixed(void* context, int32_t sys, int64_t* f) {
         if (!f) fail(ATM_ERR_INVALID_ARGUMENT, "null output");
         HIPCHK(hipSetDevice(C.device));
         fetch_results(C);
-        const int n = C.sys[sys].num_atoms;
-        const double* F = fetch_force(C, sys);
-        for (long long k = 0; k < 3ll * n; ++k) {
-            const double v = std::fmin(std::fmax(F[k] * ATM_FORCE_SCALE, -9.2e18), 9.2e18);
-            f[k] = (int64_t)std::llrint(v);
-        }
+        take_force(C, sys, [&](long long k0, const double* F, long long m) {
+            for (long long k = 0; k < m; ++k) {
+                const double v = std::fmin(std::fmax(F[k] * ATM_FORCE_SCALE, -9.2e18), 9.2e18);
+                f[k0 + k] = (int64_t)std::llrint(v);
+            }
+        });
     });
 }
 
@@ -1292,7 +1341,7 @@ int atm_get_forces(void* context, int32_t sys, double* f) {
         if (!f) fail(ATM_ERR_INVALID_ARGUMENT, "null output");
         HIPCHK(hipSetDevice(C.device));
         fetch_results(C);
-        std::memcpy(f, fetch_force(C, sys), sizeof(double) * 3 * (size_t)C.sys[sys].num_atoms);
+        take_force(C, sys, [&](long long k0, const double* F, long long m) { std::memcpy(f + k0, F, sizeof(double) * m); });
     });
 }
 
@@ -1683,7 +1732,7 @@ void backward_impl(Context& C, const double* grad_energy, double* d_charges, dou
         }
         ensure_grad_buffers(C);
         if (C.dWset.bytes < sizeof(double) * 2 * S) C.dWset.alloc(sizeof(double) * 2 * S);
-        void* stage = C.upWset.begin(sizeof(double) * 2 * S, C.stream);
+        void* stage = C.upWset.begin(C.stream);
         std::memcpy(stage, wset.data(), sizeof(double) * 2 * S);
         HIPCHK(launch_copy8(C.dWset.p, stage, 2ll * S, C.stream));
         C.upWset.end(C.stream);

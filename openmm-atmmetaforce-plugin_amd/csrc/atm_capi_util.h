@@ -92,18 +92,20 @@ struct HostBuf {
 // refuses a stream under capture, whose replays would read whatever is here by then),
 // end() marks the launch of the reader.
 struct Upload {
-    HostBuf buf;
+    void* p = nullptr;  // page-locked memory, the owner's
     hipEvent_t done = nullptr;
     bool used = false;
-    void* begin(size_t bytes, hipStream_t st) {
+    void create(void* memory) {
+        p = memory;
+        HIPCHK(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    }
+    void* begin(hipStream_t st) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         HIPCHK(hipStreamIsCapturing(st, &cap));
         if (cap != hipStreamCaptureStatusNone) fail(ATM_ERR_DEVICE, "host data cannot be set on a stream under capture");
         if (used) HIPCHK(hipEventSynchronize(done));
         used = false;
-        if (!done) HIPCHK(hipEventCreateWithFlags(&done, hipEventDisableTiming));
-        if (buf.bytes < bytes) buf.alloc(bytes);
-        return buf.p;
+        return p;
     }
     void end(hipStream_t st) {
         used = true;

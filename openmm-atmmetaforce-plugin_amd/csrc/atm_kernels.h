@@ -147,8 +147,9 @@ hipError_t launch_displaced_dump(const DevPtrs& P, int sys, int state, int nLig,
 hipError_t launch_fill_i64(long long* p, long long n, hipStream_t st);
 hipError_t launch_fill_zero(void* p, long long n8, hipStream_t st);
 hipError_t launch_copy8(void* dst, const void* src, long long n8, hipStream_t st);
-// The force of one system (SoA, n atoms) into out (AoS, page-locked host memory).
-hipError_t launch_export_forces(const double* F, int n, double* out, hipStream_t st);
+// Doubles k0 .. k0 + m - 1 of the force of one system (SoA, n atoms), atom by atom, into out[0 ...]
+// (page-locked host memory).
+hipError_t launch_export_forces(const double* F, int n, long long k0, long long m, double* out, hipStream_t st);
 hipError_t launch_pairs_dump(const DevPtrs& P, int c, int maxGroups, int2* out, long long cap,
                              unsigned long long* counters, hipStream_t st);
 

@@ -2758,11 +2758,11 @@ __global__ void k_blend(DevPtrs P, int sysBegin, int nsys, int gx, int hostMode,
 
 // Consecutive lanes write consecutive doubles (whole lines over the link to the host); the
 // gathered reads are the L2's, which the blend has just filled.
-__global__ void k_export_forces(const double* F, int n, double* out) {
-    const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (k >= 3ll * n) return;
+__global__ void k_export_forces(const double* F, int n, long long k0, long long m, double* out) {
+    const long long j = blockIdx.x * (long long)blockDim.x + threadIdx.x, k = k0 + j;
+    if (j >= m) return;
     const long long i = k / 3;
-    out[k] = F[(k - 3 * i) * n + i];
+    out[j] = F[(k - 3 * i) * n + i];
 }
 
 __global__ void k_copy8(unsigned long long* dst, const unsigned long long* src, long long n) {
@@ -2908,9 +2908,9 @@ hipError_t launch_energy(const DevPtrs& P, int sysBegin, int nsys, int estride, 
     return hipGetLastError();
 }
 
-hipError_t launch_export_forces(const double* F, int n, double* out, hipStream_t st) {
-    if (n <= 0) return hipSuccess;
-    k_export_forces<<<cdiv(3ll * n, 256), 256, 0, st>>>(F, n, out);
+hipError_t launch_export_forces(const double* F, int n, long long k0, long long m, double* out, hipStream_t st) {
+    if (m <= 0) return hipSuccess;
+    k_export_forces<<<cdiv(m, 256), 256, 0, st>>>(F, n, k0, m, out);
     return hipGetLastError();
 }
 

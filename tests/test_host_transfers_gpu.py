@@ -80,3 +80,28 @@ def test_reads_leave_the_stream_idle(gpu):
             assert np.array_equal(b.forces(k), first[k])
             assert stream.query(), k
         b.set_stream(None)
+
+
+def test_systems_beyond_the_staging(gpu):
+    """Positions of more than 65,536 atoms go in pieces, forces of more than 174,762 come in pieces,
+    and reads one after the other send what fits."""
+    p = W.ATMParams(0.2, 0.4, 0.1, 110.0, 0.0, 200.0, 100.0, 0.0625, 1.0)
+    systems = [W.lattice_system(n, (n / 33.75) ** (1.0 / 3.0), 0.6, 20, (1.0, 1.0, 1.0), 3 + n, p)
+               for n in (65536, 180001, 65537, 60000, 131075)]
+    rng = np.random.default_rng(2)
+    xs = [(s.positions + rng.uniform(-0.02, 0.02, s.positions.shape)).astype(np.float32) for s in systems]
+    with ATMBatch(systems) as b:
+        for k, x in enumerate(xs):
+            b.set_positions(k, x)
+        b.compute()
+        order = list(range(len(xs))) + [3, 4, 0, 1, 2, 2]
+        host = [(b.result(k), b.forces(k)) for k in order]
+        dev = torch.as_tensor(np.concatenate(xs), device="cuda")
+        torch.cuda.synchronize()
+        b.set_positions_device(dev.data_ptr())
+        b.compute()
+        for k, (r, F) in zip(order, host):
+            assert b.result(k) == r
+            fixed = b.forces_fixed(k)
+            assert np.array_equal(np.rint(F * 2.0 ** 24).astype(np.int64), fixed)
+            assert np.abs(F).max() > 1.0
