@@ -88,8 +88,12 @@ struct PmeForce {
     DevBuf dResult, dOverflow, dLig, dDcls, dCcls;
     PmeDesc D{};
     PmePtrs P{};
-    // page-locked memory the evaluation's kernels use in place: inputs, results, force (atom by atom)
-    HostBuf hIn, hRecord, hOut;
+    // page-locked memory the evaluation's kernels use in place, one block taken at creation: inputs,
+    // results, force (atom by atom)
+    HostBuf hBlock;
+    double* hIn = nullptr;
+    PmeHostRecord* hRecord = nullptr;
+    double* hOut = nullptr;
     // captured evaluation per (state 1 only, forces) and the descriptors it was captured with
     hipGraphExec_t graph[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
     PmeDesc graphD[2][2];
@@ -235,9 +239,6 @@ void setup(PmeForce& S) {
     HIPCHK(hipStreamSynchronize(st));
     const long long ng = (long long)S.K[0] * S.K[1] * S.K[2];
     S.dIn.alloc(sizeof(double) * (kPmeInHead + 3 * (size_t)n));
-    S.hIn.alloc(sizeof(double) * (kPmeInHead + 3 * (size_t)n));
-    S.hRecord.alloc(sizeof(PmeHostRecord));
-    S.hOut.alloc(sizeof(double) * 3 * (size_t)n);
     S.dX2.alloc(sizeof(double) * 3 * n);
     S.dCellOf.alloc(sizeof(int) * n);
     S.dRankOf.alloc(sizeof(int) * n);
@@ -328,10 +329,10 @@ void set_box(PmeForce& S, const double box[3]) {
         S.nslotAlloc = S.D.nslot;
     }
     PmePtrs& P = S.P;
-    P.hostIn = S.hIn.as<double>();
+    P.hostIn = S.hIn;
     P.in = S.dIn.as<double>();
-    P.record = S.hRecord.as<PmeHostRecord>();
-    P.hostF = S.hOut.as<double>();
+    P.record = S.hRecord;
+    P.hostF = S.hOut;
     P.x = P.in + kPmeInHead;
     P.x2 = S.dX2.as<double>();
     P.displ = S.dDispl.as<double>();
@@ -436,6 +437,12 @@ int atm_pme_create(int32_t device, const atm_pme_desc* desc, void** out) {
         S->displ.assign(3 * (size_t)S->n, 0.0);
         S->params = atm_params{0.5, 0.5, 0.0, 0.0, 0.0, 1e300, 1e300, 1.0, 1.0};
         HIPCHK(hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking));
+        static_assert(sizeof(PmeHostRecord) % sizeof(double) == 0, "the force follows the record");
+        const size_t in = kPmeInHead + 3 * (size_t)S->n, rec = sizeof(PmeHostRecord) / sizeof(double);
+        S->hBlock.alloc(sizeof(double) * (in + rec + 3 * (size_t)S->n));
+        S->hIn = S->hBlock.as<double>();
+        S->hRecord = reinterpret_cast<PmeHostRecord*>(S->hIn + in);
+        S->hOut = S->hIn + in + rec;
         *out = S.release();
     });
 }
@@ -549,8 +556,8 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
         const double head[kPmeInHead] = {S.params.lambda1, S.params.lambda2, S.params.alpha, S.params.u0,
                                          S.params.w0, S.params.umax, S.params.ubcore, S.params.acore,
                                          S.params.direction, S.eoff[0], S.eoff[1]};
-        std::memcpy(S.hIn.p, head, sizeof(head));
-        std::memcpy(S.hIn.as<double>() + kPmeInHead, positions, sizeof(double) * 3 * S.n);
+        std::memcpy(S.hIn, head, sizeof(head));
+        std::memcpy(S.hIn + kPmeInHead, positions, sizeof(double) * 3 * S.n);
         const bool single = (flags & ATM_EVAL_STATE1_ONLY) != 0;
         PmeHostRecord rec;
         for (int attempt = 0; attempt < 2; ++attempt) {
@@ -580,7 +587,7 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
             }
             HIPCHK(hipGraphLaunch(g, st));
             HIPCHK(hipStreamSynchronize(st));
-            rec = *S.hRecord.as<PmeHostRecord>();
+            rec = *S.hRecord;
             if (!rec.overflow) break;
             if (S.D.cellCap >= kPmeCellMax)
                 fail(ATM_ERR_CAPACITY, "a cell holds more than " + std::to_string(kPmeCellMax) + " atoms");
@@ -588,8 +595,7 @@ int atm_pme_eval(void* h, const double* positions, const double box[3], int32_t 
         }
         const SysResult& r = rec.result;
         if (forces) {
-            const double* F = S.hOut.as<double>();
-            for (size_t k = 0; k < 3 * (size_t)S.n; ++k) forces[k] += F[k];
+            for (size_t k = 0; k < 3 * (size_t)S.n; ++k) forces[k] += S.hOut[k];
         }
         if (parts) std::memcpy(parts, rec.parts, sizeof(rec.parts));
         if (result) {
