@@ -28,7 +28,7 @@ constexpr int kPmeLineTile = 16;   // grid lines per block of the fused line ker
 struct PmeDesc {
     int n;                       // atoms
     int m[3], ncell;             // cell grid (edge >= rc, at least 3 per axis)
-    int cellCap, chunks;         // atoms per cell the direct kernel covers (chunks of kPmeBlockAtoms)
+    int cellCap, chunks;         // atoms per cell the direct kernel covers (chunks of kPmeIBlock)
     int K[3], ngrid;             // PME grid
     int twOff[3];                // offset of each axis' twiddle table
     int nex;                     // exception pairs

@@ -10,8 +10,8 @@
 //                    positions / parameters / exclusion keys / displacement
 //                    classes gathered into cell order
 //   k_pme_direct     erfc(alpha r)/r Coulomb + LJ over minimum-image pairs with
-//                    r < rc that are not exceptions; one block per (cell, the
-//                    cell or one of its 13 forward neighbours): each pair once
+//                    r < rc that are not exceptions; one block per (64 atoms of a
+//                    cell, the cell or one of its 13 forward neighbours): each pair once
 //   k_pme_spread_tiles  order-5 B-spline charge spreading per cell into an LDS
 //                    tile of the grid, 64-bit fixed point (k_pme_spread: the
 //                    same straight into the grid, when a tile does not fit)
