@@ -14,6 +14,9 @@ constexpr int kPmeCellMax = 1024;  // atoms per cell the cell sort holds
 constexpr int kPmeIBlock = 64;
 constexpr int kPmeJBlock = 160;
 constexpr int kPmeDirectWaves = 4;
+// Displacement classes: 0 not displaced, 1 .. kPmeClassMax the same for atoms displaced alike; with the
+// atom (below 2^24) in one word.
+constexpr int kPmeClassShift = 24, kPmeClassMax = 127, kPmeAtomMask = (1 << kPmeClassShift) - 1;
 constexpr int kPmeExWords = 4;       // words of each i-atom's exclusion row it stages (groups of up to 128 atoms)
 constexpr int kPmeSpreadSplit = 4; // parts of a cell's atoms spread by separate blocks (own LDS tiles)
 constexpr int kPmeHalfShell = 14;  // the cell itself and its 13 forward neighbour cells
@@ -62,12 +65,10 @@ struct PmePtrs {
     double4* wpos;          // [n] wrapped positions
     const double2* prm;     // [n] (q sqrt(k_e), q)
     const double2* prm2;    // [n] (sigma/2, 2 sqrt(eps))
-    const int4* exkey;      // [n] (exclusion group, rank in group, bitmap row offset, 0)
+    const int4* exkey;      // [n] (exclusion group, rank in group, bitmap row offset, displacement class)
     double4* cpos;          // [n] cell order: wrapped x, y, z, q sqrt(k_e)
     double2* cprm;          // [n] cell order: sigma/2, 2 sqrt(eps)
-    int4* cex;              // [n] cell order: group, rank, row offset, atom
-    const int* dcls;        // [n] displacement class: 0 not displaced, the same for atoms displaced alike
-    int* ccls;              // [n] cell order: displacement class
+    int4* cex;              // [n] cell order: group, rank, row offset, atom | class << kPmeClassShift
     const uint32_t* exbits; // exclusion bitmaps
     const int2* expairs;    // [nex]
     const double4* exprm;   // [nex] (k_e qq', sigma', 4 eps', k_e q_i q_j)

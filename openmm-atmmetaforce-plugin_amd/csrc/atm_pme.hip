@@ -221,8 +221,7 @@ __global__ void __launch_bounds__(256) k_pme_cellsort(PmeDesc D, PmePtrs P) {
         P.cpos[slot] = make_double4(w.x, w.y, w.z, pr.x);
         P.cprm[slot] = make_double2(P.prm2[a].x, P.prm2[a].y);
         const int4 ex = P.exkey[a];
-        P.cex[slot] = make_int4(ex.x, ex.y, ex.z, a);
-        P.ccls[slot] = P.dcls[a];
+        P.cex[slot] = make_int4(ex.x, ex.y, ex.z, a | ex.w << kPmeClassShift);
     }
 }
 
@@ -274,8 +273,7 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
     static_assert(JB + W - 1 <= 64 * W, "a wave's j-atoms are looked over one per lane");
     __shared__ double4 sI[IB], sJ[JB];       // x, y, z, q sqrt(k_e); i-atoms shifted to the neighbour's image
     __shared__ double2 sIp[IB], sJp[JB];
-    __shared__ int4 sIx[IB], sJx[JB];        // exclusion group, rank, row offset, atom
-    __shared__ int sIc[IB], sJc[JB];         // displacement classes
+    __shared__ int4 sIx[IB], sJx[JB];        // exclusion group, rank, row offset, atom and displacement class
     __shared__ uint32_t sIw[kPmeExWords][IB]; // first words of the i-atoms' exclusion rows
     __shared__ unsigned long long sIF[3][IB], sJF[3][JB];
     __shared__ uint32_t sQ[W][128];
@@ -313,7 +311,6 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
         sIp[k] = P.cprm[i0 + k];
         const int4 xk = P.cex[i0 + k];
         sIx[k] = xk;
-        sIc[k] = P.ccls[i0 + k];
 #pragma unroll
         for (int w = 0; w < kPmeExWords; ++w) sIw[w][k] = P.exbits[xk.z + w];  // (padded past the last row)
         sIF[0][k] = 0ull; sIF[1][k] = 0ull; sIF[2][k] = 0ull;
@@ -379,7 +376,6 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
             sJ[k] = P.cpos[jb + k];
             sJp[k] = P.cprm[jb + k];
             sJx[k] = P.cex[jb + k];
-            sJc[k] = P.ccls[jb + k];
             sJF[0][k] = 0ull; sJF[1][k] = 0ull; sJF[2][k] = 0ull;
         }
         __syncthreads();
@@ -395,8 +391,8 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
             const uint64_t act = __ballot(active);
             const uint32_t codeI = (uint32_t)i << 16;
             const int jself = jb - (i0 + i);  // the cell itself: j slots above the i slot only
-            const int clsI = sIc[i];
-            const bool mixed = shared && __ballot((active && clsI != 0) || (ka + lane < kb && sJc[ka + lane] != 0)) != 0ull;
+            const int clsI = xi.w >> kPmeClassShift;
+            const bool mixed = shared && __ballot((active && clsI != 0) || (ka + lane < kb && sJx[ka + lane].w > kPmeAtomMask)) != 0ull;
             for (int k0 = ka; k0 < kb; k0 += G) {
                 const int k = min(k0 + jg, kb - 1);
                 const double dx = px - sJ[k].x, dy = py - sJ[k].y, dz = pz - sJ[k].z;
@@ -404,7 +400,7 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
                 uint64_t m = __ballot(r2 < rc2) & act;
                 if (G > 1) m &= __ballot(k0 + jg < kb);
                 if (nb == 0) m &= __ballot(jself + k > 0);
-                if (mixed) m &= __ballot(sJc[k] == clsI);
+                if (mixed) m &= __ballot((sJx[k].w >> kPmeClassShift) == clsI);
                 if (m == 0ull) continue;
                 const uint64_t same = __ballot(sJx[k].x == xi.x) & m;
                 if (same != 0ull) {  // atoms of one exclusion group: look the pairs up
@@ -427,7 +423,7 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
         if (tail > head) dense(tail - head);  // the staged j-atoms are replaced or flushed next
         __syncthreads();
         for (int k = threadIdx.x; k < nj; k += NT) {  // j forces of the batch
-            const int atom = sJx[k].w;
+            const int atom = sJx[k].w & kPmeAtomMask;
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
                 const unsigned long long v = sJF[q][k];
@@ -437,7 +433,7 @@ __global__ void __launch_bounds__(64 * kPmeDirectWaves, 4) k_pme_direct(PmeDesc 
         __syncthreads();
     }
     for (int k = threadIdx.x; k < ni; k += NT) {
-        const int atom = sIx[k].w;
+        const int atom = sIx[k].w & kPmeAtomMask;
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             const unsigned long long v = sIF[q][k];
@@ -481,7 +477,6 @@ __global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P) {
     const int4 xa = P.exkey[a];
     const double2 pa = P.prm2[a];
     const double qa = P.prm[a].x;
-    const int clsA = P.dcls[a];
     double e = 0.0;
     unsigned long long fx = 0ull, fy = 0ull, fz = 0ull;
     auto pair = [&](int b, double dx, double dy, double dz, double r2, int grp, int rank, double qb, double2 pb) {
@@ -500,14 +495,15 @@ __global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P) {
         const double dx = px - pj.x, dy = py - pj.y, dz = pz - pj.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
         if (!(r2 < D.rc2)) continue;
-        if (P.ccls[j] != 0) continue;  // displaced itself: below
         const int4 xj = P.cex[j];
+        if (xj.w > kPmeAtomMask) continue;  // displaced itself: below
         pair(xj.w, dx, dy, dz, r2, xj.x, xj.y, pj.w, P.cprm[j]);
     }
     if (cellOff == 0)
         for (int q = k + 1 + lane; q < D.nlig; q += 64) {
             const int b = P.lig[q];
-            if (P.dcls[b] == clsA) continue;  // displaced alike: in the shared sums
+            const int4 xb = P.exkey[b];
+            if (xb.w == xa.w) continue;  // displaced alike: in the shared sums
             double v[3];
             wrap_cell(X[3 * b], D.L[0], D.invL[0], D.m[0], &v[0]);
             wrap_cell(X[3 * b + 1], D.L[1], D.invL[1], D.m[1], &v[1]);
@@ -518,7 +514,6 @@ __global__ void __launch_bounds__(64) k_pme_displaced(PmeDesc D, PmePtrs P) {
             dz -= D.L[2] * rint(dz * D.invL[2]);
             const double r2 = dx * dx + dy * dy + dz * dz;
             if (!(r2 < D.rc2)) continue;
-            const int4 xb = P.exkey[b];
             pair(b, dx, dy, dz, r2, xb.x, xb.y, P.prm[b].x, P.prm2[b]);
         }
     e = wave_sum(e);
@@ -709,7 +704,7 @@ __global__ void __launch_bounds__(256) k_pme_spread_tiles(PmeDesc D, PmePtrs P, 
     for (int task = threadIdx.x; task < cnt * kOrder; task += 256) {
         const int sl = s0 + task / kOrder, a = task % kOrder;
         const double4 p = P.cpos[sl];
-        const double q = P.prm[P.cex[sl].w].y;
+        const double q = P.prm[P.cex[sl].w & kPmeAtomMask].y;
         if (q == 0.0) continue;
         double th[3][kOrder], dth[kOrder];
         int g0[3];

@@ -85,7 +85,7 @@ struct PmeForce {
 
     DevBuf dIn, dX2, dDispl, dCellOf, dRankOf, dCellCount, dCellStart, dCellAtoms, dWpos, dPrm, dPrm2, dExkey;
     DevBuf dCpos, dCprm, dCex, dExbits, dExpairs, dExprm, dQgrid, dG0, dG1, dTw, dBmod, dF, dEslot, dParts;
-    DevBuf dResult, dOverflow, dLig, dDcls, dCcls;
+    DevBuf dResult, dOverflow, dLig;
     PmeDesc D{};
     PmePtrs P{};
     // page-locked memory the evaluation's kernels use in place, one block taken at creation: inputs,
@@ -196,7 +196,16 @@ void setup(PmeForce& S) {
         exprm[k] = make_double4(ke * S.exQQ[k], S.exSig[k], 4.0 * S.exEps[k], ke * S.q[i] * S.q[j]);
     }
     std::vector<int4> exkey(n);
-    for (int i = 0; i < n; ++i) exkey[i] = make_int4(grp[i], rank[i], (int)rowOff[i], 0);
+    // displaced atoms and their displacement classes (1, 2, ... by first appearance)
+    std::vector<int> lig;
+    std::map<std::array<double, 3>, int> classOf;
+    for (int i = 0; i < n; ++i) {
+        exkey[i] = make_int4(grp[i], rank[i], (int)rowOff[i], 0);
+        const std::array<double, 3> d = {S.displ[3 * (size_t)i], S.displ[3 * (size_t)i + 1], S.displ[3 * (size_t)i + 2]};
+        if (d[0] == 0.0 && d[1] == 0.0 && d[2] == 0.0) continue;
+        lig.push_back(i);
+        exkey[i].w = std::min(classOf.emplace(d, (int)classOf.size() + 1).first->second, kPmeClassMax);
+    }
     // twiddles and moduli
     std::vector<double2> tw;
     std::vector<double> bmod;
@@ -219,23 +228,13 @@ void setup(PmeForce& S) {
     upload(st, S.dTw, tw.data(), sizeof(double2) * tw.size());
     upload(st, S.dBmod, bmod.data(), sizeof(double) * bmod.size());
     upload(st, S.dDispl, S.displ.data(), sizeof(double) * 3 * n);
-    // displaced atoms and their displacement classes (1, 2, ... by first appearance)
-    std::vector<int> lig, dcls(n, 0);
-    std::map<std::array<double, 3>, int> classOf;
-    for (int i = 0; i < n; ++i) {
-        const std::array<double, 3> d = {S.displ[3 * (size_t)i], S.displ[3 * (size_t)i + 1], S.displ[3 * (size_t)i + 2]};
-        if (d[0] == 0.0 && d[1] == 0.0 && d[2] == 0.0) continue;
-        lig.push_back(i);
-        dcls[i] = classOf.emplace(d, (int)classOf.size() + 1).first->second;
-    }
     S.D.nlig = (int)lig.size();
     // the displaced atoms' pairs by themselves: each costs 54 waves over its neighbour cells, so
-    // only while they are few.  Whole call in us with 21 atoms, n/64, n/32 and n/16 displaced: 201, 217,
-    // 229, 249 (8,479 atoms; both states in full 260 to 265) and 363, 398, 435, 504 (25,437; 503)
-    S.D.delta = 16ll * S.D.nlig <= n && S.D.nlig <= 65535;
+    // only while they are few.  Whole call in us with 21 atoms, n/64, n/32 and n/16 displaced: 203, 216,
+    // 227, 248 (8,479 atoms; both states in full 260 to 265) and 357, 391, 428, 498 (25,437; 503)
+    S.D.delta = 16ll * S.D.nlig <= n && S.D.nlig <= 65535 && classOf.size() <= (size_t)kPmeClassMax;
     if (lig.empty()) lig.push_back(0);
     upload(st, S.dLig, lig.data(), sizeof(int) * lig.size());
-    upload(st, S.dDcls, dcls.data(), sizeof(int) * n);
     HIPCHK(hipStreamSynchronize(st));
     const long long ng = (long long)S.K[0] * S.K[1] * S.K[2];
     S.dIn.alloc(sizeof(double) * (kPmeInHead + 3 * (size_t)n));
@@ -247,7 +246,6 @@ void setup(PmeForce& S) {
     S.dCpos.alloc(sizeof(double4) * n);
     S.dCprm.alloc(sizeof(double2) * n);
     S.dCex.alloc(sizeof(int4) * n);
-    S.dCcls.alloc(sizeof(int) * n);
     S.dQgrid.alloc(sizeof(long long) * 2 * ng);
     S.dG0.alloc(sizeof(double2) * 2 * ng);
     S.dG1.alloc(sizeof(double2) * 2 * ng);
@@ -349,8 +347,6 @@ void set_box(PmeForce& S, const double box[3]) {
     P.cpos = S.dCpos.as<double4>();
     P.cprm = S.dCprm.as<double2>();
     P.cex = S.dCex.as<int4>();
-    P.dcls = S.dDcls.as<int>();
-    P.ccls = S.dCcls.as<int>();
     P.exbits = S.dExbits.as<uint32_t>();
     P.expairs = S.dExpairs.as<int2>();
     P.exprm = S.dExprm.as<double4>();

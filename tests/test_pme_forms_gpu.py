@@ -153,3 +153,30 @@ def test_far_positions(gpu):
             assert np.isfinite(rf["state1_energy"]) and np.isfinite(Ff).all()
         r2, F2, _ = f.evaluate(x)
     assert r2 == r and np.array_equal(F2, F)
+
+
+@pytest.mark.parametrize("classes", [1, 127, 128])
+def test_displacement_classes(gpu, classes):
+    """As many different displacements as the pairs of both states tell apart, and one more."""
+    n = 2100
+    rng = np.random.default_rng(classes)
+    L = np.array([3.05, 3.1, 3.2])
+    lat = np.array([(i, j, k) for i in range(13) for j in range(13) for k in range(13)][:n], dtype=float)
+    x = (lat + 0.5) * (L / 13) + rng.uniform(-0.03, 0.03, (n, 3))
+    q = rng.normal(0, 0.5, n)
+    q -= q.mean()
+    sig, eps = rng.uniform(0.15, 0.2, n), rng.uniform(0.1, 0.6, n)
+    d = np.zeros((n, 3))
+    at = rng.permutation(n)[:131]
+    # between lattice sites, in whole steps of the lattice and a 1/512 of it that tells them apart
+    d[at] = (L / 13) * (2.5 + rng.permutation(131)[:, None] % classes / 512.0)
+    pairs = np.array([(at[0], at[1]), (at[0], 3), (4, 5)])
+    zero = np.zeros(len(pairs))
+    print(f"[pme] {classes} displacement classes", flush=True)
+    with pme.ATMPMEForce(q, sig, eps, d, L, 1.0, exceptions=(pairs, zero, zero + 0.1, zero), params=PARAMS) as f:
+        r, F, _ = f.evaluate(x)
+    ref, Fref, p1, p2 = _oracle_atm(x, q, sig, eps, L, pairs, zero, zero + 0.1, zero, d, PARAMS)
+    for key, want, p in (("state1_energy", ref["U1"], p1), ("state2_energy", ref["U2"], p2)):
+        scale = sum(abs(p[k]) for k in ("direct_coulomb", "direct_lj", "exclusion_correction", "self"))
+        assert abs(r[key] - want) <= E_REL * max(1.0, scale)
+    assert np.abs(F - Fref).max() < F_ABS + 1e-12 * np.abs(Fref).max()
