@@ -10,7 +10,9 @@ namespace atm {
 constexpr int kPmeCellMax = 1024;  // atoms per cell the cell sort holds
 // Block of the direct kernel: atoms of a cell, atoms of its neighbour cell staged at a time, waves.
 // 48 us for 8,479 atoms and 120 for 25,437 (cells of some 133); (64, 160, 8) 55 / 156,
-// (64, 160, 2) 70 / 133, (128, 160, 8) 73 / 151, (192, 192, 8) 74 / 152.
+// (64, 160, 2) 70 / 133, (128, 160, 8) 73 / 151, (192, 192, 8) 74 / 152.  Staged atoms 96 / 160 / 224 at other
+// cell sizes, whole calls of 16,958 atoms in us: cells of 39 295 / 294 / 294, 68 284 / 285 / 283, 132 296 / 287 /
+// 286, 202 318 / 310 / 300, 314 355 / 341 / 337.
 constexpr int kPmeIBlock = 64;
 constexpr int kPmeJBlock = 160;
 constexpr int kPmeDirectWaves = 4;
