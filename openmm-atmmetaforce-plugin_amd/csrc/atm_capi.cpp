@@ -152,6 +152,8 @@ struct Context {
         if (own) (void)hipStreamDestroy(own);
     }
     void dropGraphs() {
+        // an evaluation that has not been waited for may still run from one of them
+        if (!graphs.empty()) (void)hipStreamSynchronize(stream);
         for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second);
         graphs.clear();
     }
