@@ -115,7 +115,8 @@ typedef struct atm_result {
 /* Autotuned launch configuration (read back with atm_get_tuning). */
 typedef struct atm_tuning {
     double column_scale;      /* column edge / (8/density)^(1/3) */
-    int32_t pair_waves_per_block;
+    int32_t pair_waves_per_block; /* 1, 2, 4 or 8: waves per block of pair kernels 1-6 (a block of the
+                                 tile kernel is one group, its waves are pair_split's) */
     int32_t zbins_per_column; /* z-bins per column edge */
     double best_ms;           /* measured time of the chosen configuration */
     int32_t pair_kernel;      /* 0: 8x8 cluster-pair tiles; 1-4: compacted in-cutoff pairs
@@ -200,7 +201,9 @@ int atm_set_exceptions(void* context, int32_t sys, int32_t count, const int32_t*
  * the reference (CommonATMMetaForceKernels.cpp:229-251). */
 int atm_set_displacements(void* context, int32_t sys, const double* displacements);
 
-/* Positions (num_atoms*3, nm) of system `sys`; the device path stores them in FP32.
+/* Positions (num_atoms*3, nm) of system `sys`; the device path stores them in FP32.  The
+ * array is read before the call returns, its upload is enqueued on the context stream
+ * (refused while that stream is being captured).
  * Replaces the position half of CalcATMMetaForceKernel::copyState
  * (ATMMetaForceKernels.h:55; ReferenceATMMetaForceKernels.cpp:116-124). */
 int atm_set_positions(void* context, int32_t sys, const double* positions);
@@ -253,7 +256,9 @@ int atm_synchronize(void* context);
  * (ATMMetaForceKernels.h:57). */
 int atm_get_results(void* context, int32_t sys, atm_result* out);
 
-/* Accumulated ATM force of system `sys` (num_atoms*3 doubles, kJ/mol/nm). */
+/* Accumulated ATM force of system `sys` (num_atoms*3 doubles, kJ/mol/nm).  Waits for the
+ * context stream; a caller that reads one system after the other gets the next ones (up to
+ * three) fetched in the same wait. */
 int atm_get_forces(void* context, int32_t sys, double* forces);
 
 /* Accumulated ATM force in fixed point (num_atoms*3, ATM_FORCE_SCALE units,
