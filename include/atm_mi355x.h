@@ -138,10 +138,9 @@ typedef struct atm_tuning {
                                  x + d is evaluated as the difference from x (the pairs and
                                  exception terms with a displaced atom at both states; the
                                  other atoms do not move), so only x is binned and paired;
-                                 1: x + d is binned and paired in full like x.  The difference
-                                 keeps the FP32 rounding of a displaced atom's force at x in
-                                 x + d: where atoms may overlap at x while x + d is the state
-                                 that counts (direction -1, pairs below 0.15 nm), set 1 */
+                                 1: x + d is binned and paired in full like x.  Where the
+                                 direction is not above 0 (x + d is the state whose force
+                                 counts) x is evaluated as the difference from x + d */
     int32_t pair_order;       /* the tile kernel's group order: 0 launch order; 1 every set's
                                  groups longest list first, interleaved over all sets; 2 the
                                  same over windows of 8 sets (default); 3 each set longest

@@ -319,8 +319,8 @@ class ATMBatch:
         the density).  pair_split: least number of waves sharing one group's list in the tile
         kernel (1, 2, 4, 8; a launch of few groups takes more, up to 16).
         full_state2: bin and pair x + d in full instead of as the difference from x at the
-        displaced atoms (used when every system displaces at most a quarter of its atoms); for legs
-        with direction -1 whose displaced atoms may overlap others at x (pairs below 0.15 nm).
+        displaced atoms (used when every system displaces at most a quarter of its atoms; where the
+        direction is not above 0, x as the difference from x + d).
         pair_order: the tile kernel's group order (0 launch order, 1 longest lists first over all
         sets, 2 the same over windows of 8 sets, 3 each set longest first, one set after another)."""
         t = C.Tuning(column_scale, pair_waves_per_block, zbins_per_column, 0.0, pair_kernel, list_capacity,

@@ -24,9 +24,9 @@ __global__ void k_fill_f64(double* p, long long n) {
 
 // wset null: the accumulators already hold weighted sums; otherwise they hold
 // dU/dp of each set and wset[2 s], wset[2 s + 1] weight the two states here.
-// delta (x + d evaluated as the difference from x, wset given): the x + d set's
-// accumulators hold dU2/dp - dU1/dp by atom, so the weights are wa + wb on the x
-// set's and wb on the difference.
+// delta (state difference, wset given): the second set's accumulators hold, by atom, dU/dp
+// of the other state minus the base's (x, or x + d where the direction is not above 0), so
+// the weights are wa + wb on the base set's and the other state's on the difference.
 __global__ void k_backward_gather(DevPtrs P, int sysBegin, double* dq, double* dsig, double* deps,
                                   const double* wset, int delta) {
     const int s = sysBegin + blockIdx.y;
@@ -37,9 +37,12 @@ __global__ void k_backward_gather(DevPtrs P, int sysBegin, double* dq, double* d
     const int a = D0.slotOff + P.slotOf[D0.setAtomOff + i];
     const int b = delta ? D1.slotOff + i : D1.slotOff + P.slotOf[D1.setAtomOff + i];
     const int k = D0.atomOff + i;
-    double wa = wset ? wset[2 * s] : 1.0;
-    const double wb = wset ? wset[2 * s + 1] : 1.0;
-    if (delta) wa += wb;
+    double wa = wset ? wset[2 * s] : 1.0, wb = wset ? wset[2 * s + 1] : 1.0;
+    if (delta) {
+        const double w = wa + wb;
+        if (!(P.params[s].direction > 0.0)) wb = wa;
+        wa = w;
+    }
     const double sqk = 11.787089759563214;  // sqrt(138.935456)
     const double ep = P.prm64[k].y;          // 2 sqrt(eps)
     if (dq) dq[k] = sqk * fma(wa, P.gq[a], wb * P.gq[b]);

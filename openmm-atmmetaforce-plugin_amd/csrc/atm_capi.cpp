@@ -134,7 +134,8 @@ struct Context {
     std::vector<unsigned char> ligMark;
     int maxLig = 0;
     bool deltaOK = false;        // every system displaces at most a quarter of its atoms
-    bool lastDelta = false;      // the last batched evaluation used the state difference
+    bool lastDelta = false;      // the last batched evaluation used the state difference ...
+    std::vector<char> base;      // ... taken from x (0) or x + d (1), per system, by the parameters on the device
     DevBuf dLig, dLigMark, dLenergy, dLxidx;
 
     std::map<int, hipGraphExec_t> graphs;
@@ -615,6 +616,7 @@ void flush_params(Context& C) {
     std::memcpy(stage, C.params.data(), bytes);
     HIPCHK(launch_copy8(C.dParams.p, stage, (long long)(bytes / 8), C.stream));
     C.upParams.end(C.stream);
+    for (int s = 0; s < C.nsys; ++s) C.base[s] = !(C.params[s].direction > 0.0);
     C.paramsDirty = false;
 }
 
@@ -636,7 +638,7 @@ void ensure_grad_buffers(Context& C) {
 // kernel, then after build, pair list, pair kernel, exception terms and displaced
 // atoms, energy and blend.
 // With the state difference (use_delta) only the state-0 sets are built and paired
-// (set stride 2), then the displaced-atom kernels evaluate what x + d changes.
+// (set stride 2), then the displaced-atom kernels evaluate what the other state changes.
 void enqueue_batched(Context& C, int flags, hipEvent_t* ev = nullptr) {
     const hipStream_t st = C.stream;
     const bool delta = use_delta(C, flags);
@@ -986,6 +988,7 @@ int atm_create(const atm_system_desc* systems, int32_t num_systems, int32_t devi
         C->hPrm64.assign(off, make_double4(0.0, 0.0, 0.0, 0.0));
         C->params.assign(num_systems, atm_params{0.5, 0.5, 0.0, 0.0, 0.0, 200.0, 100.0, 0.0625, 1.0});
         C->haveParticles.assign(num_systems, 0);
+        C->base.assign(num_systems, 0);
         C->results.assign(num_systems, atm_result{});
         C->dPosq.alloc(sizeof(float4) * off);
         C->dDispl.alloc(sizeof(float4) * off);
@@ -1395,15 +1398,15 @@ int atm_get_pairs(void* context, int32_t sys, int32_t state, int32_t* pairs, int
             return v;
         };
         std::vector<int2> v;
-        if (state == 1 && C.lastDelta) {
-            // x + d was evaluated as the difference from x: the state-0 pairs without those of
-            // the displaced atoms at x, with those at x + d
-            const std::vector<int2> all = dump(false, 0), d0 = dump(true, 0), d1 = dump(true, 1);
+        if (C.lastDelta && state != C.base[sys]) {
+            // the state was evaluated as the difference from the other: the pairs of that without
+            // those of its displaced atoms, with those at this state
+            const std::vector<int2> all = dump(false, 0), d0 = dump(true, state ^ 1), d1 = dump(true, state);
             std::vector<int2> keep;
             std::set_difference(all.begin(), all.end(), d0.begin(), d0.end(), std::back_inserter(keep), less);
             std::merge(keep.begin(), keep.end(), d1.begin(), d1.end(), std::back_inserter(v), less);
         } else {
-            v = dump(false, state);
+            v = dump(false, C.lastDelta ? 0 : state);
         }
         *count = (int64_t)v.size();
         const long long nout = std::min<long long>((long long)v.size(), cap);
@@ -1423,7 +1426,7 @@ int atm_get_stats(void* context, int64_t* pairs_in_cutoff, int64_t* pairs_evalua
         if (pairs_evaluated) ctr.alloc(sizeof(unsigned long long) * 4);
         for (int c = 0; c < 2 * C.nsys; ++c) {
             nin += (long long)rt[c].npairs;  // counted by the pair kernel of the evaluation
-            if (C.lastDelta && (c & 1)) continue;  // x + d was not binned (state difference)
+            if (C.lastDelta && (c & 1)) continue;  // one state was binned (state difference)
             if (pairs_evaluated) {
                 zero_on_stream(C, ctr.p, sizeof(unsigned long long) * 4);
                 HIPCHK(launch_pairs_dump(C.P, c, C.sets[c].groupCap, nullptr, 0, ctr.as<unsigned long long>(), C.stream));

@@ -21,11 +21,12 @@
 //     a nonzero charge product or epsilon are evaluated by a kernel of their own
 //     (one block per set) at the plain, non-periodic distance.
 //   * State difference: x + d differs from x only at the displaced atoms
-//     (d != 0).  When they are few, state 1 is not binned or paired: the
-//     state-0 set is, and a displaced-atom kernel evaluates every pair with a
-//     displaced atom at x and at x + d (neighbours from the state-0 cells), so
-//     U(x + d) = U(x) - E_d(x) + E_d(x + d) and F(x + d) = F(x) + dF, dF held in
-//     atom order in the state-1 set's fixed-point sums.
+//     (d != 0).  When they are few, one state is binned and paired, into the
+//     state-0 set: the base, x or (direction not above 0) x + d.  A displaced-
+//     atom kernel evaluates every pair with a displaced atom at x and at x + d
+//     (neighbours from the base's cells), so U(other) = U(base) - E_d(base) +
+//     E_d(other) and F(other) = F(base) + dF, dF held in atom order in the
+//     state-1 set's fixed-point sums.
 #pragma once
 #include <stdint.h>
 
@@ -88,7 +89,7 @@ struct SetRuntime {
     int maxAtoms;  // largest untruncated atom-level list of one cluster (this evaluation)
     int pad_;
     unsigned long long lpairs[2];  // state-difference evaluation: in-cutoff pairs with a displaced
-                                   // atom at x ([0]) and at x + d ([1]) (state-1 set of a system)
+                                   // atom at x ([0]) and at x + d ([1]) (state-0 set of a system)
 };
 
 // Per-system state of the last evaluation on the device (mirrors atm_result).

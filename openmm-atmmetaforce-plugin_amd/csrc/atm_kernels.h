@@ -133,10 +133,10 @@ hipError_t launch_backward_pairs(const DevPtrs& P, int setBegin, int nsets, int 
 hipError_t launch_blend(const DevPtrs& P, int sysBegin, int nsys, int maxAtoms, int hostMode, double sp, double dir,
                         bool clear, hipStream_t st, bool delta = false);
 // State difference: the pairs with a displaced atom of systems [sysBegin, sysBegin + nsys) at
-// x and at x + d (after the state-0 sets' build; maxLig: most displaced atoms of one system),
+// x and at x + d (after the build of the base's sets; maxLig: most displaced atoms of one system),
 // and the exception terms with a displaced atom (their difference).
 // grads: the backward mode (energies, counts and the parameter derivatives of the displaced pairs,
-// x + d minus x, into gq/gsig/geps of the x + d sets indexed by atom; no forces)
+// the other state minus the base, into gq/gsig/geps of the state-1 sets indexed by atom; no forces)
 hipError_t launch_displaced(const DevPtrs& P, int sysBegin, int nsys, int maxLig, bool forces, hipStream_t st,
                             bool grads = false);
 hipError_t launch_displaced_exceptions(const DevPtrs& P, int sysBegin, int nsys, bool forces, hipStream_t st);

@@ -376,10 +376,21 @@ __global__ void k_zero_counts(DevPtrs P, int setBegin, double* f, long long nf) 
     if (i == 0) reset_set(P, c);
 }
 
+// The state that a state difference is taken from (0: x, 1: x + d): e0 of the combine, whose force
+// counts in full.  The other state may hold overlaps, whose pairs then only enter the difference,
+// with that state's weight; taken from x where x + d counts (direction not above 0), a pair at
+// 0.05 nm left 6e4 kJ/mol/nm of FP32 rounding in the force, at 0.1 nm 16.
+__device__ __forceinline__ int base_state(const DevPtrs& P, int sys) { return P.params[sys].direction > 0.0 ? 0 : 1; }
+
+// The state whose coordinates set D is built from.
+__device__ __forceinline__ int set_state(const DevPtrs& P, const SetDesc& D) {
+    return P.setStride == 2 ? base_state(P, D.sys) : D.state;
+}
+
 // Atom i of set c: its wrapped position to bpos; returns its fine cell.
 __device__ __forceinline__ int bin_atom(const DevPtrs& P, const SetDesc& D, int c, int i) {
     float4 p = P.posq[D.atomOff + i];
-    if (D.state) {
+    if (set_state(P, D)) {
         float4 d = P.displ[D.atomOff + i];
         p.x += d.x; p.y += d.y; p.z += d.z;  // exact on the 2^-20 grid
     }
@@ -2273,7 +2284,7 @@ __global__ void __launch_bounds__(256) k_exceptions(DevPtrs P, int setBegin, int
     const int n = D.excCount;
     const float4* X = P.posq + D.atomOff;
     const float4* Xd = P.displ + D.atomOff;
-    const bool shifted = D.state == 1;
+    const bool shifted = set_state(P, D) == 1;
     const double fixMax = D.fixMax;
     double e = 0.0;
     for (int k = threadIdx.x; k < n; k += 256) {
@@ -2307,9 +2318,10 @@ __global__ void __launch_bounds__(256) k_exceptions(DevPtrs P, int setBegin, int
 
 // ---------------------------------------------------------------- state difference
 //
-// When few atoms are displaced, x + d is not binned: every pair with a displaced
-// atom is evaluated at x and at x + d from the state-0 cells (the other atoms do
-// not move), U(x + d) = U(x) - E_d(x) + E_d(x + d) and F(x + d) = F(x) + dF.
+// When few atoms are displaced, only one state is binned, the base (base_state; the set
+// with index 2 sys, here the base set): every pair with a displaced atom is evaluated at x
+// and at x + d from its cells (the other atoms do not move), U(other) = U(base) - E_d(base)
+// + E_d(other) and F(other) = F(base) + dF.
 
 // Displaced atom a of a system at state st (0: x, 1: x + d), wrapped as k_bin does.
 __device__ __forceinline__ float4 displaced_position(const DevPtrs& P, const SetDesc& D, int a, int st) {
@@ -2328,19 +2340,19 @@ __device__ __forceinline__ bool same_displacement(const DevPtrs& P, const SetDes
 }
 
 // One wave per (displaced atom, state) of system sysBegin + blockIdx.y: its
-// in-cutoff pairs with the atoms that are not displaced (from the state-0 cells
+// in-cutoff pairs with the atoms that are not displaced (from the base set's cells
 // within the cutoff of its position at that state) and with the displaced atoms
 // after it in the list whose displacement differs (pairs of atoms displaced alike
 // keep their separation, so they are the same at both states and are left to
-// the state-0 evaluation).  Exact FP64 r^2 < rc^2 and the FP64 pair function of
-// the state-0 tiles, exceptions dropped as there.  The wave's energy goes to
+// the base's evaluation).  Exact FP64 r^2 < rc^2 and the FP64 pair function of
+// the base's tiles, exceptions dropped as there.  The wave's energy goes to
 // lenergy[2 (ligOff + k) + st], its pair count to rt[state-0 set].lpairs[st];
-// with FORCES, -F (state 0) or +F (state 1) goes to dF, the state-1 set's
+// with FORCES, -F (base) or +F (other state) goes to dF, the state-1 set's
 // fixed-point sums indexed by atom.  DUMP: the pairs (lower index first) are
 // written to out instead (state dumpState, no energy or force).  BWD (no forces):
 // the derivatives of the pair energies with respect to the stored parameters
 // q' = q sqrt(k_e), h = sigma/2, e' = 2 sqrt(eps) of both atoms (the tile kernel's
-// backward formulas), -dE (state 0) or +dE (state 1), into the x + d set's
+// backward formulas), -dE (base) or +dE (other state), into the state-1 set's
 // gradient accumulators indexed by atom.
 template <bool FORCES, bool EXC, bool DUMP, bool BWD = false>
 __global__ void __launch_bounds__(256) k_displaced(DevPtrs P, int sysBegin, int dumpState, int2* out, long long cap,
@@ -2368,7 +2380,7 @@ __global__ void __launch_bounds__(256) k_displaced(DevPtrs P, int sysBegin, int 
     const unsigned long long ma = EXC ? P.xmask[D.atomOff + a] : 0ull;
     const double fixMax = P.desc[c1].fixMax;
     const long long dOff = P.desc[c1].slotOff;  // dF of atom b at dOff + b
-    const double sgn = st ? 1.0 : -1.0;
+    const double sgn = st != base_state(P, s) ? 1.0 : -1.0;
     double eacc = 0.0, fax = 0.0, fay = 0.0, faz = 0.0;
     double gaq = 0.0, gah = 0.0, gae = 0.0;  // BWD: dE/d(q', h, e') of atom a
     uint32_t npair = 0;
@@ -2556,8 +2568,8 @@ __global__ void __launch_bounds__(256) k_displaced(DevPtrs P, int sysBegin, int 
 }
 
 // One block per system: the exception terms with a displaced atom whose partner
-// is displaced differently, at x + d minus at x: energy into xenergy[state-1 set],
-// with forces their difference into dF.
+// is displaced differently, at the other state minus at the base: energy into
+// xenergy[state-1 set], with forces their difference into dF.
 __global__ void __launch_bounds__(256) k_displaced_exceptions(DevPtrs P, int sysBegin, int forces) {
     const int s = sysBegin + blockIdx.x;
     const int c1 = 2 * s + 1;
@@ -2567,6 +2579,7 @@ __global__ void __launch_bounds__(256) k_displaced_exceptions(DevPtrs P, int sys
     const float4* Xd = P.displ + D.atomOff;
     const double fixMax = P.desc[c1].fixMax;
     const long long dOff = P.desc[c1].slotOff;
+    const double sgn = base_state(P, s) ? -1.0 : 1.0;
     double e = 0.0;
     for (int k = threadIdx.x; k < D.lxCount; k += 256) {
         const int x = P.lxidx[D.lxOff + k];
@@ -2580,10 +2593,12 @@ __global__ void __launch_bounds__(256) k_displaced_exceptions(DevPtrs P, int sys
         double fs0, fs1;
         const double e0 = exception_term(q, dx0, dy0, dz0, fs0);
         const double e1 = exception_term(q, dx1, dy1, dz1, fs1);
-        e += e1 - e0;
+        e += sgn * (e1 - e0);
         if (forces) {
-            add_force64(P, c1, fixMax, dOff + pr.x, fs1 * dx1 - fs0 * dx0, fs1 * dy1 - fs0 * dy0, fs1 * dz1 - fs0 * dz0);
-            add_force64(P, c1, fixMax, dOff + pr.y, fs0 * dx0 - fs1 * dx1, fs0 * dy0 - fs1 * dy1, fs0 * dz0 - fs1 * dz1);
+            const double fx = sgn * (fs1 * dx1 - fs0 * dx0), fy = sgn * (fs1 * dy1 - fs0 * dy0);
+            const double fz = sgn * (fs1 * dz1 - fs0 * dz0);
+            add_force64(P, c1, fixMax, dOff + pr.x, fx, fy, fz);
+            add_force64(P, c1, fixMax, dOff + pr.y, -fx, -fy, -fz);
         }
     }
     red[threadIdx.x] = e;
@@ -2611,15 +2626,15 @@ __device__ __forceinline__ double block_sum_256(double v, double* red) {
     return r;
 }
 
-// delta: state difference (only the state-0 set was paired): U2 = U1 - E_d(x) +
-// E_d(x + d) + the displaced exception terms' difference, offsets per state; the
-// state-1 pair count is derived the same way.
+// delta: state difference (only the base set was paired): U(other) = U(base) -
+// E_d(base) + E_d(other) + the displaced exception terms' difference, offsets per
+// state; the pair counts of x and x + d are derived the same way.
 __global__ void __launch_bounds__(256) k_energy(DevPtrs P, int sysBegin, int estride, int delta) {
     const int s = sysBegin + blockIdx.x;
     __shared__ double red[256];
     double U[2];
     if (delta) {
-        const int c0 = 2 * s, c1 = 2 * s + 1;
+        const int c0 = 2 * s, c1 = 2 * s + 1, base = base_state(P, s);
         const SetDesc& D = P.desc[c0];
         const int ng = P.rt[c0].ngroups;
         const double acc = energy_share(P, D, ng, estride);
@@ -2629,13 +2644,16 @@ __global__ void __launch_bounds__(256) k_energy(DevPtrs P, int sysBegin, int est
             const double* e = P.lenergy + 2ll * kDisplacedParts * (D.ligOff + k);
             double e0 = e[0], e1 = e[kDisplacedParts];
             for (int q = 1; q < kDisplacedParts; ++q) { e0 += e[q]; e1 += e[kDisplacedParts + q]; }
-            dd += e1 - e0;
+            dd += base ? e0 - e1 : e1 - e0;
         }
         const double de = block_sum_256(dd, red) + (D.lxCount > 0 ? P.xenergy[c1] : 0.0);
-        U[0] = e0 + (P.eoff ? P.eoff[c0] : 0.0);
-        U[1] = (e0 + de) + (P.eoff ? P.eoff[c1] : 0.0);
-        if (threadIdx.x == 0)
-            P.rt[c1].npairs = P.rt[c0].npairs - P.rt[c0].lpairs[0] + P.rt[c0].lpairs[1];
+        U[0] = (base ? e0 + de : e0) + (P.eoff ? P.eoff[c0] : 0.0);
+        U[1] = (base ? e0 : e0 + de) + (P.eoff ? P.eoff[c1] : 0.0);
+        if (threadIdx.x == 0) {
+            const unsigned long long n = P.rt[c0].npairs, l0 = P.rt[c0].lpairs[0], l1 = P.rt[c0].lpairs[1];
+            P.rt[c0].npairs = base ? n - l1 + l0 : n;
+            P.rt[c1].npairs = base ? n : n - l0 + l1;
+        }
     }
     for (int st = 0; st < 2 && !delta; ++st) {
         const int c = 2 * s + st;
@@ -2739,9 +2757,10 @@ __global__ void k_blend(DevPtrs P, int sysBegin, int nsys, int gx, int hostMode,
             const double* d = P.sd + 3 * b;
             gx += d[0]; gy += d[1]; gz += d[2];
         }
-        F[i] = ox + (f1x + w2 * gx);
-        F[N + i] = oy + (f1y + w2 * gy);
-        F[2 * N + i] = oz + (f1z + w2 * gz);
+        const double wo = dir > 0.0 ? w2 : w1;  // the weight of the state that is not the base
+        F[i] = ox + (f1x + wo * gx);
+        F[N + i] = oy + (f1y + wo * gy);
+        F[2 * N + i] = oz + (f1z + wo * gz);
         return;
     }
     const long long b = D1.slotOff + P.slotOf[D1.setAtomOff + i];

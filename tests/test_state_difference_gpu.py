@@ -131,3 +131,76 @@ def test_backward_after_a_state_difference_evaluation(gpu):
         err = np.linalg.norm(g[key] - ref[key]) / np.linalg.norm(ref[key])
         print(f"[backward] {key} rel {err:.2e}", flush=True)
         assert err < 2e-5
+
+
+def test_direction_decides_the_base(gpu):
+    """With the direction not above 0 the difference is taken from x + d: the same results, pair
+    counts and pair sets of both states, in batches of either direction and of both."""
+    sy = [dataclasses.replace(s, params=dataclasses.replace(P0, direction=d))
+          for s, d in zip(systems(), (-1.0, -1.0, 0.0, 1.0))]
+    for group in (sy[:1], sy[1:]):
+        with ATMBatch(group) as b:
+            for k in range(len(group)):
+                b.set_energy_offsets(k, 3.5, -1.25)
+            out = []
+            for full in (True, False):
+                r = run(b, full)
+                r["pairs0"] = [b.pairs(k, 0) for k in range(len(group))]
+                b.compute(forces=False, param_grads=True)
+                r["g"] = b.backward(np.linspace(0.5, 1.5, len(group)))
+                out.append(r)
+            full, diff = out
+            for k, s in enumerate(group):
+                rd, rf = diff["res"][k], full["res"][k]
+                base = "state1_energy" if s.params.direction > 0 else "state2_energy"
+                print(f"[base] sys {k} direction {s.params.direction} U1 {rd['state1_energy']:.12g} U2 {rd['state2_energy']:.12g}", flush=True)
+                assert rd[base] == rf[base]  # the same evaluation of the base
+                scale = max(1.0, abs(rf["state1_energy"]), abs(rf["state2_energy"]))
+                for key in ("state1_energy", "state2_energy", "energy"):
+                    assert abs(rd[key] - rf[key]) <= 1e-11 * scale
+                assert np.linalg.norm(diff["F"][k] - full["F"][k]) < 1e-6 * np.linalg.norm(full["F"][k])
+                for st in (0, 1):
+                    assert diff["counts"][2 * k + st] == full["counts"][2 * k + st]
+                    got = diff["pairs1" if st else "pairs0"][k]
+                    assert np.array_equal(got, full["pairs1" if st else "pairs0"][k])
+                    assert np.array_equal(got, oracle.pairs(s.positions + (s.displacements if st else 0.0), s.box, s.cutoff,
+                                                            exceptions=getattr(s, "exceptions", None)))
+            for key in ("dq", "dsigma", "deps"):
+                # FP32 pair sums of both states, weighted
+                assert np.linalg.norm(diff["g"][key] - full["g"][key]) < 2e-5 * np.linalg.norm(full["g"][key])
+            b.set_tuning(1.3, 1, 4, 0, pair_split=2)
+            for s in group:  # the direction turned round between evaluations
+                s.params = dataclasses.replace(s.params, direction=-s.params.direction or 1.0)
+            for k, s in enumerate(group):
+                b.set_energy_offsets(k, 0.0, 0.0)
+                b.set_params(k, s.params)
+            b.compute()
+            counts = b.list_stats()["pairs"]
+            for k, s in enumerate(group):
+                check_system(b, k, s, pairs=True, tag="direction turned", counts=counts)
+
+
+@pytest.mark.parametrize("molecules", [False, True])
+@pytest.mark.parametrize("dist", [0.1, 0.05, 0.01])
+def test_overlap_at_x_where_x_plus_d_counts(gpu, dist, molecules):
+    """A displaced atom on top of another at x, at the end of a leg where x + d is the physical
+    state (direction -1, weight 0 for x): the energy and force of x + d are those of x + d alone."""
+    p = W.ATMParams(0.0, 0.0, 0.0, 0.0, 0.0, 200.0, 100.0, 0.0625, -1.0)
+    s = W.lattice_system(3000, 4.5, 0.9, 30, (1.05, 1.05, 1.05), 41, p)
+    if molecules:
+        s = W.with_molecules(s, size=4, crosslink_every=9)
+    lig = np.flatnonzero(np.any(s.displacements != 0.0, axis=1))
+    a, other = lig[3], np.setdiff1d(np.arange(s.num_atoms), lig)[500]
+    s.positions = s.positions.copy()
+    s.positions[a] = s.positions[other] + np.round(dist * np.array([0.48, 0.6, 0.64]) * 2.0 ** 20) / 2.0 ** 20
+    ref, Fref = oracle.atm_eval(s)
+    with ATMBatch([s]) as b:
+        b.compute()
+        r, F = b.result(0), b.forces(0)
+        print(f"[base] pair at {dist} nm: U2 off by {r['state2_energy'] - ref['U2']:.3g}, F by {np.abs(F - Fref).max():.3g}", flush=True)
+        # FP64 pair energies in another order: 1e-13 of the sum of their magnitudes
+        assert abs(r["state2_energy"] - ref["U2"]) <= 1e-13 * max(ref["abs2"], 1.0)
+        assert abs(r["energy"] - ref["U2"]) <= 1e-13 * max(ref["abs2"], 1.0)
+        assert abs(r["state1_energy"] - ref["U1"]) <= 1e-6 * abs(ref["U1"])
+        # FP32 force vectors (2^-24 each) and per-lane sums of up to ~100 of them
+        assert np.linalg.norm(F - Fref) <= 1e-6 * np.linalg.norm(Fref)
